@@ -33,12 +33,20 @@
 //    written back with whole 16-byte stores;
 //    the fp32 accumulators of a layer are written back as the next layer's
 //    input after ReLU (bf16/fp16 forms store the activations in 16 bit);
-//  * feature gather (channels-last maps: 4 lanes fetch the 4 quarters of a
-//    tap's channel row) and positional encoding write the first layer's input
-//    directly into LDS; per-sample occupancy and compositing weights never
-//    reach HBM; the composited per-view tokens (4 x F floats per ray) do;
+//  * each wave samples the features of its own view slots (channels-last
+//    maps: a projection per (sample, view) in the lane of the sample, its taps
+//    and weights passed through the spare tail of that column's LDS row, then
+//    a lane per 8 channels) and composites the same slots' tokens, so a
+//    chunk's front end and back end need no barriers between waves; the
+//    positional encoding is stored once per sample, in its first slot's row;
+//    per-sample occupancy and compositing weights never reach HBM; the
+//    composited per-view tokens (4 x F floats per ray) do;
 //  * the view mean is folded into the occupancy head (mean of per-column dot
-//    products); compositing keeps the reference's sequential recurrence;
+//    products); compositing keeps the reference's sequential recurrence, run
+//    by every wave on values broadcast from the samples' lanes (one thread
+//    walking LDS, with a barrier before and after, made a chunk 12 barriers
+//    instead of 8: C2 bf16 frame 7.51 -> 6.95 ms together with the MFMAs' C
+//    operand taking the biases and the shared encoding);
 //  * Hydra + RGB head run in a second kernel over 16 rays (64 tokens) per
 //    workgroup: lane = token, so the 4 views of a ray are 4 adjacent lanes
 //    (cross-view sums are two shuffles), the weights are wave-uniform reads
@@ -64,8 +72,8 @@ enum Prec { kF32 = 0, kBF16 = 1, kF16 = 2 };
 constexpr int kThreads = kWaves * 64;
 constexpr int kVP = 4;       // view slots per sample (training form, point mode)
 constexpr int kMaxViews = 8;  // view slots of the 8-view rendering instantiations
-constexpr int kXcds = 8;      // accelerator dies of an MI355X (workgroups go round-robin)
 constexpr float kHalfPi = 1.5707963267948966f;
+constexpr int kXcds = 8;      // accelerator dies of an MI355X (workgroups go round-robin)
 
 struct RenderArgs {
   const float* t;          // [n_rays, S] sorted sample distances
@@ -122,6 +130,56 @@ template <> struct Tr<kF16> {
 };
 
 __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// sin(x) and cos(x) of a positional-encoding argument.  fp32 form: two sinf,
+// the cosine as sinf(x + pi/2) as freq_encoding.cu:37-45 writes it.  16-bit
+// forms: x minus the nearest multiple n of pi/2 (three fma with pi/2 split
+// into 24-bit parts, Cody-Waite), then odd / even polynomials on
+// [-pi/4, pi/4] (weighted least-squares minimax fits, 2e-9 and 1e-10 off), one
+// reduction for both values.  Against 64-bit values over |x| <= 1e6: rms
+// 2.1e-8, max 1e-7 (correctly rounded: 1.5e-8, 3e-8; x + pi/2 rounded to 32
+// bits makes the cosine of the other form up to 2.6e-5 off at |x| = 512).
+// Larger, infinite and NaN arguments take the library's.
+template <int PREC>
+__device__ __forceinline__ void sincos_pe(float x, float& s, float& c) {
+  if constexpr (PREC == kF32) {
+    s = sinf(x);
+    c = sinf(x + kHalfPi);
+    return;
+  }
+  if (!(fabsf(x) <= 1.0e6f)) {
+    s = sinf(x);
+    c = cosf(x);
+    return;
+  }
+  const float n = rintf(x * 0.63661977236758134f);
+  float r = fmaf(-n, 1.5707963705062866f, x);
+  r = fmaf(-n, -4.3711388286737929e-8f, r);
+  r = fmaf(-n, -1.7151245100059e-15f, r);
+  const float z = r * r;
+  float p = fmaf(-1.9494950539e-4f, z, 8.3319731057e-3f);
+  p = fmaf(p, z, -1.6666650772e-1f);
+  const float sr = fmaf(p, z * r, r);
+  float q = fmaf(2.4437731554e-5f, z, -1.3887361856e-3f);
+  q = fmaf(q, z, 4.1666645557e-2f);
+  const float cr = fmaf(q, z * z, fmaf(z, -0.5f, 1.0f));
+  const int m = (int)n;
+  const float ss = (m & 1) ? cr : sr, cc = (m & 1) ? sr : cr;
+  s = __int_as_float(__float_as_int(ss) ^ ((m << 30) & 0x80000000));
+  c = __int_as_float(__float_as_int(cc) ^ (((m + 1) << 30) & 0x80000000));
+}
+
+// LDS written by some lanes of a wave and read by others of the same wave:
+// the LDS serves a wave's accesses in order, so only the compiler has to be
+// kept from moving the reads up.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
 
 // One Kahan step: sum += x with the rounding error kept in comp (negated);
 // the compensated value is sum - comp.  (No fast-math here: the compiler
@@ -248,15 +306,17 @@ __device__ __forceinline__ void load_a(const char* base, int j, unsigned lane_of
   }
 }
 
-template <int H, int PREC, int NTL>
+// SH > 1: the unit's inputs are the same for the SH columns of a sample (the
+// positional encoding) and are stored in the first of their rows only.
+template <int H, int PREC, int NTL, int SH = 1>
 __device__ __forceinline__ void read_b(const typename Tr<PREC>::E* act, int j, int n, int g,
                                        typename Chain<H, PREC, NTL>::V (&dst)[NTL]) {
   typedef Chain<H, PREC, NTL> C;
   // unit j covers chunks 4j..4j+3; lane group g reads chunk 4j + g
 #pragma unroll
   for (int nt = 0; nt < NTL; ++nt)
-    dst[nt] = *reinterpret_cast<const typename C::V*>(act + act_chunk<H, PREC>(16 * nt + n,
-                                                                               4 * j + g));
+    dst[nt] = *reinterpret_cast<const typename C::V*>(
+        act + act_chunk<H, PREC>((16 * nt + n) & ~(SH - 1), 4 * j + g));
 }
 
 // UL units of one layer whose first PD units are already in the A buffers
@@ -265,7 +325,8 @@ __device__ __forceinline__ void read_b(const typename Tr<PREC>::E* act, int j, i
 // at `nxt`.  The scheduling barriers keep both prefetches where they are
 // written: left alone, the scheduler sinks the loads next to their first use
 // and exposes the full memory latency at every unit.
-template <int H, int PREC, int NTL, int UL, int O>
+// SH, JS: units from JS on read the rows shared by SH columns (read_b).
+template <int H, int PREC, int NTL, int UL, int O, int SH = 1, int JS = UL>
 __device__ __forceinline__ void run_layer(
     const char* cur, const char* nxt, unsigned lane_off, const typename Tr<PREC>::E* act, int n,
     int g, typename Chain<H, PREC, NTL>::V (&abuf)[Chain<H, PREC, NTL>::NB][Chain<H, PREC, NTL>::AN],
@@ -278,7 +339,10 @@ __device__ __forceinline__ void run_layer(
       load_a<H, PREC, NTL>(cur, j + PD, lane_off, abuf[(O + j + PD) % NB]);
     else
       load_a<H, PREC, NTL>(nxt, j + PD - UL, lane_off, abuf[(O + j + PD) % NB]);
-    if (j + 1 < UL) read_b<H, PREC, NTL>(act, j + 1, n, g, bbuf[(j + 1) & 1]);
+    if (j + 1 < UL) {
+      if (j + 1 < JS) read_b<H, PREC, NTL>(act, j + 1, n, g, bbuf[(j + 1) & 1]);
+      else read_b<H, PREC, NTL, SH>(act, j + 1, n, g, bbuf[(j + 1) & 1]);
+    }
     __builtin_amdgcn_sched_barrier(0);
     const typename C::V (&A)[C::AN] = abuf[(O + j) % NB];
     const typename C::V (&Bv)[NTL] = bbuf[j & 1];
@@ -313,7 +377,9 @@ __device__ __forceinline__ void run_layer(
 // Layer l's weights for wave w are [w][unit][lane][m-tile][slot] (see
 // mlp_layout.h); the weight prefetch runs across layer boundaries so the
 // loads of a layer's first units overlap the previous layer's epilogue.
-template <int H, int PREC, int NTL, int K0>
+// F < K0: inputs F .. K0 - 1 of layer 0 are shared by the VP columns of a
+// sample (read_b).
+template <int H, int PREC, int NTL, int K0, int F, int VP>
 __device__ __forceinline__ void dense_chain(const typename Tr<PREC>::E* __restrict__ W,
                                             typename Tr<PREC>::E* act,
                                             const float* __restrict__ s_bias, int wave,
@@ -347,7 +413,9 @@ __device__ __forceinline__ void dense_chain(const typename Tr<PREC>::E* __restri
 #pragma unroll
   for (int j = 0; j < PD; ++j) load_a<H, PREC, NTL>(wb0, j, lane_off, abuf[(O0 + j) % NB]);
   read_b<H, PREC, NTL>(act, 0, n, g, bbuf[0]);
-  run_layer<H, PREC, NTL, U0, O0>(wb0, wbh, lane_off, act, n, g, abuf, bbuf, acc);
+  static_assert(F % C::KPU == 0, "features fill whole units");
+  run_layer<H, PREC, NTL, U0, O0, VP, F / C::KPU>(wb0, wbh, lane_off, act, n, g, abuf, bbuf,
+                                                  acc);
 #pragma unroll 1
   for (int l = 1; l < 4; ++l) {
     __syncthreads();  // every wave finished reading act
@@ -395,21 +463,39 @@ __device__ __forceinline__ void load_a16(const char* base, int j, unsigned lane_
 }
 
 // k-step j covers chunks 2j, 2j+1 of a column; lanes l/32 = h read chunk 2j+h
-template <int H, int PREC, int NT>
+// (SH as in read_b)
+template <int H, int PREC, int NT, int SH = 1>
 __device__ __forceinline__ void read_b16(const typename Tr<PREC>::E* act, int j, int lane,
                                          typename Chain16<H, PREC, NT>::V (&dst)[NT]) {
   typedef Chain16<H, PREC, NT> C;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
     dst[nt] = *reinterpret_cast<const typename C::V*>(
-        act + act_chunk<H, PREC>(32 * nt + (lane & 31), 2 * j + (lane >> 5)));
+        act + act_chunk<H, PREC>((32 * nt + (lane & 31)) & ~(SH - 1), 2 * j + (lane >> 5)));
 }
 
-template <int H, int PREC, int NT, int UL, int O>
+// This wave's biases of a layer in the accumulator layout: the first k-step's
+// MFMA takes them as its C operand, so accumulators need neither clearing nor
+// a bias add (2 x 16 NT M32 vector instructions per layer and wave before).
+template <int H>
+__device__ __forceinline__ void load_bias16(const float* bias, int wave, int lane,
+                                            f32x16 (&bc)[H / 128]) {
+#pragma unroll
+  for (int mt = 0; mt < H / 128; ++mt)
+#pragma unroll
+    for (int q = 0; q < 16; q += 4) {
+      const f32x4 b4 = *reinterpret_cast<const f32x4*>(bias + unit_of32<H>(wave, mt, lane >> 5, q));
+      bc[mt][q] = b4[0]; bc[mt][q + 1] = b4[1]; bc[mt][q + 2] = b4[2]; bc[mt][q + 3] = b4[3];
+    }
+}
+
+// acc = bc + W x; SH, JS as in run_layer.
+template <int H, int PREC, int NT, int UL, int O, int SH = 1, int JS = UL>
 __device__ __forceinline__ void run_layer16(
     const char* cur, const char* nxt, unsigned lane_off, const typename Tr<PREC>::E* act,
     int lane, typename Chain16<H, PREC, NT>::V (&abuf)[Chain16<H, PREC, NT>::NB][H / 128],
-    typename Chain16<H, PREC, NT>::V (&bbuf)[2][NT], f32x16 (&acc)[H / 128][NT]) {
+    typename Chain16<H, PREC, NT>::V (&bbuf)[2][NT], const f32x16 (&bc)[H / 128],
+    f32x16 (&acc)[H / 128][NT]) {
   typedef Chain16<H, PREC, NT> C;
   constexpr int NB = C::NB, PD = C::PD;
 #pragma unroll
@@ -418,48 +504,44 @@ __device__ __forceinline__ void run_layer16(
       load_a16<H, PREC, NT>(cur, j + PD, lane_off, abuf[(O + j + PD) % NB]);
     else
       load_a16<H, PREC, NT>(nxt, j + PD - UL, lane_off, abuf[(O + j + PD) % NB]);
-    if (j + 1 < UL) read_b16<H, PREC, NT>(act, j + 1, lane, bbuf[(j + 1) & 1]);
+    if (j + 1 < UL) {
+      if (j + 1 < JS) read_b16<H, PREC, NT>(act, j + 1, lane, bbuf[(j + 1) & 1]);
+      else read_b16<H, PREC, NT, SH>(act, j + 1, lane, bbuf[(j + 1) & 1]);
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int mt = 0; mt < C::M32; ++mt) {
+        const f32x16 c = j == 0 ? bc[mt] : acc[mt][nt];
         if constexpr (PREC == kBF16)
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(abuf[(O + j) % NB][mt],
-                                                                bbuf[j & 1][nt], acc[mt][nt],
-                                                                0, 0, 0);
+                                                                bbuf[j & 1][nt], c, 0, 0, 0);
         else
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(abuf[(O + j) % NB][mt],
-                                                               bbuf[j & 1][nt], acc[mt][nt],
-                                                               0, 0, 0);
+                                                               bbuf[j & 1][nt], c, 0, 0, 0);
       }
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// act[col][unit] = relu(acc + bias) for this wave's units (two 16-byte stores
-// per m-tile and column).
+// act[col][unit] = relu(acc) for this wave's units (two 16-byte stores per
+// m-tile and column); the accumulators hold the bias already.
 template <int H, int PREC, int NT>
-__device__ __forceinline__ void write_act16(typename Tr<PREC>::E* act, const float* bias,
-                                            int wave, int lane, const f32x16 (&acc)[H / 128][NT]) {
+__device__ __forceinline__ void write_act16(typename Tr<PREC>::E* act, int wave, int lane,
+                                            const f32x16 (&acc)[H / 128][NT]) {
   typedef typename Tr<PREC>::E E;
   const int c = lane & 31, h = lane >> 5;
 #pragma unroll
   for (int mt = 0; mt < H / 128; ++mt) {
     const int u0 = unit_of32<H>(wave, mt, h, 0);
-    float bv[16];
-#pragma unroll
-    for (int q = 0; q < 16; q += 4) {
-      const f32x4 b4 = *reinterpret_cast<const f32x4*>(bias + u0 + q);
-      bv[q] = b4[0]; bv[q + 1] = b4[1]; bv[q + 2] = b4[2]; bv[q + 3] = b4[3];
-    }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         typename Tr<PREC>::V8 v;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = (E)fmaxf(acc[mt][nt][8 * e + k] + bv[8 * e + k], 0.0f);
+        for (int k = 0; k < 8; ++k) v[k] = (E)fmaxf(acc[mt][nt][8 * e + k], 0.0f);
         *reinterpret_cast<typename Tr<PREC>::V8*>(act + act_chunk<H, PREC>(32 * nt + c,
                                                                            u0 / 8 + e)) = v;
       }
@@ -467,14 +549,16 @@ __device__ __forceinline__ void write_act16(typename Tr<PREC>::E* act, const flo
   }
 }
 
-template <int H, int PREC, int NT, int K0>
+// The four dense layers of a chunk (dense_chain's 16-bit form); the last
+// layer's accumulators hold its bias, the caller applies its ReLU.
+template <int H, int PREC, int NT, int K0, int F, int VP>
 __device__ __forceinline__ void dense_chain16(const typename Tr<PREC>::E* __restrict__ W,
                                               typename Tr<PREC>::E* act,
                                               const float* __restrict__ s_bias, int wave,
                                               int lane, f32x16 (&acc)[H / 128][NT]) {
   typedef Chain16<H, PREC, NT> C;
   constexpr int U0 = K0 / 16, UH = C::UH, NB = C::NB, PD = C::PD, M32 = C::M32;
-  static_assert(K0 % 16 == 0, "layer widths must fill whole k-steps");
+  static_assert(K0 % 16 == 0 && F % 16 == 0, "layer widths must fill whole k-steps");
   constexpr int O0 = (NB - U0 % NB) % NB;   // so that layer 1 starts at buffer 0
   const char* wb0 = reinterpret_cast<const char*>(W) + (size_t)wave * U0 * C::unit_bytes;
   const char* wbh = reinterpret_cast<const char*>(W) + (size_t)kWaves * U0 * C::unit_bytes +
@@ -485,29 +569,23 @@ __device__ __forceinline__ void dense_chain16(const typename Tr<PREC>::E* __rest
 
   typename C::V abuf[NB][M32];
   typename C::V bbuf[2][NT];
-  auto zero = [&]() {
-#pragma unroll
-    for (int mt = 0; mt < M32; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
-  };
-  zero();
+  f32x16 bc[M32];
 #pragma unroll
   for (int j = 0; j < PD; ++j) load_a16<H, PREC, NT>(wb0, j, lane_off, abuf[(O0 + j) % NB]);
+  load_bias16<H>(s_bias, wave, lane, bc);
   read_b16<H, PREC, NT>(act, 0, lane, bbuf[0]);
-  run_layer16<H, PREC, NT, U0, O0>(wb0, wbh, lane_off, act, lane, abuf, bbuf, acc);
+  run_layer16<H, PREC, NT, U0, O0, VP, F / 16>(wb0, wbh, lane_off, act, lane, abuf, bbuf, bc,
+                                               acc);
 #pragma unroll 1
   for (int l = 1; l < 4; ++l) {
     __syncthreads();  // every wave finished reading act
-    write_act16<H, PREC, NT>(act, s_bias + (l - 1) * H, wave, lane, acc);
-    zero();
+    write_act16<H, PREC, NT>(act, wave, lane, acc);
+    load_bias16<H>(s_bias + l * H, wave, lane, bc);
     __syncthreads();
     read_b16<H, PREC, NT>(act, 0, lane, bbuf[0]);
     const char* cur = wbh + (size_t)(l - 1) * lh_bytes;
     const char* nxt = l < 3 ? cur + lh_bytes : cur;  // the last layer re-reads its own head
-    run_layer16<H, PREC, NT, UH, 0>(cur, nxt, lane_off, act, lane, abuf, bbuf, acc);
+    run_layer16<H, PREC, NT, UH, 0>(cur, nxt, lane_off, act, lane, abuf, bbuf, bc, acc);
   }
 }
 
@@ -521,16 +599,10 @@ struct Smem {
   static constexpr int KF = F + 4;
   static constexpr size_t keep = (act + act_bytes + 15) / 16 * 16;      // f32 [NS][VP][KF]
   static constexpr size_t sig = keep + (size_t)NS * VP * KF * 4;       // f32 [4][NC]
-  static constexpr size_t alpha = sig + (size_t)kWaves * NC * 4;       // f32 [NS]
-  static constexpr size_t tval = alpha + (size_t)NS * 4;               // f32 [NS]
-  static constexpr size_t wts = tval + (size_t)NS * 4;                 // f32 [NS]
-  static constexpr size_t flag = wts + (size_t)NS * 4;                 // int [4]
-  // f32 [4][H] layer biases, then (fp32 form) [H] the occupancy weights;
-  // the 16-bit forms read those from L1, which keeps their 24-sample chunks
-  // within two workgroups per CU
-  static constexpr size_t bias = flag + 16;
-  static constexpr size_t pos = bias + (size_t)(PREC == kF32 ? 5 : 4) * H * 4;  // f32 [NS][4]
-  static constexpr size_t total = pos + (size_t)NS * 16;
+  // f32 [4][H] layer biases, then [H] the occupancy weights: 80 KB in all for
+  // the 16-bit forms' 24-sample chunks at H = 256, two workgroups per CU
+  static constexpr size_t bias = sig + (size_t)kWaves * NC * 4;
+  static constexpr size_t total = bias + (size_t)5 * H * 4;
 };
 
 constexpr size_t kLdsBytes = 160 * 1024;  // LDS per workgroup on gfx950
@@ -598,6 +670,48 @@ __device__ __forceinline__ void gather_quarter(const RenderArgs& a, int b, int v
   }
 }
 
+// The four taps of gather_quarter's bilinear sample at world point (x, y, z)
+// in view v of batch b: pixel index within the view's map, -1 where the tap
+// contributes nothing (outside the map, behind the camera, v >= V), and weight.
+__device__ __forceinline__ void project_taps(const RenderArgs& a, int b, int v, float x, float y,
+                                             float z, int (&pix)[4], float (&wt)[4]) {
+#pragma unroll
+  for (int tap = 0; tap < 4; ++tap) {
+    pix[tap] = -1;
+    wt[tap] = 0.0f;
+  }
+  if (v >= a.V) return;
+  const float* RT = a.RTv + ((size_t)b * a.V + v) * 12;
+  const float* K = a.Kv + ((size_t)b * a.V + v) * 9;
+  float px = RT[0] * x + RT[1] * y + RT[2] * z + RT[3];
+  float py = RT[4] * x + RT[5] * y + RT[6] * z + RT[7];
+  const float pz = RT[8] * x + RT[9] * y + RT[10] * z + RT[11];
+  if (!(pz >= 0.01f)) return;
+  px /= pz;
+  py /= pz;
+  const float u = K[0] * px + K[1] * py + K[2];
+  const float w = K[3] * px + K[4] * py + K[5];
+  const float hw = (float)(a.img_w / 2), hh2 = (float)(a.img_h / 2);
+  const float gx = (u - hw) / hw, gy = (w - hh2) / hh2;
+  const float ix = (gx + 1.0f) * 0.5f * (float)(a.Wf - 1);
+  const float iy = (gy + 1.0f) * 0.5f * (float)(a.Hf - 1);
+  if (!(ix > -1.0f && ix < (float)a.Wf && iy > -1.0f && iy < (float)a.Hf)) return;
+  const float fx0 = floorf(ix), fy0 = floorf(iy);
+  const int x0 = (int)fx0, y0 = (int)fy0;
+  const float ax = ix - fx0, ay = iy - fy0;
+#pragma unroll
+  for (int tap = 0; tap < 4; ++tap) {
+    const int xx = x0 + (tap & 1), yy = y0 + (tap >> 1);
+    if (xx < 0 || xx >= a.Wf || yy < 0 || yy >= a.Hf) continue;
+    wt[tap] = ((tap & 1) ? ax : 1.0f - ax) * ((tap >> 1) ? ay : 1.0f - ay);
+    pix[tap] = yy * a.Wf + xx;
+  }
+}
+
+// What taps that contribute nothing read, so that a map's infinities and NaN
+// never meet their zero weight.
+__device__ const f32x4 kZeroTap[2] = {};
+
 // Waves per SIMD the register allocation is fitted to: two workgroups per CU
 // let one workgroup's gather / compositing overlap the other's MFMA work.
 // (chunks of at most 96 columns -- up to 24 samples x 4 view slots -- of
@@ -618,26 +732,21 @@ render_kernel(RenderArgs a) {
   typedef Smem<F, H, PREC, NS, VP> L;
   constexpr int NC = L::NC, KF = L::KF, NTL = NC / 16, MTW = H / 64;
   constexpr int CE = Tr<PREC>::CE;
-  constexpr int CPL = F / 4;
   constexpr int K0 = F + kPeSlots;
-  constexpr int STEP = PREC == kF32 ? 4 : 32;
-  constexpr int KS0 = K0 / STEP, KSH = H / STEP;
-  constexpr int EPL = Tr<PREC>::EPL;
   constexpr SmallOffsets so = small_offsets(F, H);
-  static_assert(K0 <= H, "first-layer input must fit an activation row");
-  static_assert(CPL % CE == 0 && F % CE == 0, "feature quarters must fill whole chunks");
-  constexpr int TE = (VP * F + kThreads - 1) / kThreads;  // token entries per thread
   static_assert(VP == 4 || VP == 8, "4 or 8 view slots");
+  constexpr int VPW = VP / kWaves;       // view slots of a wave: wave, wave + 4
+  constexpr int NP = F / 8;              // 8-channel parts of a tap's channel row
+  constexpr int ROUNDS = (NS * NP + 63) / 64;
+  constexpr int NSW = (NS + kWaves - 1) / kWaves;   // samples a wave encodes
+  constexpr int TAIL = K0 / CE;          // first chunk of a row that layer 0 does not read
+  static_assert(F <= 64 && NS <= 64, "a lane per channel, a lane per sample");
+  static_assert(K0 + 3 * CE <= H, "three spare chunks behind the first layer's input");
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   E* act = reinterpret_cast<E*>(smem + L::act);
   float* keep = reinterpret_cast<float*>(smem + L::keep);
   float* sig = reinterpret_cast<float*>(smem + L::sig);
-  float* s_alpha = reinterpret_cast<float*>(smem + L::alpha);
-  float* s_t = reinterpret_cast<float*>(smem + L::tval);
-  float* s_w = reinterpret_cast<float*>(smem + L::wts);
-  int* s_flag = reinterpret_cast<int*>(smem + L::flag);
-  float* s_pos = reinterpret_cast<float*>(smem + L::pos);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -646,11 +755,11 @@ render_kernel(RenderArgs a) {
   const E* W0 = reinterpret_cast<const E*>(a.wdense);
   float* s_bias = reinterpret_cast<float*>(smem + L::bias);
   // layer biases and the occupancy-head weights stay in LDS for the whole
-  // kernel (the first loop iteration's barrier publishes them)
+  // kernel (the first chunk's barrier publishes them)
   for (int i = tid; i < 4 * H; i += kThreads) s_bias[i] = a.bdense[i];
-  if constexpr (PREC == kF32)
-    for (int i = tid; i < H; i += kThreads) s_bias[4 * H + i] = ws[so.sigma_w + i];
+  for (int i = tid; i < H; i += kThreads) s_bias[4 * H + i] = ws[so.sigma_w + i];
   const float inv_v = 1.0f / (float)V;
+  const float sigma_b = ws[so.sigma_b];
 
   // every list entry costs about the same, so a static stride over the
   // compacted list balances the workgroups (dropped rays were finished by the
@@ -668,7 +777,6 @@ render_kernel(RenderArgs a) {
   const long long item_lo = band * xcd;
   const long long item_hi = item_lo + band < n_items ? item_lo + band : n_items;
   for (long long item = item_lo + wg_in_xcd; item < item_hi; item += wgs_of_xcd) {
-    __syncthreads();  // LDS of the previous ray is no longer read
     const long long ray = POINTS ? item : (long long)a.list[item];
     const int b = (int)(ray / a.rays_per_batch);
     const long long p0 = (ray % a.rays_per_batch) * NS;  // point mode: first point
@@ -682,119 +790,191 @@ render_kernel(RenderArgs a) {
                 cz = 0.5f * (bb[4] + bb[5]);
     const float ihx = 2.0f / (bb[1] - bb[0]), ihy = 2.0f / (bb[3] - bb[2]),
                 ihz = 2.0f / (bb[5] - bb[4]);
-    // compositing state lives in thread 0; tokens: thread (v, c) = (tid / F, tid % F)
-    float T = 1.0f, dsum = 0.0f, wsum = 0.0f, asum = 0.0f;
-    float dcmp = 0.0f, wcmp = 0.0f, acmp = 0.0f;  // compensated form: lost low bits
+    // compositing state, the same in every lane of every wave; wave 0 adds up
+    // the depth, wave 1 the weights, wave 2 the alphas, and lane c of wave w
+    // channel c of view slots w and w + 4
+    float T = 1.0f;
     bool done = false;
-    float tok[TE], tcmp[TE];
+    float sum = 0.0f, comp = 0.0f;         // comp: lost low bits (compensated form)
+    float tok[VPW], tcmp[VPW];
 #pragma unroll
-    for (int j = 0; j < TE; ++j) tok[j] = tcmp[j] = 0.0f;
-    if (tid == 0) s_flag[0] = 0;
+    for (int j = 0; j < VPW; ++j) tok[j] = tcmp[j] = 0.0f;
 
     for (int c0 = 0; c0 < S; c0 += NS) {
-      __syncthreads();
-      if (a.early_exit && s_flag[0]) break;
-      // sample positions of the chunk: o + t d, or the points themselves
-      if (tid < NS) {
-        float px, py, pz, tv = 0.0f;
+      // Everything up to the barrier is a wave's own: the view slots it
+      // samples are the ones it composites, so its kept features need no
+      // barrier against the previous chunk's use, and the rows' spare tails
+      // hold only its own projections.
+      // ---- sample positions (lane = sample), projections -------------------
+      float tv = 0.0f;
+      if (lane < NS) {
+        float px, py, pz;
         if constexpr (POINTS) {
-          const long long pi = p0 + tid < a.n_points ? p0 + tid : a.n_points - 1;
+          const long long pi = p0 + lane < a.n_points ? p0 + lane : a.n_points - 1;
           const float* q = a.points + ((long long)b * a.n_points + pi) * 3;
           px = q[0]; py = q[1]; pz = q[2];
         } else {
-          tv = trow[c0 + tid];
+          tv = trow[c0 + lane];
           px = ox + tv * dx; py = oy + tv * dy; pz = oz + tv * dz;
         }
-        s_pos[4 * tid + 0] = px; s_pos[4 * tid + 1] = py; s_pos[4 * tid + 2] = pz;
-        s_t[tid] = tv;
+#pragma unroll
+        for (int j = 0; j < VPW; ++j) {
+          const int v = wave + kWaves * j, col = lane * VP + v;
+          int pix[4];
+          float wt[4];
+          project_taps(a, b, v, px, py, pz, pix, wt);
+          *reinterpret_cast<int4*>(act + act_chunk<H, PREC>(col, TAIL)) =
+              make_int4(pix[0], pix[1], pix[2], pix[3]);
+          *reinterpret_cast<f32x4*>(act + act_chunk<H, PREC>(col, TAIL + 1)) =
+              f32x4{wt[0], wt[1], wt[2], wt[3]};
+        }
+        *reinterpret_cast<f32x4*>(act + act_chunk<H, PREC>(lane * VP + wave, TAIL + 2)) =
+            f32x4{(px - cx) * ihx, (py - cy) * ihy, (pz - cz) * ihz, 0.0f};
       }
-      __syncthreads();
-      // ---- first-layer input: bilinear features (4 threads per column; the
-      // 16 lanes of a quarter-wave take 16 columns of the same quarter) ------
-      for (int item = tid; item < NC * 4; item += kThreads) {
-        const int col = (item & 15) + 16 * (item >> 6), quarter = (item >> 4) & 3;
-        const int sl = col / VP, v = col % VP;
-        const float x = s_pos[4 * sl], y = s_pos[4 * sl + 1], z = s_pos[4 * sl + 2];
-        float f[CPL];
-        gather_quarter<F, PREC, HALF_MAP>(a, b, v, x, y, z, quarter, f);
-        float* kp = keep + col * KF + quarter * CPL;
+      wave_lds_fence();
+      // ---- first-layer input: bilinear features, a lane per 8 channels of a
+      // (sample, view); the loads of up to three rounds are in flight together
 #pragma unroll
-        for (int c = 0; c < CPL; c += 4)
-          *reinterpret_cast<f32x4*>(kp + c) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
-        // layer-0 input k = channel (k < F); 16-byte chunks, swizzled
-#pragma unroll
-        for (int c = 0; c < CPL; c += CE) {
-          E* dst = act + act_chunk<H, PREC>(col, (quarter * CPL + c) / CE);
+      for (int j = 0; j < VPW; ++j) {
+        const int v = wave + kWaves * j;
+        const size_t vbase = ((size_t)b * V + (v < V ? v : 0)) * a.Hf * a.Wf * F;
+        auto finish = [&](int it, const f32x4& w4, const float (&f)[8]) {
+          const int sl = it / NP, part = it % NP, col = sl * VP + v;
+          float* kp = keep + col * KF + part * 8;
+          *reinterpret_cast<f32x4*>(kp) = f32x4{f[0], f[1], f[2], f[3]};
+          *reinterpret_cast<f32x4*>(kp + 4) = f32x4{f[4], f[5], f[6], f[7]};
           if constexpr (PREC == kF32) {
-            *reinterpret_cast<f32x4*>(dst) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
+            *reinterpret_cast<f32x4*>(act + act_chunk<H, PREC>(col, 2 * part)) =
+                f32x4{f[0], f[1], f[2], f[3]};
+            *reinterpret_cast<f32x4*>(act + act_chunk<H, PREC>(col, 2 * part + 1)) =
+                f32x4{f[4], f[5], f[6], f[7]};
           } else {
             typename Tr<PREC>::V8 h;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) h[i] = (E)f[c + i];
-            *reinterpret_cast<typename Tr<PREC>::V8*>(dst) = h;
+            for (int i = 0; i < 8; ++i) h[i] = (E)f[i];
+            *reinterpret_cast<typename Tr<PREC>::V8*>(act + act_chunk<H, PREC>(col, part)) = h;
+          }
+        };
+        if constexpr (HALF_MAP) {
+          typedef typename Tr<PREC>::V8 V8;
+          const E* map = static_cast<const E*>(a.fmap) + vbase;
+          constexpr int RB = ROUNDS < 3 ? ROUNDS : 3;
+#pragma unroll
+          for (int r0 = 0; r0 < ROUNDS; r0 += RB) {
+            V8 raw[RB][4];
+            f32x4 w4[RB];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+              const int it = lane + 64 * (r0 + r);
+              if (r0 + r < ROUNDS && it < NS * NP) {
+                const int col = (it / NP) * VP + v;
+                const int4 px4 = *reinterpret_cast<const int4*>(act + act_chunk<H, PREC>(col, TAIL));
+                w4[r] = *reinterpret_cast<const f32x4*>(act + act_chunk<H, PREC>(col, TAIL + 1));
+                const int pix[4] = {px4.x, px4.y, px4.z, px4.w};
+#pragma unroll
+                for (int tap = 0; tap < 4; ++tap) {
+                  const E* src = map + (size_t)(unsigned)pix[tap] * F + (it % NP) * 8;
+                  raw[r][tap] = *reinterpret_cast<const V8*>(
+                      pix[tap] >= 0 ? src : reinterpret_cast<const E*>(kZeroTap));
+                }
+              }
+            }
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+              const int it = lane + 64 * (r0 + r);
+              if (r0 + r < ROUNDS && it < NS * NP) {
+                float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int tap = 0; tap < 4; ++tap)
+#pragma unroll
+                  for (int i = 0; i < 8; ++i) f[i] += w4[r][tap] * (float)raw[r][tap][i];
+                finish(it, w4[r], f);
+              }
+            }
+          }
+        } else {
+          const float* map = static_cast<const float*>(a.fmap) + vbase;
+#pragma unroll 1
+          for (int it = lane; it < NS * NP; it += 64) {
+            const int col = (it / NP) * VP + v;
+            const int4 px4 = *reinterpret_cast<const int4*>(act + act_chunk<H, PREC>(col, TAIL));
+            const f32x4 w4 = *reinterpret_cast<const f32x4*>(act + act_chunk<H, PREC>(col, TAIL + 1));
+            const int pix[4] = {px4.x, px4.y, px4.z, px4.w};
+            f32x4 raw[4][2];
+#pragma unroll
+            for (int tap = 0; tap < 4; ++tap) {
+              const float* src = map + (size_t)(unsigned)pix[tap] * F + (it % NP) * 8;
+              const f32x4* q = pix[tap] >= 0 ? reinterpret_cast<const f32x4*>(src) : kZeroTap;
+              raw[tap][0] = q[0];
+              raw[tap][1] = q[1];
+            }
+            float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int tap = 0; tap < 4; ++tap)
+#pragma unroll
+              for (int i = 0; i < 8; ++i) f[i] += w4[tap] * raw[tap][i / 4][i % 4];
+            finish(it, w4, f);
           }
         }
       }
-      // ---- positional encoding (freq_encoding.cu:37-45 layout), shared by views;
-      // a thread computes two adjacent slots and stores them as one pair
-      for (int item = tid; item < NS * kPeSlots / 2; item += kThreads) {
-        const int sl = item / (kPeSlots / 2), q0 = 2 * (item % (kPeSlots / 2));
-        float val[2];
+      // ---- positional encoding (freq_encoding.cu:37-45 layout), once per
+      // sample: into the row of its first view slot, which layer 0 reads for
+      // all of them.  A lane per (sample, frequency, axis).
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int q = q0 + h;
-          val[h] = 0.0f;
-          if (q < 63) {
-            const int d = q % 3;
-            const float xd = d == 0 ? (s_pos[4 * sl] - cx) * ihx
-                                    : (d == 1 ? (s_pos[4 * sl + 1] - cy) * ihy
-                                              : (s_pos[4 * sl + 2] - cz) * ihz);
-            if (q < 3) {
-              val[h] = xd;
-            } else {
-              const int col = q / 3 - 1;
-              val[h] = sinf(ldexpf(xd, col >> 1) + (float)(col & 1) * kHalfPi);
-            }
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < VP; ++v) {
-          const int col = sl * VP + v, k = F + q0;  // the pair never straddles a chunk
-          E* d2 = act + act_chunk<H, PREC>(col, k / CE) + k % CE;
-          if constexpr (PREC == kF32) {
-            *reinterpret_cast<f32x2*>(d2) = f32x2{val[0], val[1]};
-          } else {
-            typedef E E2 __attribute__((ext_vector_type(2)));
-            *reinterpret_cast<E2*>(d2) = E2{(E)val[0], (E)val[1]};
+      for (int r = 0; r < (NSW * 32 + 63) / 64; ++r) {
+        const int q = (lane & 31), sl = wave * NSW + 2 * r + (lane >> 5);
+        if (2 * r + (lane >> 5) < NSW && sl < NS) {
+          E* row = act;
+          const float* xn = reinterpret_cast<const float*>(
+              act + act_chunk<H, PREC>(sl * VP + wave, TAIL + 2));
+          auto put = [&](int k, float val) {
+            row[act_chunk<H, PREC>(sl * VP, k / CE) + k % CE] = (E)val;
+          };
+          if (q < 30) {
+            const int fr = q / 3, ax = q - 3 * fr;
+            float sn, cs;
+            sincos_pe<PREC>(ldexpf(xn[ax], fr), sn, cs);
+            put(F + 3 + 6 * fr + ax, sn);
+            put(F + 6 + 6 * fr + ax, cs);
+          } else if (q == 30) {
+            put(F + 0, xn[0]);
+            put(F + 1, xn[1]);
+            put(F + 2, xn[2]);
+            put(F + 63, 0.0f);
           }
         }
       }
       __syncthreads();
-      // ---- dense layers on MFMA --------------------------------------------
-      // ---- dense layers + occupancy head (per-column partial dot products) --
+      // ---- dense layers on MFMA + occupancy head (per-column dot products) --
       if constexpr (PREC != kF32) {
         constexpr int NT = NC / 32;
         static_assert(NC % 32 == 0, "16-bit forms need chunks of a multiple of 8 samples");
         f32x16 acc[H / 128][NT];
-        dense_chain16<H, PREC, NT, K0>(W0, act, s_bias, wave, lane, acc);
+        dense_chain16<H, PREC, NT, K0, F, VP>(W0, act, s_bias, wave, lane, acc);
         const int c = lane & 31, h = lane >> 5;
-        const float* bias = s_bias + 3 * H;
+        float part[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) part[nt] = 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < H / 128; ++mt) {
+          const int u0 = unit_of32<H>(wave, mt, h, 0);
+#pragma unroll
+          for (int r = 0; r < 16; r += 4) {
+            const f32x4 w4 = *reinterpret_cast<const f32x4*>(s_bias + 4 * H + u0 + r);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) part[nt] += w4[i] * fmaxf(acc[mt][nt][r + i], 0.0f);
+          }
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-          float part = 0.0f;
-#pragma unroll
-          for (int mt = 0; mt < H / 128; ++mt) {
-            const int u0 = unit_of32<H>(wave, mt, h, 0);
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              part += ws[so.sigma_w + u0 + r] * fmaxf(acc[mt][nt][r] + bias[u0 + r], 0.0f);
-          }
-          part += __shfl_xor(part, 32, 64);
-          if (h == 0) sig[wave * NC + 32 * nt + c] = part;
+          part[nt] += __shfl_xor(part[nt], 32, 64);
+          if (h == 0) sig[wave * NC + 32 * nt + c] = part[nt];
         }
       } else {
         f32x4 acc[MTW][NTL];
-        dense_chain<H, PREC, NTL, K0>(W0, act, s_bias, wave, lane, acc);
+        dense_chain<H, PREC, NTL, K0, F, VP>(W0, act, s_bias, wave, lane, acc);
         const int n = lane & 15, g = lane >> 4;
         const float* bias = s_bias + 3 * H;
 #pragma unroll
@@ -814,79 +994,83 @@ render_kernel(RenderArgs a) {
         }
       }
       __syncthreads();
-      if (tid < NS) {
-        float sum = 0.0f;
+      // ---- occupancy (lane = sample), in every wave --------------------------
+      float al = 0.0f;
+      if (lane < NS) {
+        float x = 0.0f;
         for (int v = 0; v < V; ++v)
-          for (int w = 0; w < kWaves; ++w) sum += sig[w * NC + tid * VP + v];
-        const float al = sigmoidf(sum * inv_v + ws[so.sigma_b]);
+#pragma unroll
+          for (int w = 0; w < kWaves; ++w) x += sig[w * NC + lane * VP + v];
+        al = sigmoidf(x * inv_v + sigma_b);
         if constexpr (POINTS) {
-          if (p0 + tid < a.n_points) a.out_occ[(long long)b * a.n_points + p0 + tid] = al;
+          if (wave == 0 && p0 + lane < a.n_points)
+            a.out_occ[(long long)b * a.n_points + p0 + lane] = al;
         } else {
-          s_alpha[tid] = al;
-          if (a.out_occ) a.out_occ[ray * S + c0 + tid] = al;
+          if (wave == 0 && a.out_occ) a.out_occ[ray * S + c0 + lane] = al;
         }
       }
       if constexpr (POINTS) continue;  // density query: no compositing (S == NS)
-      __syncthreads();
       // ---- front-to-back compositing (volume_rendering.cu:713-734) ---------
-      if (tid == 0) {
-        for (int sl = 0; sl < NS; ++sl) {
-          float w = 0.0f;
-          if (!done) {
-            const float al = s_alpha[sl];
-            w = al * T;
-            if (a.compensated) {
-              kahan_add(dsum, dcmp, w * s_t[sl]);
-              kahan_add(wsum, wcmp, w);
-              kahan_add(asum, acmp, w * al);
-            } else {
-              dsum += w * s_t[sl];
-              wsum += w;
-              asum += w * al;
-            }
-            T *= 1.0f - al;
-            if (T < a.t_thres) done = true;
-          }
-          s_w[sl] = w;
-        }
-        s_flag[0] = done ? 1 : 0;
+      // the transmittance runs in sample order on values broadcast from their
+      // lanes; a sample counts until the one that took T below the threshold
+      const float keep_al = 1.0f - al;
+      float Ti = 0.0f;
+#pragma unroll
+      for (int sl = 0; sl < NS; ++sl) {
+        if (lane == sl) Ti = T;
+        T *= lane_value(keep_al, sl);
       }
-      __syncthreads();
+      const unsigned long long low = __ballot(lane < NS && (c0 > 0 || lane > 0) && Ti < a.t_thres);
+      const int n_live = done ? 0 : (low ? __ffsll((long long)low) - 1 : NS);
+      const float w = lane < n_live ? al * Ti : 0.0f;
+      done = done || low != 0 || __builtin_amdgcn_readfirstlane((int)(T < a.t_thres));
+      // depth, weight and alpha sums in sample order, one per wave
+      if (wave < 3) {
+        const float q = lane < n_live ? (wave == 0 ? tv : (wave == 1 ? 1.0f : al)) : 0.0f;
+        if (a.compensated) {
+          for (int sl = 0; sl < n_live; ++sl)
+            kahan_add(sum, comp, lane_value(w, sl) * lane_value(q, sl));
+        } else {
+#pragma unroll
+          for (int sl = 0; sl < NS; ++sl) {
+            const float qs = lane_value(q, sl);
+            sum = fmaf(lane_value(w, sl), qs, sum);
+          }
+        }
+      }
       // ---- per-view tokens: sum_i w_i f_v(x_i) -----------------------------
 #pragma unroll
-      for (int j = 0; j < TE; ++j) {
-        const int e = tid + j * kThreads;
-        if (e < VP * F) {
-          const int v = e / F, c = e % F;
-          if (a.compensated) {
-            for (int sl = 0; sl < NS; ++sl)
-              kahan_add(tok[j], tcmp[j], s_w[sl] * keep[(sl * VP + v) * KF + c]);
-          } else {
-#pragma unroll 4
-            for (int sl = 0; sl < NS; ++sl) tok[j] += s_w[sl] * keep[(sl * VP + v) * KF + c];
-          }
+      for (int j = 0; j < VPW; ++j) {
+        const float* kp = keep + (wave + kWaves * j) * KF + (F == 64 ? lane : lane & (F - 1));
+        if (a.compensated) {
+          for (int sl = 0; sl < NS; ++sl)
+            kahan_add(tok[j], tcmp[j], lane_value(w, sl) * kp[sl * VP * KF]);
+        } else {
+#pragma unroll
+          for (int sl = 0; sl < NS; ++sl) tok[j] += lane_value(w, sl) * kp[sl * VP * KF];
         }
       }
+      if (a.early_exit && done) break;
+      wave_lds_fence();
     }
-    __syncthreads();
     if constexpr (!POINTS) {
       // ---- outputs: per-view tokens for the Hydra/RGB kernel, depth, sums --
+      if (F == 64 || lane < F) {
+        // quantised maps hold x / s_c: a power-of-two scale restores the
+        // token exactly
+        const float sc = a.fscale ? a.fscale[lane] : 1.0f;
 #pragma unroll
-      for (int j = 0; j < TE; ++j) {
-        const int e = tid + j * kThreads;
-        if (e < VP * F) {
-          // quantised maps hold x / s_c: a power-of-two scale restores the
-          // token exactly
-          const float sc = a.fscale ? a.fscale[e % F] : 1.0f;
-          a.out_tok[item * VP * F + e] = (e / F) < V ? (tok[j] - tcmp[j]) * sc : 0.0f;
+        for (int j = 0; j < VPW; ++j) {
+          const int v = wave + kWaves * j;
+          a.out_tok[(item * VP + v) * F + lane] = v < V ? (tok[j] - tcmp[j]) * sc : 0.0f;
         }
       }
-      if (tid == 0) {
-        const float* zd = a.zdir + b * 3;
-        a.out_depth[ray] = (dsum - dcmp) * (zd[0] * dx + zd[1] * dy + zd[2] * dz);
-        if (a.out_aux) {
-          a.out_aux[ray * 2 + 0] = wsum - wcmp;
-          a.out_aux[ray * 2 + 1] = asum - acmp;
+      if (lane == 0) {
+        if (wave == 0) {
+          const float* zd = a.zdir + b * 3;
+          a.out_depth[ray] = (sum - comp) * (zd[0] * dx + zd[1] * dy + zd[2] * dz);
+        } else if (wave < 3 && a.out_aux) {
+          a.out_aux[ray * 2 + wave - 1] = sum - comp;
         }
       }
     }
@@ -1386,11 +1570,12 @@ __device__ __forceinline__ void one_layer(const typename Tr<PREC>::E* Wl,
   run_layer<H, PREC, NTL, UL, 0>(wb, wb, lane_off, in, n, g, abuf, bbuf, acc);
 }
 
-// The same for the 16-bit forms (32x32x16 MFMA, NT column tiles of 32).
+// The same for the 16-bit forms (32x32x16 MFMA, NT column tiles of 32), plus
+// the layer's biases in LDS where given.
 template <int H, int PREC, int NT, int K>
 __device__ __forceinline__ void one_layer16(const typename Tr<PREC>::E* Wl,
-                                            const typename Tr<PREC>::E* in, int wave, int lane,
-                                            f32x16 (&acc)[H / 128][NT]) {
+                                            const typename Tr<PREC>::E* in, const float* bias,
+                                            int wave, int lane, f32x16 (&acc)[H / 128][NT]) {
   typedef Chain16<H, PREC, NT> C;
   constexpr int UL = K / 16, NB = C::NB, PD = C::PD;
   static_assert(K % 16 == 0, "layer width must fill whole k-steps");
@@ -1399,16 +1584,19 @@ __device__ __forceinline__ void one_layer16(const typename Tr<PREC>::E* Wl,
   const unsigned lane_off = (unsigned)lane * C::M32 * 16;
   typename C::V abuf[NB][C::M32];
   typename C::V bbuf[2][NT];
-#pragma unroll
-  for (int mt = 0; mt < C::M32; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
+  f32x16 bc[C::M32];
 #pragma unroll
   for (int j = 0; j < PD; ++j) load_a16<H, PREC, NT>(wb, j, lane_off, abuf[j % NB]);
+  if (bias) {
+    load_bias16<H>(bias, wave, lane, bc);
+  } else {
+#pragma unroll
+    for (int mt = 0; mt < C::M32; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bc[mt][r] = 0.0f;
+  }
   read_b16<H, PREC, NT>(in, 0, lane, bbuf[0]);
-  run_layer16<H, PREC, NT, UL, 0>(wb, wb, lane_off, in, lane, abuf, bbuf, acc);
+  run_layer16<H, PREC, NT, UL, 0>(wb, wb, lane_off, in, lane, abuf, bbuf, bc, acc);
 }
 
 // Copies NC columns x K elements of a swizzled LDS buffer to rows of a
@@ -1733,36 +1921,28 @@ render_backward_kernel(BackArgs ba) {
           *reinterpret_cast<typename Tr<PREC>::V8*>(d) = h;
         }
       }
-      for (int it = t0; it < NS * kPeSlots / 2; it += tstep) {
-        const int sl = it / (kPeSlots / 2), q0 = 2 * (it % (kPeSlots / 2));
+      // positional encoding: a thread per (sample, frequency, axis) -> its sine
+      // and cosine in the rows of the sample's view slots
+      for (int it = t0; it < NS * 32; it += tstep) {
+        const int sl = it >> 5, q = it & 31;
         const float* ps = s_pos + 4 * (c0 + sl);
-        float val[2];
+        const float xn[3] = {(ps[0] - cx) * ihx, (ps[1] - cy) * ihy, (ps[2] - cz) * ihz};
+        auto put = [&](int k, float val) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int q = q0 + h;
-          val[h] = 0.0f;
-          if (q < 63) {
-            const int d = q % 3;
-            const float xd = d == 0 ? (ps[0] - cx) * ihx
-                                    : (d == 1 ? (ps[1] - cy) * ihy : (ps[2] - cz) * ihz);
-            if (q < 3) {
-              val[h] = xd;
-            } else {
-              const int col = q / 3 - 1;
-              val[h] = sinf(ldexpf(xd, col >> 1) + (float)(col & 1) * kHalfPi);
-            }
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < kVP; ++v) {
-          const int col = sl * kVP + v, k = F + q0;
-          E* d2 = x0 + act_chunk<H, PREC>(col, k / CE) + k % CE;
-          if constexpr (F32) {
-            *reinterpret_cast<f32x2*>(d2) = f32x2{val[0], val[1]};
-          } else {
-            typedef E E2 __attribute__((ext_vector_type(2)));
-            *reinterpret_cast<E2*>(d2) = E2{(E)val[0], (E)val[1]};
-          }
+          for (int v = 0; v < kVP; ++v)
+            x0[act_chunk<H, PREC>(sl * kVP + v, k / CE) + k % CE] = (E)val;
+        };
+        if (q < 30) {
+          const int fr = q / 3, ax = q - 3 * fr;
+          float sn, cs;
+          sincos_pe<PREC>(ldexpf(ax == 0 ? xn[0] : (ax == 1 ? xn[1] : xn[2]), fr), sn, cs);
+          put(F + 3 + 6 * fr + ax, sn);
+          put(F + 6 + 6 * fr + ax, cs);
+        } else if (q == 30) {
+          put(F + 0, xn[0]);
+          put(F + 1, xn[1]);
+          put(F + 2, xn[2]);
+          put(F + 63, 0.0f);
         }
       }
     };
@@ -1865,16 +2045,16 @@ render_backward_kernel(BackArgs ba) {
         }
       } else {
         f32x16 acc[H / 128][NT32];
-        one_layer16<H, PREC, NT32, K0>(W, x0, wave, lane, acc);
-        write_act16<H, PREC, NT32>(hb(0), s_bias, wave, lane, acc);
+        one_layer16<H, PREC, NT32, K0>(W, x0, s_bias, wave, lane, acc);
+        write_act16<H, PREC, NT32>(hb(0), wave, lane, acc);
         __syncthreads();
-        one_layer16<H, PREC, NT32, H>(W + l0e, hb(0), wave, lane, acc);
-        write_act16<H, PREC, NT32>(hb(1), s_bias + H, wave, lane, acc);
+        one_layer16<H, PREC, NT32, H>(W + l0e, hb(0), s_bias + H, wave, lane, acc);
+        write_act16<H, PREC, NT32>(hb(1), wave, lane, acc);
         __syncthreads();
-        one_layer16<H, PREC, NT32, H>(W + l0e + lhe, hb(1), wave, lane, acc);
-        write_act16<H, PREC, NT32>(hb(2), s_bias + 2 * H, wave, lane, acc);
+        one_layer16<H, PREC, NT32, H>(W + l0e + lhe, hb(1), s_bias + 2 * H, wave, lane, acc);
+        write_act16<H, PREC, NT32>(hb(2), wave, lane, acc);
         __syncthreads();
-        one_layer16<H, PREC, NT32, H>(W + l0e + 2 * lhe, hb(2), wave, lane, acc);
+        one_layer16<H, PREC, NT32, H>(W + l0e + 2 * lhe, hb(2), s_bias + 3 * H, wave, lane, acc);
         {
           const int c = lane & 31, h = lane >> 5;
 #pragma unroll
@@ -1887,7 +2067,7 @@ render_backward_kernel(BackArgs ba) {
 #pragma unroll
               for (int r = 0; r < 16; ++r) {
                 const int u = unit_of32<H>(wave, mt, h, r);
-                const float pre = acc[mt][nt][r] + s_bias[3 * H + u];
+                const float pre = acc[mt][nt][r];
                 gsw[16 * mt + r] += dzc * fmaxf(pre, 0.0f);
                 acc[mt][nt][r] = pre > 0.0f ? dzc * s_bias[4 * H + u] : 0.0f;
               }
@@ -1906,7 +2086,7 @@ render_backward_kernel(BackArgs ba) {
         void* Ds[3] = {ba.D2, ba.D1, ba.D0};
 #pragma unroll
         for (int l = 0; l < 3; ++l) {
-          one_layer16<H, PREC, NT32, H>(WT + l * lhe, dl, wave, lane, acc);
+          one_layer16<H, PREC, NT32, H>(WT + l * lhe, dl, nullptr, wave, lane, acc);
           __syncthreads();
           write_vals16<H, PREC, NT32>(dl, acc, hb(2 - l), wave, lane);
           __syncthreads();
