@@ -68,6 +68,17 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
+// Pointers that went through an opaque asm or a select are generic to the
+// compiler, and a generic (flat) load counts against the LDS counter too:
+// every wait for an LDS operand then waited for the weight fragments
+// prefetched behind it.  Loads of device memory say so.
+#define SAILOR_GLOBAL __attribute__((address_space(1)))
+template <typename T>
+__device__ __forceinline__ T load_global(const void* p) {
+  return *reinterpret_cast<const SAILOR_GLOBAL T*>(
+      (const SAILOR_GLOBAL char*)(static_cast<const char*>(p)));
+}
+
 enum Prec { kF32 = 0, kBF16 = 1, kF16 = 2 };
 constexpr int kThreads = kWaves * 64;
 constexpr int kVP = 4;       // view slots per sample (training form, point mode)
@@ -128,6 +139,19 @@ template <> struct Tr<kF16> {
   typedef f16x4 V4;
   static constexpr int EPL = 8, CE = 8;
 };
+
+// max(x, 0), 0 for a NaN: what fmaxf gives, in one instruction (the median
+// of x, 0 and infinity; of a NaN the minimum of the others).  fmaxf on a
+// matrix accumulator takes two, the first to quiet it.  `inf` is infinity
+// the compiler does not see (opaque_inf), or it would write fmaxf again.
+__device__ __forceinline__ float relu(float x, float inf) {
+  return __builtin_amdgcn_fmed3f(x, 0.0f, inf);
+}
+__device__ __forceinline__ float opaque_inf() {
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  return inf;
+}
 
 __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
 
@@ -293,16 +317,16 @@ __device__ __forceinline__ void load_a(const char* base, int j, unsigned lane_of
     for (int i = 0; i < 4; ++i) {
       const char* ap = ub + (size_t)i * 64 * C::MTW * sizeof(float);
       if constexpr (C::MTW == 4) {
-        dst[i] = *reinterpret_cast<const f32x4*>(ap);
+        dst[i] = load_global<f32x4>(ap);
       } else {
-        const f32x2 v = *reinterpret_cast<const f32x2*>(ap);
+        const f32x2 v = load_global<f32x2>(ap);
         dst[i] = f32x4{v[0], v[1], 0.f, 0.f};
       }
     }
   } else {
     const typename C::V* ap = reinterpret_cast<const typename C::V*>(ub);
 #pragma unroll
-    for (int mt = 0; mt < C::MTW; ++mt) dst[mt] = ap[mt];
+    for (int mt = 0; mt < C::MTW; ++mt) dst[mt] = load_global<typename C::V>(ap + mt);
   }
 }
 
@@ -459,7 +483,7 @@ __device__ __forceinline__ void load_a16(const char* base, int j, unsigned lane_
   const typename C::V* ap =
       reinterpret_cast<const typename C::V*>(base + (size_t)j * C::unit_bytes + lane_off);
 #pragma unroll
-  for (int mt = 0; mt < C::M32; ++mt) dst[mt] = ap[mt];
+  for (int mt = 0; mt < C::M32; ++mt) dst[mt] = load_global<typename C::V>(ap + mt);
 }
 
 // k-step j covers chunks 2j, 2j+1 of a column; lanes l/32 = h read chunk 2j+h
@@ -532,6 +556,7 @@ __device__ __forceinline__ void write_act16(typename Tr<PREC>::E* act, int wave,
                                             const f32x16 (&acc)[H / 128][NT]) {
   typedef typename Tr<PREC>::E E;
   const int c = lane & 31, h = lane >> 5;
+  const float inf = opaque_inf();
 #pragma unroll
   for (int mt = 0; mt < H / 128; ++mt) {
     const int u0 = unit_of32<H>(wave, mt, h, 0);
@@ -541,7 +566,7 @@ __device__ __forceinline__ void write_act16(typename Tr<PREC>::E* act, int wave,
       for (int e = 0; e < 2; ++e) {
         typename Tr<PREC>::V8 v;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = (E)fmaxf(acc[mt][nt][8 * e + k], 0.0f);
+        for (int k = 0; k < 8; ++k) v[k] = (E)relu(acc[mt][nt][8 * e + k], inf);
         *reinterpret_cast<typename Tr<PREC>::V8*>(act + act_chunk<H, PREC>(32 * nt + c,
                                                                            u0 / 8 + e)) = v;
       }
@@ -874,7 +899,7 @@ render_kernel(RenderArgs a) {
 #pragma unroll
                 for (int tap = 0; tap < 4; ++tap) {
                   const E* src = map + (size_t)(unsigned)pix[tap] * F + (it % NP) * 8;
-                  raw[r][tap] = *reinterpret_cast<const V8*>(
+                  raw[r][tap] = load_global<V8>(
                       pix[tap] >= 0 ? src : reinterpret_cast<const E*>(kZeroTap));
                 }
               }
@@ -905,8 +930,8 @@ render_kernel(RenderArgs a) {
             for (int tap = 0; tap < 4; ++tap) {
               const float* src = map + (size_t)(unsigned)pix[tap] * F + (it % NP) * 8;
               const f32x4* q = pix[tap] >= 0 ? reinterpret_cast<const f32x4*>(src) : kZeroTap;
-              raw[tap][0] = q[0];
-              raw[tap][1] = q[1];
+              raw[tap][0] = load_global<f32x4>(q);
+              raw[tap][1] = load_global<f32x4>(q + 1);
             }
             float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -952,6 +977,7 @@ render_kernel(RenderArgs a) {
         f32x16 acc[H / 128][NT];
         dense_chain16<H, PREC, NT, K0, F, VP>(W0, act, s_bias, wave, lane, acc);
         const int c = lane & 31, h = lane >> 5;
+        const float inf = opaque_inf();
         float part[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) part[nt] = 0.0f;
@@ -964,7 +990,7 @@ render_kernel(RenderArgs a) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-              for (int i = 0; i < 4; ++i) part[nt] += w4[i] * fmaxf(acc[mt][nt][r + i], 0.0f);
+              for (int i = 0; i < 4; ++i) part[nt] += w4[i] * relu(acc[mt][nt][r + i], inf);
           }
         }
 #pragma unroll
@@ -1010,44 +1036,39 @@ render_kernel(RenderArgs a) {
         }
       }
       if constexpr (POINTS) continue;  // density query: no compositing (S == NS)
-      // ---- front-to-back compositing (volume_rendering.cu:713-734) ---------
-      // the transmittance runs in sample order on values broadcast from their
-      // lanes; a sample counts until the one that took T below the threshold
-      const float keep_al = 1.0f - al;
-      float Ti = 0.0f;
+      // ---- front-to-back compositing (volume_rendering.cu:713-734) and
+      // per-view tokens sum_i w_i f_v(x_i), in sample order on occupancies
+      // broadcast from their lanes; the sample that takes T below the
+      // threshold is the ray's last
+      if (!done) {
+        const float q = wave == 0 ? tv : al;
+        const float* kp = keep + wave * KF + (F == 64 ? lane : lane & (F - 1));
+        constexpr int G = NS % 8 == 0 ? 8 : 4;   // kept features in flight together
+        static_assert(NS % G == 0, "whole groups");
+#pragma unroll 1
+        for (int g0 = 0; g0 < NS && !done; g0 += G) {
+          float f[VPW][G];
 #pragma unroll
-      for (int sl = 0; sl < NS; ++sl) {
-        if (lane == sl) Ti = T;
-        T *= lane_value(keep_al, sl);
-      }
-      const unsigned long long low = __ballot(lane < NS && (c0 > 0 || lane > 0) && Ti < a.t_thres);
-      const int n_live = done ? 0 : (low ? __ffsll((long long)low) - 1 : NS);
-      const float w = lane < n_live ? al * Ti : 0.0f;
-      done = done || low != 0 || __builtin_amdgcn_readfirstlane((int)(T < a.t_thres));
-      // depth, weight and alpha sums in sample order, one per wave
-      if (wave < 3) {
-        const float q = lane < n_live ? (wave == 0 ? tv : (wave == 1 ? 1.0f : al)) : 0.0f;
-        if (a.compensated) {
-          for (int sl = 0; sl < n_live; ++sl)
-            kahan_add(sum, comp, lane_value(w, sl) * lane_value(q, sl));
-        } else {
+          for (int j = 0; j < VPW; ++j)
 #pragma unroll
-          for (int sl = 0; sl < NS; ++sl) {
-            const float qs = lane_value(q, sl);
-            sum = fmaf(lane_value(w, sl), qs, sum);
+            for (int i = 0; i < G; ++i) f[j][i] = kp[((g0 + i) * VP + kWaves * j) * KF];
+#pragma unroll
+          for (int i = 0; i < G; ++i) {
+            const float ai = lane_value(al, g0 + i);
+            const float w = ai * T;
+            if (a.compensated) {
+              kahan_add(sum, comp, wave == 1 ? w : w * lane_value(q, g0 + i));
+#pragma unroll
+              for (int j = 0; j < VPW; ++j) kahan_add(tok[j], tcmp[j], w * f[j][i]);
+            } else {
+              sum = wave == 1 ? sum + w : fmaf(w, lane_value(q, g0 + i), sum);
+#pragma unroll
+              for (int j = 0; j < VPW; ++j) tok[j] += w * f[j][i];
+            }
+            T *= 1.0f - ai;
+            done = T < a.t_thres;
+            if (__builtin_amdgcn_readfirstlane((int)done)) break;
           }
-        }
-      }
-      // ---- per-view tokens: sum_i w_i f_v(x_i) -----------------------------
-#pragma unroll
-      for (int j = 0; j < VPW; ++j) {
-        const float* kp = keep + (wave + kWaves * j) * KF + (F == 64 ? lane : lane & (F - 1));
-        if (a.compensated) {
-          for (int sl = 0; sl < NS; ++sl)
-            kahan_add(tok[j], tcmp[j], lane_value(w, sl) * kp[sl * VP * KF]);
-        } else {
-#pragma unroll
-          for (int sl = 0; sl < NS; ++sl) tok[j] += lane_value(w, sl) * kp[sl * VP * KF];
         }
       }
       if (a.early_exit && done) break;
@@ -2945,8 +2966,9 @@ hydra_rgb_backward_mfma_kernel(const float* __restrict__ tok, const int* __restr
     // the weights are re-read from L1/L2 every step: an opaque copy of the
     // pointer keeps the compiler from hoisting thousands of loop-invariant
     // weight loads into registers
-    const float* wsl = ws;
-    asm volatile("" : "+s"(wsl));
+    const SAILOR_GLOBAL float* wsg = (const SAILOR_GLOBAL float*)ws;
+    asm volatile("" : "+s"(wsg));
+    const float* wsl = (const float*)wsg;
     __syncthreads();
     for (int i = lane; i < 16 * F / 4; i += 64) {
       const int tk = (4 * i) / F, c = (4 * i) % F;
