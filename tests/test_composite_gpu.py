@@ -133,3 +133,40 @@ def test_sigma_gradient_central_differences(occ_mode):
         worst = max(worst, abs(fd - g[i]) / scale)
     print(f"{'occ' if occ_mode else 'density'}: worst |fd - g| / max|g| = {worst:.2e}")
     assert worst <= 1e-4, worst
+
+
+# segment edges (8, 16, 32, 64 lanes), rows in pieces, odd and 16-byte channel
+# counts, more than one channel group in the forward
+@pytest.mark.parametrize("S,F", [(1, 1), (7, 4), (8, 3), (9, 5), (16, 64), (17, 2), (32, 12),
+                                 (33, 33), (64, 16), (65, 20), (130, 7), (200, 64)])
+@pytest.mark.parametrize("occ_mode", [False, True])
+def test_every_segment_shape_matches_float64(S, F, occ_mode):
+    """Forward and gradients at a ray count that leaves the last wave partly
+    empty, features once at an odd 4-byte offset.  A row's sums and products
+    have at most S + 8 roundings of 2^-24 each way; the sigma gradient's
+    suffix is divided by 1 - alpha >= 0.65 (occupancy) and multiplies sums of
+    F products, so S + F + 16 roundings of the largest term bound it."""
+    import sailor_amd.VoxelEncoding as VE
+    R = 37
+    t, s, f, valid = _case(occ_mode, B=1, R=R, S=S, F=F, seed=100 + S)
+    rng = np.random.default_rng(S * 100 + F)
+    grads = [rng.normal(0, 1, (1, R, n)).astype(np.float32) for n in (F, 1, 1, 1)]
+    s64 = torch.from_numpy(s).double().requires_grad_()
+    f64 = torch.from_numpy(f).double().requires_grad_()
+    ref = cr.render(torch.from_numpy(t).double(), s64, f64, occ_mode, torch.from_numpy(valid))
+    rs, rf = torch.autograd.grad(ref, [s64, f64], [torch.from_numpy(g).double() for g in grads])
+    cu = lambda a: torch.from_numpy(a).cuda()
+    shifted = torch.empty(f.size + 1, device="cuda")[1:].view(f.shape)
+    shifted.copy_(cu(f))
+    vr = cu(valid).to(torch.uint8)
+    for feats in (cu(f), shifted):
+        out = VE.volume_render_torch_forward(cu(t), cu(s[..., 0]), feats, vr, occ_mode)
+        for o, r in zip(out, ref):
+            r = r.detach().numpy()
+            assert np.abs(o.cpu().numpy() - r).max() <= (S + 8) * 2.0 ** -24 * max(
+                1.0, np.abs(r).max()) * 2
+        gs, gf = VE.volume_render_torch_backward(*[cu(g) for g in grads], cu(t), cu(s[..., 0]),
+                                                 feats, vr, occ_mode)
+        for o, r in ((gs, rs.numpy()[..., 0]), (gf, rf.numpy())):
+            assert np.abs(o.cpu().numpy() - r).max() <= (S + F + 16) * 2.0 ** -24 * max(
+                1.0, np.abs(r).max()) * 4
