@@ -121,15 +121,60 @@ struct Dda {
   }
 };
 
-// Sink interface: put(pos, node, t0, t1) receives hit number `pos`;
-// stop() is polled after every coarse cell and may end the walk early (used
-// by the fused kernel once all samples are placed; never changes hits that
-// were already emitted).
+// ---- Lane groups -----------------------------------------------------------
+// kGroup lanes walk a ray together: all of them run the same DDA, and a
+// coarse node's children (up to rate^3 records, contiguous in the node array)
+// are tested kGroup at a time, so a test is one coalesced load and one slab
+// test instead of a serial chain of them.  8 lanes: a wave is as long as the
+// longest of 8 rays instead of 64, a launch has 8 times the waves to hide the
+// chain's loads behind, and the DDA that all lanes repeat is still cheap
+// (a wave per ray spends its time there).
+constexpr int kGroup = 8;
+
+struct LaneGroup {
+  int sub, base;   // lane within the group, first lane of the group in its wave
+  __device__ __forceinline__ LaneGroup() {
+    const int lane = threadIdx.x & 63;
+    sub = lane % kGroup;
+    base = lane - sub;
+  }
+  // the group's lanes for which p holds, bit i = lane i
+  __device__ __forceinline__ unsigned vote(bool p) const {
+    return (unsigned)(__ballot(p) >> base) & ((1u << kGroup) - 1);
+  }
+  __device__ __forceinline__ float from(float x, int i) const { return __shfl(x, i, kGroup); }
+  __device__ __forceinline__ int from(int x, int i) const { return __shfl(x, i, kGroup); }
+  __device__ __forceinline__ int before(unsigned votes) const {
+    return __popc(votes & ((1u << sub) - 1));
+  }
+  __device__ __forceinline__ int inclusive_sum(int x) const {
+#pragma unroll
+    for (int o = 1; o < kGroup; o <<= 1) {
+      const int y = __shfl_up(x, o, kGroup);
+      if (sub >= o) x += y;
+    }
+    return x;
+  }
+};
+
+// LDS written by some lanes of a wave and read by others of it: the LDS
+// serves a wave in order, only the compiler has to keep it.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Sink interface (every lane of the group makes the same calls):
+// put(pos, node, t0, t1) receives hit number `pos`; put_lanes(pos, node, t0,
+// t1, hit, votes) the hits of up to kGroup children, one per lane in order,
+// the first of them number `pos`; stop() is polled after every coarse cell
+// and may end the walk early (used once all samples are placed; never changes
+// hits that were already emitted).
 //
 // Returns the number of hits; *vl_out receives the weighted valid length
 // (children weighted by `rate`, the coarse interval by 1).
 template <class Sink>
-__device__ __forceinline__ int traverse(const RayCtx& c, int th_early_stop,
+__device__ __forceinline__ int traverse(const RayCtx& c, const LaneGroup& grp, int th_early_stop,
                                         bool training, int opt_num, Sink& sink,
                                         float* vl_out) {
   float vl = 0.0f;
@@ -166,18 +211,26 @@ __device__ __forceinline__ int traverse(const RayCtx& c, int th_early_stop,
           int r = count;
           if (!training && info.z >= 0) {
             const int ch_end = min(info.z + info.w, c.n_nodes);
-            // the next child's record is loaded while this one is tested
-            float4 qn = info.z < ch_end ? c.np[info.z] : make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int ch = info.z; ch < ch_end; ++ch) {
+            // the next children's records are loaded while these are tested
+            int ch = info.z + grp.sub;
+            float4 qn = ch < ch_end ? c.np[ch] : make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int ch0 = info.z; ch0 < ch_end; ch0 += kGroup, ch += kGroup) {
               const float4 q = qn;
-              if (ch + 1 < ch_end) qn = c.np[ch + 1];
+              if (ch + kGroup < ch_end) qn = c.np[ch + kGroup];
               const float2 cd = slab_test(c.o, c.inv, make_float3(q.x, q.y, q.z), q.w);
-              if (cd.x < 0 || cd.y < 0) continue;
-              sink.put(r, ch, cd.x, cd.y);
+              const bool hit = ch < ch_end && !(cd.x < 0 || cd.y < 0);
+              unsigned votes = grp.vote(hit);
+              if (votes == 0) continue;
+              sink.put_lanes(r, ch, cd.x, cd.y, hit, votes);
+              r += __popc(votes);
               // float += double in the reference (:252): one rounding of the
-              // exact double sum
-              vl = (float)((double)vl + (double)(cd.y - cd.x) * (double)c.rate);
-              ++r;
+              // exact double sum, in hit order
+              const float len = cd.y - cd.x;
+              do {
+                const int i = __ffs(votes) - 1;
+                votes &= votes - 1;
+                vl = (float)((double)vl + (double)grp.from(len, i) * (double)c.rate);
+              } while (votes);
             }
           }
           sink.put(r, node, vd.x, vd.y);
@@ -213,25 +266,24 @@ __device__ __forceinline__ int traverse(const RayCtx& c, int th_early_stop,
   return count;
 }
 
-// Length-weighted per-interval sampling (sampling_kernel.cu:1125-1154).
-struct SampleState {
-  float valid_len;
-  float start_vs;
+// Length-weighted per-interval sampling (sampling_kernel.cu:1125-1174) of one
+// row by a lane group: kGroup hits at a time, one per lane in hit order.
+struct SampleRow {
+  float valid_len, start_vs;
   int S;
-  __device__ __forceinline__ void init(float vl, float svs, int s) {
+  const float* nz;   // the row's noise
+  int* oi;           // the row's outputs
+  float* ot;
+  int has;           // slots used
+  __device__ __forceinline__ void init(float vl, float svs, int s, const float* noise,
+                                       int* out_idx, float* out_t) {
     valid_len = vl;
     start_vs = svs;
     S = s;
-  }
-  // Number of samples interval (mn, mx) of a node of size `cvs` receives
-  // when `has` slots are already used.
-  __device__ __forceinline__ int count_for(float mn, float mx, float cvs, int has) const {
-    const float rate = start_vs / cvs;
-    int n = sat_f2i((mx - mn) * rate * (float)S / valid_len);
-    n = n >= 1 ? n : 1;
-    const int left = S - has;
-    if (left < n) n = left;
-    return n;
+    nz = noise;
+    oi = out_idx;
+    ot = out_t;
+    has = 0;
   }
   // Sample j (0-based) of an interval that receives n samples; r = noise.
   __device__ __forceinline__ static float sample_z(float mn, float mx, int n, int j,
@@ -245,25 +297,32 @@ struct SampleState {
     const float base = mn + off;
     return (float)((double)base - (double)off / 2.0 + (double)(off * r));
   }
-  // Writes the samples of one interval into (oi, ot) from slot `has`.
-  __device__ __forceinline__ int interval(int v, float mn, float mx, float cvs,
-                                          const float* nz, int* oi, float* ot,
-                                          int has) const {
-    const int n = count_for(mn, mx, cvs, has);
-    for (int j = 0; j < n; ++j) {
-      if (has >= S) break;
-      ot[has] = sample_z(mn, mx, n, j, nz[has]);
-      oi[has] = v;
-      ++has;
+  // Places the samples of this lane's interval (mn, mx) of node v, size cvs:
+  // as many as its share of the valid length, at least one, at most what the
+  // intervals before it left.
+  __device__ __forceinline__ void intervals(const LaneGroup& grp, bool on, int v, float mn,
+                                            float mx, float cvs) {
+    int want = 0;
+    if (on) {
+      const float rate = start_vs / cvs;
+      want = sat_f2i((mx - mn) * rate * (float)S / valid_len);
+      want = want >= 1 ? want : 1;
+      want = want < S ? want : S;
     }
-    return has;
+    const int end = grp.inclusive_sum(want);
+    int slot = has + end - want;
+    slot = slot < S ? slot : S;
+    const int n = min(want, S - slot);
+    for (int j = 0; j < n; ++j) {
+      ot[slot + j] = sample_z(mn, mx, n, j, nz[slot + j]);
+      oi[slot + j] = v;
+    }
+    has = min(S, has + grp.from(end, kGroup - 1));
   }
-  __device__ __forceinline__ static int leftover(int v, float mn, float mx,
-                                                 const float* nz, int* oi, float* ot,
-                                                 int has) {
-    ot[has] = leftover_z(mn, mx, nz[has]);
-    oi[has] = v;
-    return has + 1;
+  // One midpoint sample of a hit into `slot`.
+  __device__ __forceinline__ void leftover(int slot, int v, float mn, float mx) {
+    ot[slot] = leftover_z(mn, mx, nz[slot]);
+    oi[slot] = v;
   }
 };
 
