@@ -15,7 +15,7 @@
 // bit-identical to the unfused path.
 // Bound by the latency of the walk (few of 262,144 rays meet the performer):
 // one lane per ray took 551 us for a 512^2 target of a 256^3 grid, 8
-// lanes 487 us.
+// lanes 289 us.
 // Compiled with -ffp-contract=off.
 #include "common.h"
 #include "traversal_common.h"
@@ -26,9 +26,12 @@ using sailor::kGroup;
 using sailor::LaneGroup;
 using sailor::SampleRow;
 
-constexpr int kThreads = 128;
-constexpr int kRays = kThreads / kGroup;   // rays a workgroup walks at a time
-constexpr int kTiles = 4;                  // times kRays consecutive rays per workgroup
+// One wave per workgroup, 8 rays: waves differ widely in how much of the
+// performer they meet, and a workgroup holds its place until its last wave is
+// done (512^2 target: 16 rays x 4 tiles of two waves 487, 16 rays 380, this
+// 300 us).
+constexpr int kThreads = 64;
+constexpr int kRays = kThreads / kGroup;
 
 // Hits of walk 1 kept in LDS (up to kHitCache per ray): rays with at most that
 // many place their samples from there instead of walking the DDA again.  44
@@ -106,8 +109,8 @@ __device__ __forceinline__ void inv3(const float* M, float* out) {
   out[8] = (b2 * a1 - a2 * b1) / det;
 }
 
-// grid = (ceil(H*W / (kRays * kTiles)), B); 8 lanes per target pixel.
-__global__ void __launch_bounds__(kThreads)
+// grid = (ceil(H*W / kRays), B); 8 lanes per target pixel.
+__global__ void __launch_bounds__(kThreads, 6)
 trace_kernel(const float* __restrict__ K, const float* __restrict__ Rm,
              const float* __restrict__ Tv, int H, int W,
              const int* __restrict__ vc, const float4* __restrict__ node_pos,
@@ -120,98 +123,94 @@ trace_kernel(const float* __restrict__ K, const float* __restrict__ Rm,
   __shared__ int s_node[kHitCache * kRays];
   __shared__ float s_t0[kHitCache * kRays], s_t1[kHitCache * kRays];
   const int b = blockIdx.y;
-  if (threadIdx.x == 0) inv3(K + (size_t)b * 9, s_m);
-  if (threadIdx.x == 64) inv3(Rm + (size_t)b * 9, s_m + 9);
+  if (threadIdx.x < 2) inv3((threadIdx.x ? Rm : K) + (size_t)b * 9, s_m + 9 * threadIdx.x);
   __syncthreads();
   const LaneGroup grp;
   const int slot = threadIdx.x / kGroup;
   const int HW = H * W;
-  for (int tile = 0; tile < kTiles; ++tile) {
-    const long long p64 = ((long long)blockIdx.x * kTiles + tile) * kRays + slot;
-    // groups past the image carry no ray but stay for the wave's tail fill
-    const bool live = p64 < HW;
-    const int p = (int)p64;
-    const long long ray = (long long)b * HW + p64;
-    int has = S;   // samples placed; rows past the image have no tail
-    if (live) {
-      // ---- camera ray (rays_calculating_kernel, :443-484)
-      const int h = p / W, w = p - h * W;
-      const float* ki = s_m;
-      const float* ri = s_m + 9;
-      const float* t = Tv + (size_t)b * 3;
-      float o[3], cd[3], wd[3], d[3];
+  const long long p64 = (long long)blockIdx.x * kRays + slot;
+  // groups past the image carry no ray but stay for the wave's tail fill
+  const bool live = p64 < HW;
+  const int p = (int)p64;
+  const long long ray = (long long)b * HW + p64;
+  int has = S;   // samples placed; rows past the image have no tail
+  if (live) {
+    // ---- camera ray (rays_calculating_kernel, :443-484)
+    const int h = p / W, w = p - h * W;
+    const float* ki = s_m;
+    const float* ri = s_m + 9;
+    const float* t = Tv + (size_t)b * 3;
+    float o[3], cd[3], wd[3], d[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        o[k] = -ri[3 * k + 0] * t[0] - ri[3 * k + 1] * t[1] - ri[3 * k + 2] * t[2];
+    for (int k = 0; k < 3; ++k)
+      o[k] = -ri[3 * k + 0] * t[0] - ri[3 * k + 1] * t[1] - ri[3 * k + 2] * t[2];
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        cd[k] = (float)w * ki[3 * k + 0] + (float)h * ki[3 * k + 1] + 1.0f * ki[3 * k + 2];
+    for (int k = 0; k < 3; ++k)
+      cd[k] = (float)w * ki[3 * k + 0] + (float)h * ki[3 * k + 1] + 1.0f * ki[3 * k + 2];
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        wd[k] = cd[0] * ri[3 * k + 0] + cd[1] * ri[3 * k + 1] + cd[2] * ri[3 * k + 2];
-      const float nrm = sqrtf(wd[0] * wd[0] + wd[1] * wd[1] + wd[2] * wd[2]);
-      const double den = (double)nrm + 1e-10;
+    for (int k = 0; k < 3; ++k)
+      wd[k] = cd[0] * ri[3 * k + 0] + cd[1] * ri[3 * k + 1] + cd[2] * ri[3 * k + 2];
+    const float nrm = sqrtf(wd[0] * wd[0] + wd[1] * wd[1] + wd[2] * wd[2]);
+    const double den = (double)nrm + 1e-10;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) d[k] = (float)((double)wd[k] / den);
-      if (rays_out && grp.sub < 6) {
-        const int k = grp.sub;
-        rays_out[ray * 6 + k] = k == 0 ? o[0] : k == 1 ? o[1] : k == 2 ? o[2]
-                                : k == 3 ? d[0] : k == 4 ? d[1] : d[2];
-      }
-      // ---- walk 1: weighted valid length
-      sailor::RayCtx ctx;
-      ctx.init(vc, node_pos, node_info, n_nodes, vol_bbox, voxel_size, b, dim_fine, dim_coarse,
-               rate, o, d);
-      CacheSink cs{s_node + slot, s_t0 + slot, s_t1 + slot, grp};
-      float vl = 0.0f;
-      const int count = sailor::traverse(ctx, grp, -1, false, -1, cs, &vl);
-      sailor::wave_fence();
-      if (vl_out && grp.sub == 0) vl_out[ray] = vl;
-      has = 0;
-      if (count > 0) {
-        SampleRow row;
-        row.init(vl, voxel_size[b] * (float)start_scale, S, noise + ray * S, sidx + ray * S,
-                 st + ray * S);
-        if (count <= kHitCache) {
-          // ---- samples (sampling_kernel.cu:1125-1154) ...
-          for (int k0 = 0; k0 < count && row.has < S; k0 += kGroup) {
-            const int k = k0 + grp.sub;
-            const bool on = k < count;
-            const int nd = on ? cs.node[k * kRays] : 0;
-            const float a0 = on ? cs.t0[k * kRays] : 0.0f, a1 = on ? cs.t1[k * kRays] : 0.0f;
-            row.intervals(grp, on, nd, a0, a1, on ? node_pos[nd].w : 1.0f);
-          }
-          // ---- ... and leftover midpoints (:1156-1174)
-          const int left = min(S - row.has, count);
-          for (int k = grp.sub; k < left; k += kGroup)
-            row.leftover(row.has + k, cs.node[k * kRays], cs.t0[k * kRays], cs.t1[k * kRays]);
-          row.has += left;
-        } else {
-          float dummy;
-          SampleSink ss{row, node_pos, grp};
-          sailor::traverse(ctx, grp, -1, false, -1, ss, &dummy);
-          if (row.has < S) {
-            LeftoverSink ls{row, grp, S - row.has, 0};
-            sailor::traverse(ctx, grp, -1, false, -1, ls, &dummy);
-            row.has += min(S - row.has, count);
-          }
-        }
-        has = row.has;
-      }
-      sailor::wave_fence();   // the next tile's hits go into the same slots
+    for (int k = 0; k < 3; ++k) d[k] = (float)((double)wd[k] / den);
+    if (rays_out && grp.sub < 6) {
+      const int k = grp.sub;
+      rays_out[ray * 6 + k] = k == 0 ? o[0] : k == 1 ? o[1] : k == 2 ? o[2]
+                              : k == 3 ? d[0] : k == 4 ? d[1] : d[2];
     }
-    // ---- the rest of every row is -1, written row by row by the whole wave
-    // (most rays have no sample: their rows are one stretch of memory)
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int k = 0; k < 64 / kGroup; ++k) {
-      const int hk = __builtin_amdgcn_readlane(has, k * kGroup);
-      if (hk >= S) continue;
-      const long long rk = ray - grp.base / kGroup + k;
-      for (int j = hk + lane; j < S; j += 64) {
-        sidx[rk * S + j] = -1;
-        st[rk * S + j] = -1.0f;
+    // ---- walk 1: weighted valid length
+    sailor::RayCtx ctx;
+    ctx.init(vc, node_pos, node_info, n_nodes, vol_bbox, voxel_size, b, dim_fine, dim_coarse,
+             rate, o, d);
+    CacheSink cs{s_node + slot, s_t0 + slot, s_t1 + slot, grp};
+    float vl = 0.0f;
+    const int count = sailor::traverse(ctx, grp, -1, false, -1, cs, &vl);
+    sailor::wave_fence();
+    if (vl_out && grp.sub == 0) vl_out[ray] = vl;
+    has = 0;
+    if (count > 0) {
+      SampleRow row;
+      row.init(vl, voxel_size[b] * (float)start_scale, S, noise + ray * S, sidx + ray * S,
+               st + ray * S);
+      if (count <= kHitCache) {
+        // ---- samples (sampling_kernel.cu:1125-1154) ...
+        for (int k0 = 0; k0 < count && row.has < S; k0 += kGroup) {
+          const int k = k0 + grp.sub;
+          const bool on = k < count;
+          const int nd = on ? cs.node[k * kRays] : 0;
+          const float a0 = on ? cs.t0[k * kRays] : 0.0f, a1 = on ? cs.t1[k * kRays] : 0.0f;
+          row.intervals(grp, on, nd, a0, a1, on ? node_pos[nd].w : 1.0f);
+        }
+        // ---- ... and leftover midpoints (:1156-1174)
+        const int left = min(S - row.has, count);
+        for (int k = grp.sub; k < left; k += kGroup)
+          row.leftover(row.has + k, cs.node[k * kRays], cs.t0[k * kRays], cs.t1[k * kRays]);
+        row.has += left;
+      } else {
+        float dummy;
+        SampleSink ss{row, node_pos, grp};
+        sailor::traverse(ctx, grp, -1, false, -1, ss, &dummy);
+        if (row.has < S) {
+          LeftoverSink ls{row, grp, S - row.has, 0};
+          sailor::traverse(ctx, grp, -1, false, -1, ls, &dummy);
+          row.has += min(S - row.has, count);
+        }
       }
+      has = row.has;
+    }
+  }
+  // ---- the rest of every row is -1, written row by row by the whole wave
+  // (most rays have no sample: their rows are one stretch of memory)
+  const int lane = threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < 64 / kGroup; ++k) {
+    const int hk = __builtin_amdgcn_readlane(has, k * kGroup);
+    if (hk >= S) continue;
+    const long long rk = ray - grp.base / kGroup + k;
+    for (int j = hk + lane; j < S; j += 64) {
+      sidx[rk * S + j] = -1;
+      st[rk * S + j] = -1.0f;
     }
   }
 }
@@ -229,7 +228,7 @@ extern "C" int sailor_trace_sample(const float* K, const float* R, const float* 
   SAILOR_REQUIRE(B > 0 && H > 0 && W > 0 && S > 0, "trace_sample: bad sizes");
   SAILOR_REQUIRE(dim_coarse > 0 && dim_fine % dim_coarse == 0, "trace_sample: bad dims");
   const int rate = dim_fine / dim_coarse;
-  hipLaunchKernelGGL(trace_kernel, dim3(sailor::ceil_div((long long)H * W, kRays * kTiles), B),
+  hipLaunchKernelGGL(trace_kernel, dim3(sailor::ceil_div((long long)H * W, kRays), B),
                      dim3(kThreads), 0, sailor::as_stream(stream), K, R, T, H, W, vol_coarse,
                      reinterpret_cast<const float4*>(node_pos),
                      reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,

@@ -24,20 +24,11 @@ namespace {
 
 constexpr int kThreads = 256;
 
-__global__ void fill_lists(int* __restrict__ idx, float* __restrict__ a, float* __restrict__ b,
-                           long long n) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    idx[i] = -1;
-    a[i] = -1.0f;
-    b[i] = -1.0f;
-  }
-}
-
 using sailor::kGroup;
 using sailor::LaneGroup;
 
-constexpr int kRays = kThreads / kGroup;   // rays of a workgroup, 8 lanes each
+constexpr int kWalkThreads = 64;               // one wave: rays differ widely in length
+constexpr int kRays = kWalkThreads / kGroup;   // rays of a workgroup, 8 lanes each
 constexpr int kEntries = 32;               // entries of a coarse hit kept in LDS per ray
 
 // Receives the coarse hits of the DDA (RayVoxelIntersectionNodeList) and
@@ -174,9 +165,10 @@ struct TreeSink {
   __device__ __forceinline__ bool stop() const { return false; }
 };
 
-// 8 lanes per ray (traversal_common.h): 20,000 random rays through a 128^3 tree
-// filled 79 of 256 CUs with a lane per ray and took 1221 us, now 164 us.
-__global__ void __launch_bounds__(kThreads)
+// 8 lanes per ray (traversal_common.h); each wave then fills what its 8 rows
+// have left with -1.  20,000 random rays through a 128^3 tree filled 79 of 256
+// CUs with a lane per ray and took 1221 us after two fills, now 171 us in all.
+__global__ void __launch_bounds__(kWalkThreads)
 octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos,
                         const int4* __restrict__ node_info, int n_nodes,
                         const float* __restrict__ vol_bbox, const float* __restrict__ voxel_size,
@@ -192,7 +184,7 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
   const LaneGroup grp;
   const int slot = threadIdx.x / kGroup;
   const long long ray = (long long)blockIdx.x * kRays + slot;
-  int n_coarse = 0, n_fine = 0;
+  int n_coarse = 0, n_fine = 0, filled_c = n_max_c, filled = n_max;
   bool overflow = false;
   if (ray < (long long)B * R) {
     const int b = (int)(ray / R);
@@ -209,7 +201,24 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
     if (grp.sub == 0) valid_len[ray] = sink.vl;
     n_fine = sink.cnt;
     overflow = sink.overflow;
+    filled_c = min(n_coarse, n_max_c);
+    filled = min(n_fine, n_max);
   }
+  const long long ray0 = ray - grp.base / kGroup;
+  auto fill = [&](int used, int cap, int* ids, float* a, float* c) {
+#pragma unroll 1
+    for (int k = 0; k < 64 / kGroup; ++k) {
+      const int from = __builtin_amdgcn_readlane(used, k * kGroup);
+      if (from >= cap) continue;
+      const long long row = (ray0 + k) * cap;
+      const int lane = threadIdx.x & 63;
+      sailor::fill_row(reinterpret_cast<unsigned*>(ids + row), from, cap, 0xffffffffu, lane);
+      sailor::fill_row(reinterpret_cast<unsigned*>(a + row), from, cap, 0xbf800000u, lane);
+      sailor::fill_row(reinterpret_cast<unsigned*>(c + row), from, cap, 0xbf800000u, lane);
+    }
+  };
+  fill(filled_c, n_max_c, idx_c, t0_c, t1_c);
+  fill(filled, n_max, idx, t0, t1);
   int mc = n_coarse, mf = n_fine;
   for (int o = 32; o > 0; o >>= 1) {
     mc = max(mc, __shfl_xor(mc, o, 64));
@@ -223,9 +232,11 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
   }
 }
 
-// One thread per ray: ray_voxels_sampling_kernel over the hits in order,
-// then ray_voxels_further_sampling_kernel.
-__global__ void __launch_bounds__(kThreads)
+// ray_voxels_sampling_kernel over the hits in order, then
+// ray_voxels_further_sampling_kernel, by 8 lanes per ray: 8 hits at a time
+// (their slots by a prefix sum), slots written 8 at a time.  A lane per ray,
+// every row access in another line, took 92 us for 20,000 rays, this 20 us.
+__global__ void __launch_bounds__(kWalkThreads)
 adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
                          const float* __restrict__ tmax, const float* __restrict__ noise,
                          const float* __restrict__ valid_len,
@@ -233,8 +244,9 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
                          const float* __restrict__ voxel_size, int B, int R, int n_max,
                          int max_hits, int S, int start_scale, int* __restrict__ sidx,
                          float* __restrict__ st) {
-  const long long ray = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ray >= (long long)B * R) return;
+  const LaneGroup grp;
+  const long long ray = (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
+  if (ray >= (long long)B * R) return;   // whole groups
   const int b = (int)(ray / R);
   const int* hi = hit_idx + ray * n_max;
   const float* mn_ = tmin + ray * n_max;
@@ -242,69 +254,88 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
   const float* rnd = noise + ray * S;
   int* oi = sidx + ray * S;
   float* ot = st + ray * S;
-  for (int j = 0; j < S; ++j) {
-    oi[j] = -1;
-    ot[j] = -1.0f;
-  }
   const float vlen = valid_len[ray];
   const float start_vs = voxel_size[b] * (float)start_scale;
   int cnt = 0;
   // ray_voxels_sampling_kernel visits the first max_hits slots of every ray
   // (num_max_intersected_voxels_fine, :944)
-  for (int i = 0; i < max_hits; ++i) {
-    const int vi = hi[i];
-    if (vi == -1 || vi < 0 || vi >= n_nodes) continue;
-    const float mn = mn_[i], mx = mx_[i];
-    const float rate = start_vs / node_pos[vi].w;
-    int n = sailor::sat_f2i((mx - mn) * rate * (float)S / vlen);
-    n = n >= 1 ? n : 1;
-    const float off = (mx - mn) / (float)(n + 1);
-    for (int j = 0; j < n; ++j) {
-      if (cnt >= S) break;
-      const int rid = cnt++;
-      const float u = rnd[rid];
+  for (int i0 = 0; i0 < max_hits && cnt < S; i0 += kGroup) {
+    const int i = i0 + grp.sub;
+    const int vi = i < max_hits ? hi[i] : -1;
+    const bool on = vi >= 0 && vi < n_nodes;
+    int n = 0;
+    float mn = 0.0f, off = 0.0f;
+    if (on) {
+      mn = mn_[i];
+      const float mx = mx_[i];
+      const float rate = start_vs / node_pos[vi].w;
+      n = sailor::sat_f2i((mx - mn) * rate * (float)S / vlen);
+      n = n >= 1 ? n : 1;
+      off = (mx - mn) / (float)(n + 1);
+    }
+    const int want = n < S ? n : S;
+    const int end = grp.inclusive_sum(want);
+    const int slot = cnt + end - want;
+    for (int j = 0; j < want && slot + j < S; ++j) {
+      const float u = rnd[slot + j];
       const float basic = mn + off * (float)(j + 1);
-      ot[rid] = (float)((double)basic - (double)off / 2.0 + (double)(off * u));
-      oi[rid] = vi;
+      ot[slot + j] = (float)((double)basic - (double)off / 2.0 + (double)(off * u));
+      oi[slot + j] = vi;
     }
+    cnt = min(S, cnt + grp.from(end, kGroup - 1));
   }
+  // the first of the smallest nodes' hits with the smallest midpoint: each
+  // lane's own hits in order, then the lanes'
   float min_mid = 99999.0f, min_vs = 99999.0f, z0 = -1.0f, z1 = -1.0f;
-  int min_idx = -1;
-  for (int i = 0; i < n_max; ++i) {
-    const int vi = hi[i];
-    if (vi == -1) break;
-    if (vi < 0 || vi >= n_nodes) continue;
+  int min_idx = -1, min_at = n_max;
+  bool end = cnt >= S;   // no slot left to fill
+  for (int i0 = 0; i0 < n_max && !end; i0 += kGroup) {
+    const int i = i0 + grp.sub;
+    const int vi = i < n_max ? hi[i] : -1;
+    const unsigned gone = grp.vote(vi == -1);
+    end = gone != 0;
+    if (vi < 0 || vi >= n_nodes || (gone && grp.sub >= __ffs(gone) - 1)) continue;
     const float vs = node_pos[vi].w;
-    if (vs <= min_vs) {
-      const float a = mn_[i], c = mx_[i];
-      const float mid = (float)((double)(a + c) / 2.0);
-      if (vs == min_vs) {
-        if (mid < min_mid) {
-          min_mid = mid;
-          z0 = a;
-          z1 = c;
-          min_idx = vi;
-        }
-      } else {
-        min_mid = mid;
-        z0 = a;
-        z1 = c;
-        min_idx = vi;
-      }
+    if (!(vs <= min_vs)) continue;
+    const float a = mn_[i], c = mx_[i];
+    const float mid = (float)((double)(a + c) / 2.0);
+    if (vs < min_vs || mid < min_mid) {
+      min_mid = mid;
+      z0 = a;
+      z1 = c;
+      min_idx = vi;
+      min_at = i;
+    }
+    min_vs = vs;
+  }
+#pragma unroll
+  for (int o = 1; o < kGroup; o <<= 1) {
+    const float vs = __shfl_xor(min_vs, o, kGroup), mid = __shfl_xor(min_mid, o, kGroup);
+    const float a = __shfl_xor(z0, o, kGroup), c = __shfl_xor(z1, o, kGroup);
+    const int vi = __shfl_xor(min_idx, o, kGroup), at = __shfl_xor(min_at, o, kGroup);
+    const bool take = vi >= 0 && (min_idx < 0 || vs < min_vs ||
+                                  (vs == min_vs && (mid < min_mid ||
+                                                    (mid == min_mid && at < min_at))));
+    if (take) {
       min_vs = vs;
+      min_mid = mid;
+      z0 = a;
+      z1 = c;
+      min_idx = vi;
+      min_at = at;
     }
   }
-  if (min_idx < 0) return;
   const int n_new = S - cnt;
-  if (n_new <= 0) return;
   const float off = (z1 - z0) / (float)(n_new + 1);
-  int j = 0;
-  for (int i = cnt; i < S; ++i) {
-    const float basic = z0 + off * (float)(j + 1);
-    const float u = rnd[i];
-    ot[i] = (float)((double)basic - (double)off / 2.0 + (double)(off * u));
+  for (int i = cnt + grp.sub; i < S; i += kGroup) {
+    float z = -1.0f;
+    if (min_idx >= 0) {
+      const float basic = z0 + off * (float)(i - cnt + 1);
+      const float u = rnd[i];
+      z = (float)((double)basic - (double)off / 2.0 + (double)(off * u));
+    }
+    ot[i] = z;
     oi[i] = min_idx;
-    ++j;
   }
 }
 
@@ -494,14 +525,8 @@ extern "C" int sailor_octree_traversal(
   SAILOR_REQUIRE(dim_coarse > 0 && rate >= 1 && n_nodes >= 0, "octree_traversal: bad tree dims");
   if (R == 0) return SAILOR_OK;
   hipStream_t st = sailor::as_stream(stream);
-  const long long nc = (long long)B * R * n_max_hits_coarse, nf = (long long)B * R * n_max_hits;
-  hipLaunchKernelGGL(fill_lists, dim3(grid_of(nc)), dim3(kThreads), 0, st, hit_idx_coarse,
-                     tmin_coarse, tmax_coarse, nc);
-  hipLaunchKernelGGL(fill_lists, dim3(grid_of(nf)), dim3(kThreads), 0, st, hit_idx, tmin, tmax,
-                     nf);
-  if (int e = sailor::check_launch("octree_traversal (fill)")) return e;
   hipLaunchKernelGGL(octree_traversal_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kThreads), 0, st, vol_coarse,
+                     dim3(kWalkThreads), 0, st, vol_coarse,
                      reinterpret_cast<const float4*>(node_pos),
                      reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size, B,
                      dim_fine, dim_coarse, rate, ray_ori, ray_dir, R, n_max_hits_coarse,
@@ -521,8 +546,8 @@ extern "C" int sailor_octree_sampling(const int32_t* hit_idx, const float* tmin,
   SAILOR_REQUIRE(max_hits >= 0 && max_hits <= n_max_hits,
                  "ray_voxels_points_sampling: max_hits %d outside [0, %d]", max_hits, n_max_hits);
   if (R == 0) return SAILOR_OK;
-  hipLaunchKernelGGL(adaptive_sampling_kernel, dim3(sailor::ceil_div((long long)B * R, kThreads)),
-                     dim3(kThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax, noise,
+  hipLaunchKernelGGL(adaptive_sampling_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
+                     dim3(kWalkThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax, noise,
                      valid_len, reinterpret_cast<const float4*>(node_pos), n_nodes, voxel_size,
                      B, R, n_max_hits, max_hits, S, start_scale, sampled_idx, sampled_t);
   return sailor::check_launch("ray_voxels_points_sampling");

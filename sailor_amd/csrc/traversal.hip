@@ -26,7 +26,8 @@ using sailor::kGroup;
 using sailor::LaneGroup;
 using sailor::SampleRow;
 
-constexpr int kRays = kThreads / kGroup;   // rays of a workgroup, 8 lanes each
+constexpr int kWalkThreads = 64;               // one wave: rays differ widely in length
+constexpr int kRays = kWalkThreads / kGroup;   // rays of a workgroup, 8 lanes each
 
 struct ListSink {
   int* idx;
@@ -54,23 +55,11 @@ struct ListSink {
   __device__ __forceinline__ bool stop() const { return false; }
 };
 
-// Words [from, n) of a row set to v by the whole wave, 16 bytes a lane where
-// the row allows it.
-__device__ __forceinline__ void fill_row(unsigned* row, int from, int n, unsigned v, int lane) {
-  const int head = min(n, from + (int)(((16 - ((uintptr_t)(row + from) & 15)) & 15) / 4));
-  if (from + lane < head) row[from + lane] = v;
-  const int quads = (n - head) / 4;
-  for (int q = lane; q < quads; q += 64)
-    reinterpret_cast<uint4*>(row + head)[q] = make_uint4(v, v, v, v);
-  const int tail = head + 4 * quads;
-  if (tail + lane < n) row[tail + lane] = v;
-}
-
 // 8 lanes per ray (traversal_common.h); each wave then fills what its 8 rows
 // have left with -1.  The rows are what bounds the call (n_max 1024: 12 KB a
 // ray), so they are written once: a fill of all rows before a lane-per-ray
-// walk took 225 + 256 us for 102,400 rays, this kernel 282 us (4.5 TB/s).
-__global__ void __launch_bounds__(kThreads)
+// walk took 225 + 256 us for 102,400 rays, this kernel 239 us (5.3 TB/s).
+__global__ void __launch_bounds__(kWalkThreads)
 traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos,
                  const int4* __restrict__ node_info, int n_nodes,
                  const float* __restrict__ vol_bbox,
@@ -105,9 +94,9 @@ traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos
     const int from = __builtin_amdgcn_readlane(filled, k * kGroup);
     if (from >= n_max) continue;
     const long long row = (ray0 + k) * n_max;
-    fill_row(reinterpret_cast<unsigned*>(hit_idx + row), from, n_max, 0xffffffffu, lane);
-    fill_row(reinterpret_cast<unsigned*>(tmin + row), from, n_max, 0xbf800000u, lane);
-    fill_row(reinterpret_cast<unsigned*>(tmax + row), from, n_max, 0xbf800000u, lane);
+    sailor::fill_row(reinterpret_cast<unsigned*>(hit_idx + row), from, n_max, 0xffffffffu, lane);
+    sailor::fill_row(reinterpret_cast<unsigned*>(tmin + row), from, n_max, 0xbf800000u, lane);
+    sailor::fill_row(reinterpret_cast<unsigned*>(tmax + row), from, n_max, 0xbf800000u, lane);
   }
   // global max hit count (reference: atomicMax per step, :405) and overflow
   int m = count;
@@ -120,7 +109,7 @@ traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos
 }
 
 // 8 lanes per ray, 8 hits at a time; the row's unused slots are -1.
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kWalkThreads)
 sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
                 const float* __restrict__ tmax, const float* __restrict__ noise,
                 const float* __restrict__ valid_len,
@@ -244,7 +233,7 @@ extern "C" int sailor_octree_voxel_traversal(
   hipStream_t st = sailor::as_stream(stream);
   if (R == 0) return SAILOR_OK;
   hipLaunchKernelGGL(traversal_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kThreads), 0, st, vol_coarse,
+                     dim3(kWalkThreads), 0, st, vol_coarse,
                      reinterpret_cast<const float4*>(node_pos),
                      reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox,
                      voxel_size, B,
@@ -262,7 +251,7 @@ extern "C" int sailor_octree_sampling_coarse(
   SAILOR_REQUIRE(B > 0 && R >= 0 && S > 0 && n_max_hits > 0, "sampling: bad sizes");
   if (R == 0) return SAILOR_OK;
   hipLaunchKernelGGL(sampling_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax,
+                     dim3(kWalkThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax,
                      noise, valid_len, reinterpret_cast<const float4*>(node_pos),
                      voxel_size, B, R, n_max_hits, S, start_scale, sampled_idx,
                      sampled_t);

@@ -130,6 +130,7 @@ struct Dda {
 // chain's loads behind, and the DDA that all lanes repeat is still cheap
 // (a wave per ray spends its time there).
 constexpr int kGroup = 8;
+constexpr int kChildBatch = 2;   // children per lane loaded together (4: the same)
 
 struct LaneGroup {
   int sub, base;   // lane within the group, first lane of the group in its wave
@@ -162,6 +163,18 @@ struct LaneGroup {
 __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
+}
+
+// Words [from, n) of a row set to v by the whole wave, 16 bytes a lane where
+// the row allows it.
+__device__ __forceinline__ void fill_row(unsigned* row, int from, int n, unsigned v, int lane) {
+  const int head = min(n, from + (int)(((16 - ((uintptr_t)(row + from) & 15)) & 15) / 4));
+  if (from + lane < head) row[from + lane] = v;
+  const int quads = (n - head) / 4;
+  for (int q = lane; q < quads; q += 64)
+    reinterpret_cast<uint4*>(row + head)[q] = make_uint4(v, v, v, v);
+  const int tail = head + 4 * quads;
+  if (tail + lane < n) row[tail + lane] = v;
 }
 
 // Sink interface (every lane of the group makes the same calls):
@@ -211,26 +224,34 @@ __device__ __forceinline__ int traverse(const RayCtx& c, const LaneGroup& grp, i
           int r = count;
           if (!training && info.z >= 0) {
             const int ch_end = min(info.z + info.w, c.n_nodes);
-            // the next children's records are loaded while these are tested
-            int ch = info.z + grp.sub;
-            float4 qn = ch < ch_end ? c.np[ch] : make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int ch0 = info.z; ch0 < ch_end; ch0 += kGroup, ch += kGroup) {
-              const float4 q = qn;
-              if (ch + kGroup < ch_end) qn = c.np[ch + kGroup];
-              const float2 cd = slab_test(c.o, c.inv, make_float3(q.x, q.y, q.z), q.w);
-              const bool hit = ch < ch_end && !(cd.x < 0 || cd.y < 0);
-              unsigned votes = grp.vote(hit);
-              if (votes == 0) continue;
-              sink.put_lanes(r, ch, cd.x, cd.y, hit, votes);
-              r += __popc(votes);
-              // float += double in the reference (:252): one rounding of the
-              // exact double sum, in hit order
-              const float len = cd.y - cd.x;
-              do {
-                const int i = __ffs(votes) - 1;
-                votes &= votes - 1;
-                vl = (float)((double)vl + (double)grp.from(len, i) * (double)c.rate);
-              } while (votes);
+            // the records of up to kChildBatch children per lane are loaded
+            // together: a round of loads tests 16 children
+            for (int ch0 = info.z; ch0 < ch_end; ch0 += kGroup * kChildBatch) {
+              float4 q[kChildBatch];
+#pragma unroll
+              for (int u = 0; u < kChildBatch; ++u) {
+                const int ch = ch0 + u * kGroup + grp.sub;
+                q[u] = c.np[ch < ch_end ? ch : ch_end - 1];
+              }
+#pragma unroll
+              for (int u = 0; u < kChildBatch; ++u) {
+                const int ch = ch0 + u * kGroup + grp.sub;
+                const float2 cd =
+                    slab_test(c.o, c.inv, make_float3(q[u].x, q[u].y, q[u].z), q[u].w);
+                const bool hit = ch < ch_end && !(cd.x < 0 || cd.y < 0);
+                unsigned votes = grp.vote(hit);
+                if (votes == 0) continue;
+                sink.put_lanes(r, ch, cd.x, cd.y, hit, votes);
+                r += __popc(votes);
+                // float += double in the reference (:252): one rounding of the
+                // exact double sum, in hit order
+                const float len = cd.y - cd.x;
+                do {
+                  const int i = __ffs(votes) - 1;
+                  votes &= votes - 1;
+                  vl = (float)((double)vl + (double)grp.from(len, i) * (double)c.rate);
+                } while (votes);
+              }
             }
           }
           sink.put(r, node, vd.x, vd.y);
@@ -313,9 +334,19 @@ struct SampleRow {
     int slot = has + end - want;
     slot = slot < S ? slot : S;
     const int n = min(want, S - slot);
-    for (int j = 0; j < n; ++j) {
-      ot[slot + j] = sample_z(mn, mx, n, j, nz[slot + j]);
-      oi[slot + j] = v;
+    // the noise of several samples is loaded before the first is stored (the
+    // compiler cannot tell that the stores leave it alone)
+    constexpr int kAhead = 4;
+    for (int j0 = 0; j0 < n; j0 += kAhead) {
+      float r[kAhead];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) r[j] = nz[slot + min(j0 + j, n - 1)];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+        if (j0 + j < n) {
+          ot[slot + j0 + j] = sample_z(mn, mx, n, j0 + j, r[j]);
+          oi[slot + j0 + j] = v;
+        }
     }
     has = min(S, has + grp.from(end, kGroup - 1));
   }
