@@ -196,7 +196,7 @@ __device__ __forceinline__ constexpr int acc_unit(int mt, int r, int h) {
 
 struct DensityMfmaLds {
   f16x8 frag[kMfmaFrags];
-  float bias[kMfmaLayers][64];
+  alignas(16) float bias[kMfmaLayers][64];
   float w_out[64];
   float b_out;
 };
@@ -223,12 +223,22 @@ __device__ __forceinline__ void mfma_layer(const DensityMfmaLds& L, int layer,
                                                        acc[mt], 0, 0, 0);
 }
 
-// B operands of the next layer: relu(acc), rounded to half
+// B operands of the next layer: acc rounded to half, then the ReLU on packed
+// pairs (rounding keeps the sign; a NaN gives 0 as fmaxf does)
+__device__ __forceinline__ f16x8 relu8(f16x8 x) {
+  f16x8 zero;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) zero[j] = (half_t)0.0f;
+  return __builtin_elementwise_max(x, zero);
+}
 __device__ __forceinline__ void relu_to_b(const f32x16 (&acc)[2], f16x8 (&b)[4]) {
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
+  for (int s = 0; s < 4; ++s) {
+    f16x8 v;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) b[s][j] = (half_t)fmaxf(acc[s / 2][8 * (s % 2) + j], 0.0f);
+    for (int j = 0; j < 8; ++j) v[j] = (half_t)acc[s / 2][8 * (s % 2) + j];
+    b[s] = relu8(v);
+  }
 }
 
 // one M-tile (the geometry layers: <= 32 outputs)
@@ -245,8 +255,55 @@ __device__ __forceinline__ void mfma_layer1(const DensityMfmaLds& L, int layer,
     acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[s * 64 + lane], bin[s], acc, 0, 0, 0);
 }
 
+// x + (the value of another lane of the aligned group of 2, 4 or 8), without
+// the LDS: quad permutations, and the mirrored half row once the quads of 8
+// lanes hold one value each.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  return x + __int_as_float(
+                 __builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+}
 template <int VS>
-__global__ void __launch_bounds__(kBlock)
+__device__ __forceinline__ float view_sum(float x) {
+  if constexpr (VS > 1) x = dpp_add<0xB1>(x);    // lanes 1, 0, 3, 2
+  if constexpr (VS > 2) x = dpp_add<0x4E>(x);    // lanes 2, 3, 0, 1
+  if constexpr (VS > 4) x = dpp_add<0x141>(x);   // lanes 7 .. 0 of 8
+  return x;
+}
+
+// acc = bias + W x with the layer's A fragments in registers
+template <int STEPS>
+__device__ __forceinline__ void mfma_layer_r(const f16x8 (&w)[2][STEPS], const float* bias,
+                                             const f16x8* bin, f32x16 (&acc)[2], int lane,
+                                             int zo) {
+  const float4* b4 = reinterpret_cast<const float4*>(bias) + 2 * (lane >> 5) + zo;
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {   // units 32 mt + 16 (q/2) + 8 h + 4 (q%2) ..
+      const float4 t = b4[8 * mt + 4 * (q / 2) + q % 2];
+      acc[mt][4 * q] = t.x; acc[mt][4 * q + 1] = t.y;
+      acc[mt][4 * q + 2] = t.z; acc[mt][4 * q + 3] = t.w;
+    }
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+      acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[mt][s], bin[s], acc[mt], 0, 0, 0);
+}
+
+// Per wave and step 32 consecutive points as VS tiles of P = 32 / VS points:
+// each tile's columns are its (point, view) pairs through the feature layers;
+// after the view mean the VS lanes of a point hold the same values, so lane v
+// of each point keeps them for tile v, and the occupancy layers run once for
+// all 32 points.  The feature layers' fragments (112 registers) stay in
+// registers at two waves per SIMD, the others in LDS.
+// Bound by vector issue: per tile 28 + 3 + 16 / VS MFMAs and about as many
+// vector instruction cycles for bias, ReLU and rounding (65,536 rays x 48
+// samples x 4 views: 1264 us with the occupancy layers run per tile, view sums
+// through LDS shuffles and two v_max per ReLU; 722 us now).
+template <int VS>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
 density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__ z,
                     const float* __restrict__ tpsdf, const float* __restrict__ geo, int B,
                     long long n_pts, int V, float* __restrict__ occ,
@@ -275,114 +332,132 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
 
   constexpr int P = 32 / VS;
   const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
-  const int v = n % VS;
-  const long long total = (long long)B * n_pts;
-  const long long tiles = (total + P - 1) / P;
+  const int v = n % VS, lp = n / VS;
+  const long long steps = (n_pts + 31) / 32;
   const long long wave0 = (long long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   const long long n_waves = (long long)gridDim.x * (kBlock / 64);
   const float inv = 1.0f / (float)V;
-  // this lane's share of a column's inputs x = [z, tpsdf, geo 0..15]:
-  // half 0 holds x 0..7 and x 16..17, half 1 holds x 8..15 (its layer-0 B
-  // operand); the next tile's share is loaded before the current tile's
-  // MFMA chain runs (one wave per SIMD: nothing else hides the latency)
-  auto load_share = [&](long long tile, float (&x)[10]) {
+  f16x8 w0[2][2], wf[3][2][4];
 #pragma unroll
-    for (int i = 0; i < 10; ++i) x[i] = 0.0f;
-    const long long p = tile * P + n / VS;
-    if (tile < tiles && p < total && v < V) {
-      const long long b = p / n_pts, q = p - b * n_pts;
-      const long long e = (b * V + v) * n_pts + q;
-      const float* g = geo + e * 16;
-      if (h == 0) {
-        x[0] = z[e];
-        x[1] = tpsdf[e];
+  for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
-        for (int i = 0; i < 6; ++i) x[2 + i] = g[i];
-        x[8] = g[14];
-        x[9] = g[15];
-      } else {
+    for (int s = 0; s < 2; ++s) w0[mt][s] = L.frag[(mt * 2 + s) * 64 + lane];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = g[6 + i];
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        wf[l][mt][s] = L.frag[mfma_frag_base(l + 1) + (mt * 4 + s) * 64 + lane];
+  }
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));   // kept from the compiler, which would make the median a maximum again
+  for (int b = blockIdx.y; b < B; b += gridDim.y) {
+    // this lane's share of a column's inputs x = [z, tpsdf, geo 0..15]: half 0
+    // holds x 0..7 and x 16..17, half 1 holds x 8..15 (its layer-0 B
+    // operand); the next tile's share is loaded before the current tile's
+    // MFMA chain runs
+    const long long col0 = ((long long)b * V + (v < V ? v : 0)) * n_pts;
+    auto load_share = [&](long long tile, float (&x)[10]) {
+#pragma unroll
+      for (int i = 0; i < 10; ++i) x[i] = 0.0f;
+      const long long p = tile * P + lp;
+      if (p < n_pts && v < V) {
+        const float* g = geo + (col0 + p) * 16;
+        const float4 a = *reinterpret_cast<const float4*>(g + (h ? 8 : 0));
+        const float2 c = *reinterpret_cast<const float2*>(g + (h ? 6 : 4));
+        const float2 d = *reinterpret_cast<const float2*>(g + (h ? 12 : 14));
+        float2 f = c;
+        if (h == 0) f = make_float2(z[col0 + p], tpsdf[col0 + p]);
+        x[0] = f.x; x[1] = f.y;
+        x[2] = a.x; x[3] = a.y; x[4] = a.z; x[5] = a.w;
+        x[6] = h ? d.x : c.x;
+        x[7] = h ? d.y : c.y;
+        x[8] = h ? 0.0f : d.x;
+        x[9] = h ? 0.0f : d.y;
       }
-    }
-  };
-  float xc[10];
-  load_share(wave0, xc);
-  for (long long tile = wave0; tile < tiles; tile += n_waves) {
-    float xn[10];
-    load_share(tile + n_waves, xn);
-    const long long p = tile * P + n / VS;
-    const bool col_ok = p < total && v < V;
-    const long long b = p / n_pts, q = p - b * n_pts;
-    f16x8 bin[4];
+    };
+    float xc[10];
+    load_share(wave0 * VS, xc);
+    for (long long it = wave0; it < steps; it += n_waves) {
+      f16x8 comb[4] = {};
+      int zo;
+#pragma unroll 1
+      for (int k = 0; k < VS; ++k) {
+        const long long tile = it * VS + k;
+        float xn[10];
+        load_share(k + 1 < VS ? tile + 1 : (it + n_waves) * VS, xn);
+        const long long p = tile * P + lp;
+        const bool col_ok = p < n_pts && v < V;
+        f16x8 bin[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      bin[0][j] = (half_t)xc[j];
-      bin[1][j] = (half_t)(h == 0 && j < 2 ? xc[8 + j] : 0.0f);
-      bin[2][j] = (half_t)0.0f;
-      bin[3][j] = (half_t)0.0f;
-    }
-    int zo;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(zo));
-    f16x8 bin0[4];
+        for (int j = 0; j < 8; ++j) {
+          bin[0][j] = (half_t)xc[j];
+          bin[1][j] = (half_t)(j < 2 ? xc[8 + j] : 0.0f);
+        }
+        // an opaque zero redefined every tile keeps the bias reads in the
+        // loop, so the registers go to the weight fragments
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zo));
+        f32x16 acc[2];
+        // geometry features of the texture views: 18 -> 16 -> 8 on MFMA from
+        // the layer-0 operand; hidden unit 8 h + r sits in accumulator r < 8
+        // of half h, which is the next layer's B operand, and output r < 8
+        // lands in accumulator r of half 0.  The whole wave runs the MFMAs (an
+        // MFMA reads the A and B registers of every lane, so a lane-dependent
+        // branch around it would feed it stale rows); only the store is per
+        // lane.
+        if (geo_out) {
+          f32x16 g;
+          f16x8 gb[4];
+          mfma_layer1<2>(L, 6, bin, g, lane, 4 * zo);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) bin0[t] = bin[t];
-    f32x16 acc[2];
-    mfma_layer<2>(L, 0, bin, acc, lane, zo);
+          for (int j = 0; j < 8; ++j) gb[0][j] = (half_t)g[j];
+          gb[0] = relu8(gb[0]);
+          mfma_layer1<1>(L, 7, gb, g, lane, 4 * zo);
+          if (h == 0 && col_ok && v < n_geo_out) {
+            float4* o4 = reinterpret_cast<float4*>(
+                geo_out + (((long long)b * n_geo_out + v) * n_pts + p) * 8);
+            o4[0] = make_float4(fmaxf(g[0], 0.f), fmaxf(g[1], 0.f), fmaxf(g[2], 0.f),
+                                fmaxf(g[3], 0.f));
+            o4[1] = make_float4(fmaxf(g[4], 0.f), fmaxf(g[5], 0.f), fmaxf(g[6], 0.f),
+                                fmaxf(g[7], 0.f));
+          }
+        }
+        mfma_layer_r<2>(w0, L.bias[0], bin, acc, lane, zo);
 #pragma unroll
-    for (int layer = 1; layer < 4; ++layer) {
-      relu_to_b(acc, bin);
-      mfma_layer<4>(L, layer, bin, acc, lane, zo);
-    }
-    // mean of the ReLU outputs over the point's views (fp32)
-    const float cm = col_ok ? 1.0f : 0.0f;
+        for (int l = 0; l < 3; ++l) {
+          relu_to_b(acc, bin);
+          mfma_layer_r<4>(wf[l], L.bias[l + 1], bin, acc, lane, zo);
+        }
+        // mean of the ReLU outputs over the point's views (fp32): the median
+        // of x, 0 and the bound is the ReLU, and 0 in a column without a view
+        const float bound = col_ok ? inf : 0.0f;
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+        for (int s = 0; s < 4; ++s) {
+          f16x8 m;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float t = fmaxf(acc[mt][r], 0.0f) * cm;
+          for (int j = 0; j < 8; ++j)
+            m[j] = (half_t)(view_sum<VS>(__builtin_amdgcn_fmed3f(acc[s / 2][8 * (s % 2) + j],
+                                                                 0.0f, bound)) * inv);
+          comb[s] = VS == 1 || v == k ? m : comb[s];
+        }
 #pragma unroll
-        for (int off = 1; off < VS; off <<= 1) t += __shfl_xor(t, off, 64);
-        acc[mt][r] = t * inv;
+        for (int i = 0; i < 10; ++i) xc[i] = xn[i];
       }
+      // occupancy layers: column n is point lp of tile v
+      f32x16 acc[2];
+      mfma_layer<4>(L, 4, comb, acc, lane, 4 * zo);
+      relu_to_b(acc, comb);
+      mfma_layer<4>(L, 5, comb, acc, lane, 4 * zo);
+      float part = 0.0f;
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+      for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) bin[s][j] = (half_t)acc[s / 2][8 * (s % 2) + j];
-    mfma_layer<4>(L, 4, bin, acc, lane, zo);
-    relu_to_b(acc, bin);
-    mfma_layer<4>(L, 5, bin, acc, lane, zo);
-    float part = 0.0f;
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) part += L.w_out[acc_unit(mt, r, h)] * fmaxf(acc[mt][r], 0.0f);
-    part += __shfl_xor(part, 32, 64);
-    if (h == 0 && v == 0 && p < total) occ[p] = 1.0f / (1.0f + expf(-(part + L.b_out)));
-    // geometry features of the texture views: 18 -> 16 -> 8 on MFMA from the
-    // layer-0 operand; hidden unit 8 h + r sits in accumulator r < 8 of half
-    // h, which is the next layer's B operand, and output r < 8 lands in
-    // accumulator r of half 0.  The whole wave runs the MFMAs (an MFMA reads
-    // the A and B registers of every lane, so a lane-dependent branch around
-    // it would feed it stale rows); only the store is per lane.
-    if (geo_out) {
-      f32x16 g;
-      mfma_layer1<2>(L, 6, bin0, g, lane, zo);
-      f16x8 gb[4];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) gb[0][j] = (half_t)fmaxf(g[j], 0.0f);
-      mfma_layer1<1>(L, 7, gb, g, lane, zo);
-      if (h == 0 && col_ok && v < n_geo_out) {
-        float4* o4 =
-            reinterpret_cast<float4*>(geo_out + ((b * n_geo_out + v) * n_pts + q) * 8);
-        o4[0] = make_float4(fmaxf(g[0], 0.f), fmaxf(g[1], 0.f), fmaxf(g[2], 0.f),
-                            fmaxf(g[3], 0.f));
-        o4[1] = make_float4(fmaxf(g[4], 0.f), fmaxf(g[5], 0.f), fmaxf(g[6], 0.f),
-                            fmaxf(g[7], 0.f));
-      }
+        for (int r = 0; r < 16; ++r)
+          part += L.w_out[acc_unit(mt, r, h)] * __builtin_amdgcn_fmed3f(acc[mt][r], 0.0f, inf);
+      part += __shfl_xor(part, 32, 64);
+      const long long p = (it * VS + v) * P + lp;
+      if (h == 0 && p < n_pts)
+        occ[(long long)b * n_pts + p] = 1.0f / (1.0f + expf(-(part + L.b_out)));
     }
-#pragma unroll
-    for (int i = 0; i < 10; ++i) xc[i] = xn[i];
   }
 }
 
@@ -506,9 +581,9 @@ color_kernel(const half_t* __restrict__ params, const float* __restrict__ t,
 }
 
 // ---- Colour path of the fp16 form ------------------------------------------
-// color_composite_kernel: one lane per (ray, texture slot) composites the 30
-// features exactly as color_kernel does and writes the token, padded to 32
-// with zeros, to the workspace (slot 0's lane also writes the depth).
+// color_composite_kernel: composites the 30 features of a (ray, texture slot)
+// exactly as color_kernel does and writes the token, padded to 32 with zeros,
+// to the workspace (and slot 0's depth).
 // color_mfma_kernel: Hydra stacks + RGB head with every product on
 // v_mfma_f32_16x16x32_f16.  Each wave takes 16 tokens (4 rays x 4 slots): the
 // MFMA's N = 16 columns are the tokens, M = 16 output units per tile, K = 32
@@ -525,62 +600,76 @@ constexpr int kCxLd = kTokW + 4;           // fp32 token rows in LDS
 constexpr int kChLd = 64 + 4;              // fp32 rows of attention / hidden units
 constexpr int kStackRows = 6 * 32;         // q | k | v | fc | w1 | w2 rows, 32 each
 
+// 8 lanes own a (ray, texture slot): lanes 0-3 the colour features, 4 and 5 the
+// geometry features (16 bytes of a sample each), 6 the colour, 7 the direction,
+// each summing its channels in sample order.  kAhead samples are loaded at a
+// time and walked until the one that takes T below the threshold.  A lane per
+// (ray, slot) with 30 channels read each sample's rows from 64 places at once:
+// 502 us for 65,536 rays x 48 samples x 4 views, now 180 us.
 __global__ void __launch_bounds__(kBlock)
 color_composite_kernel(const float* __restrict__ t, const float* __restrict__ occ,
                        const float* __restrict__ feats_rgb, const float* __restrict__ rgbs,
                        const float* __restrict__ geo8, const float* __restrict__ dirs, int B,
                        int R, int S, int Vt, float t_thres, float* __restrict__ out_depth,
                        float* __restrict__ tok) {
-  const long long lanes = (long long)B * R * kTexSlots;
-  for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < lanes;
-       id += (long long)gridDim.x * blockDim.x) {
+  constexpr int kAhead = 8;
+  const long long items = (long long)B * R * kTexSlots;
+  const int sub = threadIdx.x & 7;
+  for (long long id = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / 8; id < items;
+       id += (long long)gridDim.x * blockDim.x / 8) {
     const long long ray = id / kTexSlots;
     const int v = (int)(id % kTexSlots);
-    float x[kTokW];
-#pragma unroll
-    for (int c = 0; c < kTokW; ++c) x[c] = 0.0f;
+    float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     float depth = 0.0f;
-    if (v < Vt) {
+    const float* tr = t + ray * S;
+    const float* oc = occ + ray * S;
+    if (v < Vt && !(tr[S - 1] < 0.0f)) {
       const long long b = ray / R, r = ray - b * R;
-      const float* tr = t + ray * S;
-      const float* oc = occ + ray * S;
-      if (!(tr[S - 1] < 0.0f)) {
-        const long long e0 = ((b * Vt + v) * R + r) * S;
-        float T = 1.0f;
-        for (int s = 0; s < S; ++s) {
-          const float ts = tr[s];
-          if (ts < 0.0f) continue;
-          const float a = oc[s];
-          const float wgt = a * T;
-          const long long e = e0 + s;
-          const float4* f4 = reinterpret_cast<const float4*>(feats_rgb + e * 16);
+      const long long e0 = ((b * Vt + v) * R + r) * S;
+      // this lane's channels: a row pitch and 3 or 4 floats per sample
+      const float* src = sub < 4    ? feats_rgb + e0 * 16 + 4 * sub
+                         : sub < 6  ? geo8 + e0 * 8 + 4 * (sub - 4)
+                         : sub == 6 ? rgbs + e0 * 3
+                                    : dirs + e0 * 3;
+      const int pitch = sub < 4 ? 16 : sub < 6 ? 8 : 3;
+      float T = 1.0f;
+      bool done = false;
+      for (int s0 = 0; s0 < S && !done; s0 += kAhead) {
+        const int sm = min(s0 + sub, S - 1);
+        const float tl = tr[sm], al = oc[sm];
+        float f[kAhead][4];
 #pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const float4 f = f4[c];
-            x[4 * c + 0] += wgt * f.x;
-            x[4 * c + 1] += wgt * f.y;
-            x[4 * c + 2] += wgt * f.z;
-            x[4 * c + 3] += wgt * f.w;
+        for (int i = 0; i < kAhead; ++i) {
+          const float* q = src + (long long)min(s0 + i, S - 1) * pitch;
+          if (sub < 6) {
+            const float4 q4 = *reinterpret_cast<const float4*>(q);
+            f[i][0] = q4.x; f[i][1] = q4.y; f[i][2] = q4.z; f[i][3] = q4.w;
+          } else {
+            f[i][0] = q[0]; f[i][1] = q[1]; f[i][2] = q[2]; f[i][3] = 0.0f;
           }
+        }
 #pragma unroll
-          for (int c = 0; c < 3; ++c) x[16 + c] += wgt * rgbs[e * 3 + c];
-          const float4* g4 = reinterpret_cast<const float4*>(geo8 + e * 8);
-          const float4 ga = g4[0], gb = g4[1];
-          x[19] += wgt * ga.x; x[20] += wgt * ga.y; x[21] += wgt * ga.z; x[22] += wgt * ga.w;
-          x[23] += wgt * gb.x; x[24] += wgt * gb.y; x[25] += wgt * gb.z; x[26] += wgt * gb.w;
+        for (int i = 0; i < kAhead; ++i) {
+          const float ts = __shfl(tl, i, 8), a = __shfl(al, i, 8);
+          if (done || s0 + i >= S || ts < 0.0f) continue;
+          const float wgt = a * T;
 #pragma unroll
-          for (int c = 0; c < 3; ++c) x[27 + c] += wgt * dirs[e * 3 + c];
+          for (int c = 0; c < 4; ++c) x[c] += wgt * f[i][c];
           depth += wgt * ts;
           T *= 1.0f - a;
-          if (T < t_thres) break;
+          done = T < t_thres;
         }
       }
     }
-    float4* o4 = reinterpret_cast<float4*>(tok + id * kTokW);
-#pragma unroll
-    for (int c = 0; c < kTokW / 4; ++c)
-      o4[c] = make_float4(x[4 * c], x[4 * c + 1], x[4 * c + 2], x[4 * c + 3]);
-    if (v == 0) out_depth[ray] = depth;
+    // token [rgb feats 16 | rgb 3 | geometry features 8 | direction 3 | 0 0]
+    float* o = tok + id * kTokW + (sub < 4 ? 4 * sub : sub < 6 ? 19 + 4 * (sub - 4)
+                                                    : sub == 6 ? 16 : 27);
+    o[0] = x[0];
+    o[1] = x[1];
+    o[2] = x[2];
+    if (sub != 6) o[3] = sub < 6 ? x[3] : 0.0f;
+    if (sub == 7) o[4] = 0.0f;
+    if (v == 0 && sub == 0) out_depth[ray] = depth;
   }
 }
 
@@ -1285,17 +1374,19 @@ int launch_density(bool mfma, const half_t* pd, const float* z, const float* tps
                    int n_geo_out, hipStream_t st) {
   if (mfma && V <= 8) {
     const int VS = V <= 1 ? 1 : V <= 2 ? 2 : V <= 4 ? 4 : 8;
-    const long long tiles = ((long long)B * n_pts + 32 / VS - 1) / (32 / VS);
-    // persistent workgroups, 3 per CU (50 KB of LDS and ~150 registers per
-    // lane each): the weights are staged once per workgroup
+    const long long steps = (n_pts + 31) / 32;
+    // persistent workgroups, 2 per CU (256 registers per lane, 50 KB of LDS):
+    // the weights are staged once per workgroup
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    const unsigned grid = (unsigned)std::max<long long>(
-        1, std::min<long long>((tiles + kBlock / 64 - 1) / (kBlock / 64), 3LL * cus));
+    const long long slots = std::max<long long>(1, 2LL * cus / std::min(B, 2 * cus));
+    const dim3 grid((unsigned)std::max<long long>(
+                        1, std::min<long long>((steps + kBlock / 64 - 1) / (kBlock / 64), slots)),
+                    (unsigned)std::min(B, 65535));
 #define SAILOR_DENSITY_MFMA(N)                                                            \
-  hipLaunchKernelGGL(density_mfma_kernel<N>, dim3(grid), dim3(kBlock), 0, st, pd, z, tpsdf, \
+  hipLaunchKernelGGL(density_mfma_kernel<N>, grid, dim3(kBlock), 0, st, pd, z, tpsdf, \
                      geo, B, n_pts, V, occ, geo_out, n_geo_out)
     if (VS == 1) SAILOR_DENSITY_MFMA(1);
     else if (VS == 2) SAILOR_DENSITY_MFMA(2);
@@ -1339,7 +1430,7 @@ int infer_nerf_impl(bool mfma, const float* sorted_dists, const float* points_z,
     float* tok = reinterpret_cast<float*>(
         reinterpret_cast<char*>(geo8) +
         ((size_t)B * n_pts * tex_views * 8 * sizeof(float) + 255) / 256 * 256);
-    hipLaunchKernelGGL(color_composite_kernel, dim3(grid_for((long long)B * R * kTexSlots)),
+    hipLaunchKernelGGL(color_composite_kernel, dim3(grid_for((long long)B * R * kTexSlots * 8)),
                        dim3(kBlock), 0, st, sorted_dists, occ, feats_rgb, rgbs, geo8, dirs, B, R,
                        S, tex_views, 1e-4f, out_depth, tok);
     if (int err = sailor::check_launch("infer_nerf (compositing)")) return err;
