@@ -77,6 +77,22 @@ int sailor_integrate_compensated(int32_t* occ_vol, int32_t* num_occ, const float
                                  float* color, float* vol_origin, float* vol_bbox,
                                  float* voxel_size, void* stream);
 
+/* sailor_integrate (compensated == 0) or sailor_integrate_compensated with
+ * room for tables with which bricks of voxels skip the views that cannot
+ * observe them: the same outputs, bit for bit, faster.  workspace:
+ * sailor_integrate_workspace_bytes bytes, 8-byte aligned, no clearing needed;
+ * calls that share it must not overlap.  `masks` (read by no kernel) is left out. */
+size_t sailor_integrate_workspace_bytes(int B, int V, int H, int W, int X, int Y, int Z);
+int sailor_integrate_workspace(int compensated, int32_t* occ_vol, int32_t* num_occ,
+                               const float* K, const float* RT, const float* R, const float* T,
+                               const float* colors, const float* depths, int B, int V, int H,
+                               int W, int X, int Y, int Z, float obs_weight, float th_bbox,
+                               float trunc_weight, float tsdf_th_low, float tsdf_th_high,
+                               const float* fixed_bbox, float* tsdf, float* weight,
+                               float* color, float* vol_origin, float* vol_bbox,
+                               float* voxel_size, void* workspace, size_t workspace_bytes,
+                               void* stream);
+
 /* Replaces get_origin_bbox (fusion_kernel.cu:473-534).
  *  depths f32 [B,V,H,W], K/R f32 [B,V,3,3], T f32 [B,V,3] -> vol_origin [B,3,2] */
 int sailor_get_origin_bbox(const float* depths, const float* K, const float* R,

@@ -75,12 +75,15 @@ def integrate(occupied_vol, num_occ_voxel, cam_intr, cam_pose, cam_R, cam_T, col
     vol_bbox = torch.empty((B, 3, 2), **opts)
     voxel_size = torch.empty((B, 1), **opts)
     with torch.cuda.device(dev):
-        call("sailor_integrate_compensated" if compensated else "sailor_integrate",
+        wsb = _lib.lib().sailor_integrate_workspace_bytes(B, V, H, W, X, Y, Z)
+        ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
+        call("sailor_integrate_workspace", int(bool(compensated)),
              ptr(occupied_vol), ptr(num_occ_voxel), ptr(K), ptr(RT),
-             ptr(R), ptr(T), ptr(colors), ptr(depths), ptr(masks), B, V, H, W, X, Y, Z,
+             ptr(R), ptr(T), ptr(colors), ptr(depths), B, V, H, W, X, Y, Z,
              float(obs_weight), float(th_bbox), float(trunc_weight), float(tsdf_th_low),
              float(tsdf_th_high), ptr(fb), ptr(tsdf), ptr(weight), ptr(color),
-             ptr(vol_origin), ptr(vol_bbox), ptr(voxel_size), stream_of(dev))
+             ptr(vol_origin), ptr(vol_bbox), ptr(voxel_size), ptr(ws), ws.numel(),
+             stream_of(dev))
     return tsdf, weight, color, vol_origin, vol_bbox, voxel_size
 
 

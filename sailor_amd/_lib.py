@@ -25,6 +25,8 @@ _SIGS = {
     "sailor_abi_version": [],
     "sailor_integrate": [P] * 9 + [I] * 7 + [F] * 5 + [P] * 8,
     "sailor_integrate_compensated": [P] * 9 + [I] * 7 + [F] * 5 + [P] * 8,
+    "sailor_integrate_workspace_bytes": [I] * 7,
+    "sailor_integrate_workspace": [I] + [P] * 8 + [I] * 7 + [F] * 5 + [P] * 8 + [SZ, P],
     "sailor_get_origin_bbox": [P] * 4 + [I] * 4 + [F, P, P],
     "sailor_get_center_xyz": [P, P, P, P, I, I, I, I, P, P, P, SZ, P],
     "sailor_build_multi_res_volumes": [P, P, I, I, I, I, P],
@@ -90,6 +92,7 @@ _SIGS = {
 }
 _RESTYPES = {
     "sailor_last_error": ctypes.c_char_p,
+    "sailor_integrate_workspace_bytes": SZ,
     "sailor_octree_workspace_bytes": SZ,
     "sailor_render_small_weights_floats": SZ,
     "sailor_render_workspace_bytes": SZ,

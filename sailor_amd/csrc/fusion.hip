@@ -10,10 +10,12 @@
 //  * bbox: one pass over the depth maps; each workgroup reduces its pixels in
 //    registers / LDS and issues 6 integer atomics (order-preserving float keys)
 //    instead of one CAS loop per pixel and bound.
-//  * integrate: one lane per voxel, z fastest, so the 16 B/voxel of output
-//    (tsdf, weight, colour, occupancy) is written with fully coalesced stores;
-//    the per-view camera rows are wave-uniform scalar loads; the occupied
-//    count is aggregated with a wave ballot and one atomic per workgroup.
+//  * integrate: one lane per voxel, a wave per 4 x 4 x 16 brick, z fastest, so
+//    the 16 B/voxel of output (tsdf, weight, colour, occupancy) is written in
+//    64-byte runs; views that cannot observe a brick are skipped, by its
+//    projection and a table of the views' deepest usable depth per 16^2 pixel
+//    tile; the occupied count is aggregated with wave ballots and one atomic
+//    per workgroup.
 #include "common.h"
 
 namespace {
@@ -173,12 +175,161 @@ __global__ void keys_to_float(float* buf, int n) {
   buf[i] = sailor::fkey_inv(reinterpret_cast<const int*>(buf)[i]);
 }
 
-// One lane per voxel; grid = (ceil(X*Y*Z / 256), B).  COMP (precision form):
-// the TSDF is formed as the Kahan-compensated sum of obs_weight * dist over
-// the observing views divided once by the weight sum, instead of the
-// reference's running average (tsdf * w_old + obs_weight * dist) / w_new --
-// the same value in exact arithmetic, with one rounding of the sum instead
-// of one per view.
+// Largest depth of every kTile x kTile pixel tile that an integration may use
+// (0.1 m <= d <= 4 m; a NaN, which passes those tests, as infinity), -1 where
+// the tile has none.  grid = (ceil(tiles_x / 4), tiles_y, B * V): 4 tiles of a
+// tile row per workgroup.
+constexpr int kTile = 16;
+
+__global__ void __launch_bounds__(kThreads)
+depth_tiles_kernel(const float* __restrict__ depths, int H, int W, int tiles_x, int tiles_y,
+                   float* __restrict__ tiles) {
+  __shared__ float s_max[kThreads / 64][4];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const float* img = depths + (size_t)blockIdx.z * H * W;
+  const int x = blockIdx.x * 64 + lane;
+  float m = -1.0f;
+  for (int r = wid; r < kTile; r += kThreads / 64) {
+    const int y = blockIdx.y * kTile + r;
+    if (x < W && y < H) {
+      const float d = img[(size_t)y * W + x];
+      if (!(d < 0.1f || d > 4.0f)) m = fmaxf(m, d != d ? __builtin_inff() : d);
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < kTile; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if (lane % kTile == 0) s_max[wid][lane / kTile] = m;
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    for (int w = 0; w < kThreads / 64; ++w) m = w ? fmaxf(m, s_max[w][threadIdx.x])
+                                                  : s_max[0][threadIdx.x];
+    const int tx = blockIdx.x * 4 + threadIdx.x;
+    if (tx < tiles_x) tiles[((size_t)blockIdx.z * tiles_y + blockIdx.y) * tiles_x + tx] = m;
+  }
+}
+
+// Bricks of kBx x kBy x kBz voxels, z fastest: a wave integrates one, 64 voxels
+// per pass.
+constexpr int kBx = 4, kBy = 4, kBz = 16;
+constexpr int kPassY = 64 / kBz;
+static_assert(64 % kBz == 0 && kBy % kPassY == 0, "whole passes over the brick");
+
+struct Bricks {
+  unsigned ny, nz, n;
+  __host__ __device__ Bricks(int X, int Y, int Z)
+      : ny((Y + kBy - 1) / kBy), nz((Z + kBz - 1) / kBz),
+        n((unsigned)((X + kBx - 1) / kBx) * ny * nz) {}
+  __device__ void corner(unsigned brick, int& x, int& y, int& z) const {
+    x = (int)(brick / (ny * nz)) * kBx;
+    y = (int)(brick / nz % ny) * kBy;
+    z = (int)(brick % nz) * kBz;
+  }
+};
+
+// masks[b * bricks + i], bit k: view k may observe a voxel of brick i of volume
+// b; every other view leaves all of the brick's voxels unchanged.  VP lanes (V
+// rounded up to a power of two) per brick, a view each; grid = (.., B).  A lane
+// projects the 8 corners of the brick's voxel centres: where all are in front
+// of the camera, the brick's pixels lie within the corners' bounding box, taken
+// 2 pixels wider than they can round, and an observation needs a depth of at
+// least cz - trunc there (tiles).  Bounds that are not finite, and bricks that
+// reach the camera plane, count as observed.
+__global__ void __launch_bounds__(kThreads)
+observing_views_kernel(const float* __restrict__ vol_bbox, const float* __restrict__ voxel_size,
+                       const float* __restrict__ K, const float* __restrict__ RT,
+                       const float* __restrict__ tiles, int tiles_x, int tiles_y, int V, int VP,
+                       int H, int W, int X, int Y, int Z, float trunc_weight,
+                       unsigned long long* __restrict__ masks) {
+  const Bricks br(X, Y, Z);
+  const int b = blockIdx.y, per = kThreads / VP;
+  const int k = threadIdx.x & (VP - 1);
+  const float vs = voxel_size[b], trunc = vs * trunc_weight;
+  const float* bb = vol_bbox + b * 6;
+  // whole groups of VP lanes stay together: the vote below is theirs
+  for (unsigned brick = blockIdx.x * per + threadIdx.x / VP; brick < br.n;
+       brick += gridDim.x * per) {
+    bool seen = false;
+    if (k < V) {
+      int x0, y0, z0;
+      br.corner(brick, x0, y0, z0);
+      const float lo[3] = {bb[0] + (float)x0 * vs, bb[2] + (float)y0 * vs,
+                           bb[4] + (float)z0 * vs};
+      const float hi[3] = {bb[0] + (float)(min(x0 + kBx, X) - 1) * vs,
+                           bb[2] + (float)(min(y0 + kBy, Y) - 1) * vs,
+                           bb[4] + (float)(min(z0 + kBz, Z) - 1) * vs};
+      const float* rt = RT + ((size_t)b * V + k) * 12;
+      const float* kk = K + ((size_t)b * V + k) * 9;
+      const float inf = __builtin_inff();
+      float u0 = inf, u1 = -inf, v0 = inf, v1 = -inf, c0 = inf, c1 = -inf, p0 = inf;
+      float ec = 0.0f, eu = 0.0f, ev = 0.0f;
+      bool finite = true;
+#pragma unroll
+      for (int corner = 0; corner < 8; ++corner) {
+        const float x = corner & 1 ? hi[0] : lo[0], y = corner & 2 ? hi[1] : lo[1],
+                    z = corner & 4 ? hi[2] : lo[2];
+        const float cx = rt[0] * x + rt[1] * y + rt[2] * z + rt[3];
+        const float cy = rt[4] * x + rt[5] * y + rt[6] * z + rt[7];
+        const float cz = rt[8] * x + rt[9] * y + rt[10] * z + rt[11];
+        const float pz = kk[6] * cx + kk[7] * cy + kk[8] * cz;
+        const float u = (kk[0] * cx + kk[1] * cy + kk[2] * cz) / pz;
+        const float v = (kk[3] * cx + kk[4] * cy + kk[5] * cz) / pz;
+        // 1e-6 of the sums of magnitudes bounds the rounding of 7 operations
+        const float ax = fabsf(rt[0] * x) + fabsf(rt[1] * y) + fabsf(rt[2] * z) + fabsf(rt[3]);
+        const float ay = fabsf(rt[4] * x) + fabsf(rt[5] * y) + fabsf(rt[6] * z) + fabsf(rt[7]);
+        const float az = fabsf(rt[8] * x) + fabsf(rt[9] * y) + fabsf(rt[10] * z) + fabsf(rt[11]);
+        const float ap = fabsf(kk[6]) * ax + fabsf(kk[7]) * ay + fabsf(kk[8]) * az;
+        const float au = fabsf(kk[0]) * ax + fabsf(kk[1]) * ay + fabsf(kk[2]) * az;
+        const float av = fabsf(kk[3]) * ax + fabsf(kk[4]) * ay + fabsf(kk[5]) * az;
+        u0 = fminf(u0, u);
+        u1 = fmaxf(u1, u);
+        v0 = fminf(v0, v);
+        v1 = fmaxf(v1, v);
+        c0 = fminf(c0, cz);
+        c1 = fmaxf(c1, cz);
+        p0 = fminf(p0, pz - 1e-6f * ap);
+        ec = fmaxf(ec, 1e-6f * az);
+        eu = fmaxf(eu, 1e-6f * (au + fabsf(u) * ap));
+        ev = fmaxf(ev, 1e-6f * (av + fabsf(v) * ap));
+        finite = finite && fabsf(u) < 1e8f && fabsf(v) < 1e8f && au + av + ap + az < 1e12f;
+      }
+      if (!finite || !(p0 > 0.05f)) {
+        seen = !(finite && c1 < -1e-3f - ec);   // cz < 0 throughout: never observed
+      } else {
+        const float ex = 2.0f + eu / p0, ey = 2.0f + ev / p0;
+        u0 -= ex; u1 += ex; v0 -= ey; v1 += ey;
+        if (u1 >= 0.0f && v1 >= 0.0f && u0 <= (float)W && v0 <= (float)H) {
+          const int tx0 = (int)fmaxf(u0, 0.0f) / kTile, ty0 = (int)fmaxf(v0, 0.0f) / kTile;
+          const int tx1 = min((int)fminf(u1, (float)W) / kTile, tiles_x - 1);
+          const int ty1 = min((int)fminf(v1, (float)H) / kTile, tiles_y - 1);
+          const float need = c0 - trunc - 1e-3f - ec;
+          const float* tv = tiles + ((size_t)b * V + k) * tiles_x * tiles_y;
+          seen = (tx1 - tx0 + 1) * (ty1 - ty0 + 1) > 512;   // wide: as observed
+          for (int ty = ty0; ty <= ty1 && !seen; ++ty) {
+            float m = -1.0f;
+            for (int tx = tx0; tx <= tx1; ++tx) m = fmaxf(m, tv[(size_t)ty * tiles_x + tx]);
+            seen = m >= 0.0f && !(m < need);
+          }
+        }
+      }
+    }
+    unsigned long long m = __ballot(seen) >> ((threadIdx.x & 63) & ~(VP - 1));
+    if (VP < 64) m &= (1ull << VP) - 1;
+    if (k == 0) masks[(size_t)b * br.n + brick] = m;
+  }
+}
+
+// One lane per voxel, a brick per wave; grid = (ceil(bricks / 4), B).  masks:
+// the views to evaluate for each brick (null: all of them).  Bound by vector
+// issue where views remain (the reference's IEEE divisions, 7 per view and
+// voxel) and by the 16 B written per voxel elsewhere: 256^3 voxels, 4 views of
+// 1024^2 around one performer 290 us without the masks, 93 us with them and
+// about 20 us to make them (0.27 GB written; bricks of 4 x 4 x 32 and 8^3
+// voxels -8 and +27 us, but at 128^3 the former costs 15 us more); masks made
+// by one wave of each 512-voxel workgroup before its voxels: 156 us.  COMP (precision form): the TSDF is
+// formed as the Kahan-compensated sum of obs_weight * dist over the observing
+// views divided once by the weight sum, instead of the reference's running
+// average (tsdf * w_old + obs_weight * dist) / w_new -- the same value in exact
+// arithmetic, with one rounding of the sum instead of one per view.
 template <bool COMP>
 __global__ void __launch_bounds__(kThreads)
 integrate_kernel(float* __restrict__ tsdf_vol, float* __restrict__ weight_vol,
@@ -187,87 +338,99 @@ integrate_kernel(float* __restrict__ tsdf_vol, float* __restrict__ weight_vol,
                  const float* __restrict__ K, const float* __restrict__ RT,
                  const float* __restrict__ colors,
                  const float* __restrict__ depths,
-                 const float* __restrict__ voxel_size, float obs_weight, int H,
+                 const float* __restrict__ voxel_size,
+                 const unsigned long long* __restrict__ masks, float obs_weight, int H,
                  int W, int V, int X, int Y, int Z, float trunc_weight,
                  float th_low, float th_high) {
   __shared__ int s_cnt[kThreads / 64];
+  const Bricks br(X, Y, Z);
   const int b = blockIdx.y;
-  const int YZ = Y * Z;
-  const int nvox = X * YZ;
-  const int vid = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool active = vid < nvox;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float vs = voxel_size[b];
   const float trunc = vs * trunc_weight;
-  bool occupied = false;
-  if (active) {
-    int vx = vid / YZ;
-    int vy = (vid - vx * YZ) / Z;
-    int vz = vid - vx * YZ - vy * Z;
-    const float* bb = vol_bbox + b * 6;
-    float pt_x = bb[0] + (float)vx * vs;
-    float pt_y = bb[2] + (float)vy * vs;
-    float pt_z = bb[4] + (float)vz * vs;
-    float tsdf = 1.0f, w = 0.0f, col = 0.0f;
-    float ksum = 0.0f, kcomp = 0.0f;  // COMP: sum of obs_weight * dist, lost low bits
-    const size_t img = (size_t)H * W;
-    for (int k = 0; k < V; ++k) {
-      const float* rt = RT + ((size_t)b * V + k) * 12;
-      const float* kk = K + ((size_t)b * V + k) * 9;
-      float cx = rt[0] * pt_x + rt[1] * pt_y + rt[2] * pt_z + rt[3];
-      float cy = rt[4] * pt_x + rt[5] * pt_y + rt[6] * pt_z + rt[7];
-      float cz = rt[8] * pt_x + rt[9] * pt_y + rt[10] * pt_z + rt[11];
-      float px = kk[0] * cx + kk[1] * cy + kk[2] * cz;
-      float py = kk[3] * cx + kk[4] * cy + kk[5] * cz;
-      float pz = kk[6] * cx + kk[7] * cy + kk[8] * cz;
-      px = px / pz;
-      py = py / pz;
-      int ix = sailor::sat_f2i(roundf(px));
-      int iy = sailor::sat_f2i(roundf(py));
-      if (ix < 0 || ix >= W || iy < 0 || iy >= H || cz < 0) continue;
-      size_t pix = ((size_t)b * V + k) * img + (size_t)iy * W + ix;
-      float d = depths[pix];
-      if (d < 0.1f || d > 4.0f) continue;
-      float diff = d - cz;
-      if (diff < -trunc) continue;
-      float dist = fminf(1.0f, diff / trunc);
-      float w_old = w;
-      float w_new = w_old + obs_weight;
-      w = w_new;
-      if constexpr (COMP) {
-        const float y = obs_weight * dist - kcomp;
-        const float t = ksum + y;
-        kcomp = (t - ksum) - y;
-        ksum = t;
-      } else {
-        tsdf = (tsdf * w_old + obs_weight * dist) / w_new;
+  const float* bb = vol_bbox + b * 6;
+  int count = 0;
+  for (unsigned brick = blockIdx.x * (kThreads / 64) + wid; brick < br.n;
+       brick += gridDim.x * (kThreads / 64)) {
+    int x0, y0, z0;
+    br.corner(brick, x0, y0, z0);
+    unsigned long long views = V < 64 ? (1ull << V) - 1 : ~0ull;
+    if (masks) views = masks[(size_t)b * br.n + brick];
+    const int vz = z0 + lane % kBz;
+#pragma unroll 1
+    for (int pass = 0; pass < kBx * kBy / kPassY; ++pass) {
+      const int vx = x0 + pass / (kBy / kPassY);
+      const int vy = y0 + pass % (kBy / kPassY) * kPassY + lane / kBz;
+      bool occupied = false;
+      if (vx < X && vy < Y && vz < Z) {
+        const int vid = (vx * Y + vy) * Z + vz;
+        float pt_x = bb[0] + (float)vx * vs;
+        float pt_y = bb[2] + (float)vy * vs;
+        float pt_z = bb[4] + (float)vz * vs;
+        float tsdf = 1.0f, w = 0.0f, col = 0.0f;
+        float ksum = 0.0f, kcomp = 0.0f;  // COMP: sum of obs_weight * dist, lost low bits
+        const size_t img = (size_t)H * W;
+        for (unsigned long long left = views; left; left &= left - 1) {
+          const int k = __ffsll((long long)left) - 1;
+          const float* rt = RT + ((size_t)b * V + k) * 12;
+          const float* kk = K + ((size_t)b * V + k) * 9;
+          float cx = rt[0] * pt_x + rt[1] * pt_y + rt[2] * pt_z + rt[3];
+          float cy = rt[4] * pt_x + rt[5] * pt_y + rt[6] * pt_z + rt[7];
+          float cz = rt[8] * pt_x + rt[9] * pt_y + rt[10] * pt_z + rt[11];
+          float px = kk[0] * cx + kk[1] * cy + kk[2] * cz;
+          float py = kk[3] * cx + kk[4] * cy + kk[5] * cz;
+          float pz = kk[6] * cx + kk[7] * cy + kk[8] * cz;
+          px = px / pz;
+          py = py / pz;
+          int ix = sailor::sat_f2i(roundf(px));
+          int iy = sailor::sat_f2i(roundf(py));
+          if (ix < 0 || ix >= W || iy < 0 || iy >= H || cz < 0) continue;
+          size_t pix = ((size_t)b * V + k) * img + (size_t)iy * W + ix;
+          float d = depths[pix];
+          if (d < 0.1f || d > 4.0f) continue;
+          float diff = d - cz;
+          if (diff < -trunc) continue;
+          float dist = fminf(1.0f, diff / trunc);
+          float w_old = w;
+          float w_new = w_old + obs_weight;
+          w = w_new;
+          if constexpr (COMP) {
+            const float y = obs_weight * dist - kcomp;
+            const float t = ksum + y;
+            kcomp = (t - ksum) - y;
+            ksum = t;
+          } else {
+            tsdf = (tsdf * w_old + obs_weight * dist) / w_new;
+          }
+          // packed colour running average (fusion_kernel.cu:320-331)
+          float old_b = floorf(col / 65536.0f);
+          float old_g = floorf((col - old_b * 256.0f * 256.0f) / 256.0f);
+          float old_r = col - old_b * 256.0f * 256.0f - old_g * 256.0f;
+          float nc = colors[pix];
+          float new_b = floorf(nc / 65536.0f);
+          float new_g = floorf((nc - new_b * 256.0f * 256.0f) / 256.0f);
+          float new_r = nc - new_b * 256.0f * 256.0f - new_g * 256.0f;
+          new_b = fminf(roundf((old_b * w_old + obs_weight * new_b) / w_new), 255.0f);
+          new_g = fminf(roundf((old_g * w_old + obs_weight * new_g) / w_new), 255.0f);
+          new_r = fminf(roundf((old_r * w_old + obs_weight * new_r) / w_new), 255.0f);
+          col = new_b * 256.0f * 256.0f + new_g * 256.0f + new_r;
+        }
+        if constexpr (COMP) {
+          if (w > 0.0f) tsdf = (ksum - kcomp) / w;
+        }
+        occupied = tsdf < trunc * th_high && tsdf > -trunc * th_low;
+        size_t o = (size_t)b * X * Y * Z + vid;
+        tsdf_vol[o] = tsdf;
+        weight_vol[o] = w;
+        color_vol[o] = col;
+        occ_vol[o] = occupied ? vid : -1;
       }
-      // packed colour running average (fusion_kernel.cu:320-331)
-      float old_b = floorf(col / 65536.0f);
-      float old_g = floorf((col - old_b * 256.0f * 256.0f) / 256.0f);
-      float old_r = col - old_b * 256.0f * 256.0f - old_g * 256.0f;
-      float nc = colors[pix];
-      float new_b = floorf(nc / 65536.0f);
-      float new_g = floorf((nc - new_b * 256.0f * 256.0f) / 256.0f);
-      float new_r = nc - new_b * 256.0f * 256.0f - new_g * 256.0f;
-      new_b = fminf(roundf((old_b * w_old + obs_weight * new_b) / w_new), 255.0f);
-      new_g = fminf(roundf((old_g * w_old + obs_weight * new_g) / w_new), 255.0f);
-      new_r = fminf(roundf((old_r * w_old + obs_weight * new_r) / w_new), 255.0f);
-      col = new_b * 256.0f * 256.0f + new_g * 256.0f + new_r;
+      count += __popcll(__ballot(occupied));
     }
-    if constexpr (COMP) {
-      if (w > 0.0f) tsdf = (ksum - kcomp) / w;
-    }
-    occupied = tsdf < trunc * th_high && tsdf > -trunc * th_low;
-    size_t o = (size_t)b * nvox + vid;
-    tsdf_vol[o] = tsdf;
-    weight_vol[o] = w;
-    color_vol[o] = col;
-    occ_vol[o] = occupied ? vid : -1;
   }
-  // occupied count: ballot per wave, one atomic per workgroup
-  unsigned long long m = __ballot(occupied);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) s_cnt[wid] = __popcll(m);
+  // occupied count: ballots per wave, one atomic per workgroup
+  if (lane == 0) s_cnt[wid] = count;
   __syncthreads();
   if (threadIdx.x == 0) {
     int c = 0;
@@ -368,6 +531,14 @@ int launch_bbox(const float* depths, const float* K, const float* R,
 
 }  // namespace
 
+// Workspace: a mask of views per brick, then the depth of each pixel tile.
+extern "C" size_t sailor_integrate_workspace_bytes(int B, int V, int H, int W, int X, int Y,
+                                                   int Z) {
+  if (B <= 0 || V <= 0 || H <= 0 || W <= 0 || X <= 0 || Y <= 0 || Z <= 0) return 0;
+  return (size_t)B * Bricks(X, Y, Z).n * sizeof(unsigned long long) +
+         (size_t)B * V * ((H + kTile - 1) / kTile) * ((W + kTile - 1) / kTile) * sizeof(float);
+}
+
 namespace {
 
 int integrate_impl(bool comp, int32_t* occ_vol, int32_t* num_occ, const float* K,
@@ -376,7 +547,7 @@ int integrate_impl(bool comp, int32_t* occ_vol, int32_t* num_occ, const float* K
                    float obs_weight, float th_bbox, float trunc_weight, float tsdf_th_low,
                    float tsdf_th_high, const float* fixed_bbox, float* tsdf, float* weight,
                    float* color, float* vol_origin, float* vol_bbox, float* voxel_size,
-                   void* stream) {
+                   void* workspace, size_t workspace_bytes, void* stream) {
   SAILOR_REQUIRE(B > 0 && V > 0 && H > 0 && W > 0, "integrate: empty input");
   SAILOR_REQUIRE(V <= kMaxViews, "integrate: at most %d views", kMaxViews);
   SAILOR_REQUIRE(X > 1 && Y > 0 && Z > 0, "integrate: bad volume dims");
@@ -389,13 +560,38 @@ int integrate_impl(bool comp, int32_t* occ_vol, int32_t* num_occ, const float* K
   }
   hipLaunchKernelGGL(bbox_finalize, dim3(sailor::ceil_div(B, 64)), dim3(64), 0,
                      st, vol_bbox, B, X, fixed_bbox, vol_origin, voxel_size);
-  const int nvox = X * Y * Z;
-  hipLaunchKernelGGL(comp ? integrate_kernel<true> : integrate_kernel<false>,
-                     dim3(sailor::ceil_div(nvox, kThreads), B),
-                     dim3(kThreads), 0, st, tsdf, weight, color, occ_vol,
-                     num_occ, vol_bbox, K, RT, colors, depths, voxel_size,
-                     obs_weight, H, W, V, X, Y, Z, trunc_weight, tsdf_th_low,
-                     tsdf_th_high);
+  const unsigned n = Bricks(X, Y, Z).n;
+  const int tiles_x = sailor::ceil_div(W, kTile), tiles_y = sailor::ceil_div(H, kTile);
+  // a launch holds fewer than 2^32 lanes: larger grids loop
+  auto blocks = [](long long want) { return dim3((unsigned)std::min(want, 1LL << 23)); };
+  unsigned long long* masks = nullptr;
+  if (workspace != nullptr) {
+    SAILOR_REQUIRE(workspace_bytes >= sailor_integrate_workspace_bytes(B, V, H, W, X, Y, Z),
+                   "integrate: workspace of %zu bytes is smaller than the %zu required",
+                   workspace_bytes, sailor_integrate_workspace_bytes(B, V, H, W, X, Y, Z));
+    SAILOR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 7) == 0,
+                   "integrate: workspace must be 8-byte aligned");
+    // the tiles' launch takes a grid plane per view and a row per tile row
+    if ((long long)B * V <= 65535 && tiles_y <= 65535) {
+      masks = static_cast<unsigned long long*>(workspace);
+      float* tiles = reinterpret_cast<float*>(masks + (size_t)B * n);
+      hipLaunchKernelGGL(depth_tiles_kernel, dim3(sailor::ceil_div(tiles_x, 4), tiles_y, B * V),
+                         dim3(kThreads), 0, st, depths, H, W, tiles_x, tiles_y, tiles);
+      int VP = 1;
+      while (VP < V) VP *= 2;
+      dim3 grid = blocks(((long long)n * VP + kThreads - 1) / kThreads);
+      grid.y = B;
+      hipLaunchKernelGGL(observing_views_kernel, grid, dim3(kThreads), 0, st, vol_bbox,
+                         voxel_size, K, RT, tiles, tiles_x, tiles_y, V, VP, H, W, X, Y, Z,
+                         trunc_weight, masks);
+    }
+  }
+  dim3 grid = blocks(((long long)n + kThreads / 64 - 1) / (kThreads / 64));
+  grid.y = B;
+  hipLaunchKernelGGL(comp ? integrate_kernel<true> : integrate_kernel<false>, grid,
+                     dim3(kThreads), 0, st, tsdf, weight, color, occ_vol, num_occ, vol_bbox, K,
+                     RT, colors, depths, voxel_size, masks, obs_weight, H, W, V, X, Y, Z,
+                     trunc_weight, tsdf_th_low, tsdf_th_high);
   return sailor::check_launch("integrate");
 }
 
@@ -413,7 +609,7 @@ extern "C" int sailor_integrate(
   return integrate_impl(false, occ_vol, num_occ, K, RT, R, T, colors, depths, B, V, H, W, X, Y,
                         Z, obs_weight, th_bbox, trunc_weight, tsdf_th_low, tsdf_th_high,
                         fixed_bbox, tsdf, weight, color, vol_origin, vol_bbox, voxel_size,
-                        stream);
+                        nullptr, 0, stream);
 }
 
 extern "C" int sailor_integrate_compensated(
@@ -428,7 +624,21 @@ extern "C" int sailor_integrate_compensated(
   return integrate_impl(true, occ_vol, num_occ, K, RT, R, T, colors, depths, B, V, H, W, X, Y,
                         Z, obs_weight, th_bbox, trunc_weight, tsdf_th_low, tsdf_th_high,
                         fixed_bbox, tsdf, weight, color, vol_origin, vol_bbox, voxel_size,
-                        stream);
+                        nullptr, 0, stream);
+}
+
+extern "C" int sailor_integrate_workspace(
+    int compensated, int32_t* occ_vol, int32_t* num_occ, const float* K, const float* RT,
+    const float* R, const float* T, const float* colors, const float* depths, int B, int V,
+    int H, int W, int X, int Y, int Z, float obs_weight, float th_bbox, float trunc_weight,
+    float tsdf_th_low, float tsdf_th_high, const float* fixed_bbox, float* tsdf, float* weight,
+    float* color, float* vol_origin, float* vol_bbox, float* voxel_size, void* workspace,
+    size_t workspace_bytes, void* stream) {
+  SAILOR_REQUIRE(workspace != nullptr, "integrate: workspace missing");
+  return integrate_impl(compensated != 0, occ_vol, num_occ, K, RT, R, T, colors, depths, B, V, H,
+                        W, X, Y, Z, obs_weight, th_bbox, trunc_weight, tsdf_th_low,
+                        tsdf_th_high, fixed_bbox, tsdf, weight, color, vol_origin, vol_bbox,
+                        voxel_size, workspace, workspace_bytes, stream);
 }
 
 extern "C" int sailor_get_origin_bbox(const float* depths, const float* K,

@@ -111,6 +111,8 @@ class FramePipeline:
         self.tsdf = torch.empty((1, d, d, d), dtype=_f32, **o)
         self.weight = torch.empty_like(self.tsdf)
         self.color = torch.empty_like(self.tsdf)
+        self.integrate_ws = torch.empty(
+            _lib.lib().sailor_integrate_workspace_bytes(1, V, n, n, d, d, d), dtype=torch.uint8, **o)
         self.origin = torch.empty((1, 3, 2), dtype=_f32, **o)
         self.bbox = torch.empty((1, 3, 2), dtype=_f32, **o)
         self.vs = torch.empty((1, 1), dtype=_f32, **o)
@@ -193,12 +195,13 @@ class FramePipeline:
         elif self.fmap_lo is not None:
             self.fmap_lo.copy_(self.fmap)
         self.num.zero_()
-        call("sailor_integrate_compensated" if self.compensated else "sailor_integrate",
+        call("sailor_integrate_workspace", int(self.compensated),
              ptr(self.occ0), ptr(self.num[0]), ptr(self.K), ptr(self.RT),
-             ptr(self.R), ptr(self.T), ptr(self.colors), ptr(self.depths), ptr(self.masks), 1,
+             ptr(self.R), ptr(self.T), ptr(self.colors), ptr(self.depths), 1,
              V, n, n, d, d, d, 1.0, 0.025, cfg.trunc_weight, cfg.th_low, cfg.th_high,
              ptr(self.fixed_bbox), ptr(self.tsdf), ptr(self.weight), ptr(self.color),
-             ptr(self.origin), ptr(self.bbox), ptr(self.vs), st)
+             ptr(self.origin), ptr(self.bbox), ptr(self.vs), ptr(self.integrate_ws),
+             self.integrate_ws.numel(), st)
         vols = _ptr_array([self.occ0, self.occ1])
         cnts = _ptr_array([self.num[0], self.num[1]])
         call("sailor_build_multi_res_volumes", vols, cnts, 2, 1, d, cfg.rate, st)

@@ -138,6 +138,81 @@ def test_integrate_volumes(case):
         np.testing.assert_array_equal(g[k], o[k], err_msg=k)
 
 
+def _cull_cameras(kind, HW, fx):
+    """Camera sets whose culling has something to get wrong: cameras inside and
+    beside the volume, looking away from it, far from the world's origin, and
+    9 views (more than one pass of 8)."""
+    from sailor_amd import scenes
+    if kind == "ring9":
+        cams = scenes.ring_cameras(9, fx, HW, HW)
+    elif kind == "inside":
+        cams = [scenes.look_at_camera(c, fx, HW, HW, target=t) for c, t in
+                [((0.1, 1.0, 0.2), (0.9, 1.1, 0.3)), ((0.0, 1.0, 1.2), (0.1, 1.0, 0.0)),
+                 ((1.1, 0.4, 0.0), (3.0, 0.4, 0.2))]]
+    else:
+        cams = scenes.ring_cameras(3, fx, HW, HW)
+    K = np.stack([c.K for c in cams])
+    RT = np.stack([c.RT for c in cams])
+    return K, RT
+
+
+@pytest.mark.parametrize("comp", [0, 1])
+@pytest.mark.parametrize("kind,HW,dims", [
+    ("ring9", (61, 83), (33, 18, 47)), ("inside", (64, 48), (32, 32, 32)),
+    ("ring3", (16, 16), (2, 1, 1)), ("far", (130, 97), (40, 9, 16)),
+    ("nan", (40, 200), (17, 33, 65))])
+def test_integrate_skips_only_views_that_see_nothing(kind, HW, dims, comp):
+    """The entry that skips views per brick writes what the one that evaluates
+    every view at every voxel does, bit for bit."""
+    from sailor_amd import _lib, scenes
+    from sailor_amd._lib import call, ptr, stream_of
+    (H, W), (X, Y, Z) = HW, dims
+    B = 2
+    rng = np.random.default_rng(5)
+    K, RT = _cull_cameras(kind, max(H, W), 0.9 * max(H, W))
+    V = len(K)
+    y, x = np.mgrid[0:H, 0:W]
+    depths = np.where(((x // 11 + y // 7) % 3 == 0), rng.uniform(0.05, 4.2, (B, V, H, W)),
+                      0.0).astype(np.float32)
+    depths[1, :, H // 2:] = 0.0
+    box = np.stack([scenes.fixed_cube()] * B)
+    if kind == "nan":
+        depths[0, 0, 3, 5] = np.nan
+        depths[0, 1, :9] = np.inf
+        K[2, 1, 1] = np.nan
+    if kind == "far":
+        RT[:, :, 3] -= RT[:, :, :3] @ np.float32([512.0, 0.0, -256.0])
+        box += np.float32([512.0, 0.0, -256.0])[None, :, None]
+    K, RT = np.stack([K] * B), np.stack([RT] * B)
+    ins = [_t(np.float32(a)) for a in (K, RT, RT[..., :3], RT[..., 3],
+                                       np.floor(rng.uniform(0, 2 ** 24, depths.shape)), depths)]
+    fb, dev = _t(np.float32(box)), torch.device("cuda")
+    masks = torch.zeros(depths.shape, dtype=torch.int32, device=dev)
+    outs = []
+    for culled in (False, True):
+        occ = torch.full((B, X, Y, Z), -7, dtype=torch.int32, device=dev)
+        num = torch.zeros(B, dtype=torch.int32, device=dev)
+        vols = [torch.full((B, X, Y, Z), np.nan, device=dev) for _ in range(3)]
+        small = [torch.empty(B * 6, device=dev), torch.empty(B * 6, device=dev),
+                 torch.empty(B, device=dev)]
+        args = [ptr(occ), ptr(num)] + [ptr(t) for t in ins]
+        tail = [B, V, H, W, X, Y, Z, 1.0, 0.025, 3.0, 13.5, 13.5, ptr(fb)] + [
+            ptr(t) for t in vols + small]
+        if culled:
+            ws = torch.empty(_lib.lib().sailor_integrate_workspace_bytes(
+                B, V, H, W, X, Y, Z), dtype=torch.uint8, device=dev)
+            call("sailor_integrate_workspace", comp, *args, *tail, ptr(ws), ws.numel(),
+                 stream_of(dev))
+        else:
+            call("sailor_integrate_compensated" if comp else "sailor_integrate", *args,
+                 ptr(masks), *tail, stream_of(dev))
+        outs.append([t.cpu().numpy() for t in [occ, num] + vols])
+    for name, a, b in zip(("occ", "num", "tsdf", "weight", "color"), *outs):
+        np.testing.assert_array_equal(a, b, err_msg=name)
+    if kind in ("ring9", "far"):
+        assert (outs[0][3] > 0).any()
+
+
 def test_multi_res_merge(case):
     g, o = case
     np.testing.assert_array_equal(g["coarse"], o["coarse"])
