@@ -1523,6 +1523,7 @@ __device__ __forceinline__ void write_vals16(typename Tr<PREC>::E* dst,
                                              int lane) {
   typedef typename Tr<PREC>::E E;
   typedef typename Tr<PREC>::V8 V8;
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
   const int c = lane & 31, h = lane >> 5;
 #pragma unroll
   for (int mt = 0; mt < H / 128; ++mt) {
@@ -1533,12 +1534,13 @@ __device__ __forceinline__ void write_vals16(typename Tr<PREC>::E* dst,
       for (int e = 0; e < 2; ++e) {
         const int off = act_chunk<H, PREC>(32 * nt + c, u0 / 8 + e);
         V8 v;
-        V8 m;
-        if (mask) m = *reinterpret_cast<const V8*>(mask + off);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const float x = acc[mt][nt][8 * e + k];
-          v[k] = (E)((!mask || (float)m[k] > 0.0f) ? x : 0.0f);
+        for (int k = 0; k < 8; ++k) v[k] = (E)acc[mt][nt][8 * e + k];
+        if (mask) {
+          // the mask is a ReLU's output: all ones where its bits are positive
+          const s16x8 m = *reinterpret_cast<const s16x8*>(mask + off);
+          const s16x8 keep = 0 - __builtin_elementwise_min(m, (s16x8)1);
+          v = __builtin_bit_cast(V8, __builtin_bit_cast(s16x8, v) & keep);
         }
         *reinterpret_cast<V8*>(dst + off) = v;
       }
@@ -1620,6 +1622,29 @@ __device__ __forceinline__ void one_layer16(const typename Tr<PREC>::E* Wl,
   run_layer16<H, PREC, NT, UL, 0>(wb, wb, lane_off, in, lane, abuf, bbuf, bc, acc);
 }
 
+// one_layer16 for a sequence of layers: the first weights of this one are in
+// abuf (from buffer O on), those of the next are loaded into it on the way.
+template <int H, int PREC, int K, int O>
+__device__ __forceinline__ void chain_layer16(
+    const char* cur, const char* nxt, unsigned lane_off, const typename Tr<PREC>::E* in,
+    const float* bias, int wave, int lane,
+    typename Chain16<H, PREC, 1>::V (&abuf)[Chain16<H, PREC, 1>::NB][H / 128],
+    f32x16 (&acc)[H / 128][1]) {
+  typedef Chain16<H, PREC, 1> C;
+  typename C::V bbuf[2][1];
+  f32x16 bc[C::M32];
+  if (bias) {
+    load_bias16<H>(bias, wave, lane, bc);
+  } else {
+#pragma unroll
+    for (int mt = 0; mt < C::M32; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bc[mt][r] = 0.0f;
+  }
+  read_b16<H, PREC, 1>(in, 0, lane, bbuf[0]);
+  run_layer16<H, PREC, 1, K / 16, O>(cur, nxt, lane_off, in, lane, abuf, bbuf, bc, acc);
+}
+
 // Copies NC columns x K elements of a swizzled LDS buffer to rows of a
 // [C, H]-strided matrix in global memory (16-byte chunks).
 template <int H, int PREC, int NC, int K>
@@ -1676,28 +1701,41 @@ __device__ __forceinline__ typename Tr<PREC>::V8 col_operand(const typename Tr<P
 
 // 16-bit forms, v_mfma_f32_32x32x16: A operand = D^T (lane: unit 32w + l%32,
 // columns c0 + 8(l/32) + j), B operand = A_l (columns c0 + 8(l/32) + j,
-// input 32n + l%32); accumulator r of tile n holds
-// dW[32w + 8(r/4) + 4(l/32) + r%4][32n + l%32].
+// input 32t + l%32); accumulator r of a tile t holds
+// dW[32w + 8(r/4) + 4(l/32) + r%4][32t + l%32].  The two waves of a unit range
+// take input tiles t = 2 half + n; the first of them sums the biases.
 template <int H, int PREC, int NC, int K>
 __device__ __forceinline__ void accum_dw16(const typename Tr<PREC>::E* D,
-                                           const typename Tr<PREC>::E* A,
-                                           f32x16 (&dw)[K / 32], float& db, int wave, int lane) {
+                                           const typename Tr<PREC>::E* A, f32x16 (&dw)[2],
+                                           float& db, int wave, int half, int lane) {
   typedef typename Tr<PREC>::V8 V8;
-  static_assert(H == 128 && NC % 16 == 0 && K % 32 == 0, "32 units per wave, whole tiles");
+  static_assert(H == 128 && NC % 16 == 0 && K % 32 == 0 && K > 64, "32 units per wave");
 #pragma unroll
   for (int s = 0; s < NC / 16; ++s) {
     const V8 a = col_operand<H, PREC>(D, 16 * s, 32 * wave, lane);
+    if constexpr (PREC == kBF16) {
+      typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+      const b2 one = {(__bf16)1.0f, (__bf16)1.0f};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) db += (float)a[j];
+      for (int j = 0; j < 8; j += 2)
+        db = __builtin_amdgcn_fdot2_f32_bf16(b2{a[j], a[j + 1]}, one, db, false);
+    } else if (half == 0) {
 #pragma unroll
-    for (int n = 0; n < K / 32; ++n) {
-      const V8 b = col_operand<H, PREC>(A, 16 * s, 32 * n, lane);
+      for (int j = 0; j < 8; ++j) db += (float)a[j];
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      if (K < 128 && 64 * half + 32 * n >= K) continue;
+      const V8 b = col_operand<H, PREC>(A, 16 * s, 64 * half + 32 * n, lane);
       if constexpr (PREC == kBF16)
         dw[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, dw[n], 0, 0, 0);
       else
         dw[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, dw[n], 0, 0, 0);
     }
   }
+  // keeps the sums here: sunk to where the loop next needs them, they would
+  // hold all their operands in registers
+  asm volatile("" : "+v"(dw[0]), "+v"(dw[1]), "+v"(db));
 }
 
 // fp32 form, v_mfma_f32_16x16x4f32: two 16-unit tiles per wave; A operand =
@@ -1731,8 +1769,7 @@ __device__ __forceinline__ void accum_dw32(const float* D, const float* A,
 }
 
 // Per-wave register accumulators of the four layers' weight gradients.
-template <int F, int H, int PREC> struct DenseAcc;
-template <int F, int H> struct DenseAcc<F, H, kF32> {
+template <int F, int H> struct DenseAcc {
   static constexpr int K0 = F + kPeSlots;
   f32x4 w0[2][K0 / 16], w1[2][H / 16], w2[2][H / 16], w3[2][H / 16];
   float b[4][2];
@@ -1782,51 +1819,176 @@ template <int F, int H> struct DenseAcc<F, H, kF32> {
       }
   }
 };
-template <int F, int H, int PREC> struct DenseAcc16 {
+// 16-bit forms: the input tiles of a wave's half (accum_dw16).
+template <int F, int H> struct DenseAcc16 {
   static constexpr int K0 = F + kPeSlots;
-  f32x16 w0[K0 / 32], w1[H / 32], w2[H / 32], w3[H / 32];
+  f32x16 w0[2], w1[2], w2[2], w3[2];
   float b[4];
   __device__ __forceinline__ void zero() {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int n = 0; n < K0 / 32; ++n) w0[n][i] = 0.0f;
-#pragma unroll
-      for (int n = 0; n < H / 32; ++n) {
-        w1[n][i] = 0.0f;
-        w2[n][i] = 0.0f;
-        w3[n][i] = 0.0f;
-      }
-    }
+      for (int n = 0; n < 2; ++n) w0[n][i] = w1[n][i] = w2[n][i] = w3[n][i] = 0.0f;
 #pragma unroll
     for (int l = 0; l < 4; ++l) b[l] = 0.0f;
   }
-  template <int NTW>
-  __device__ __forceinline__ void store_tiles(float* dst, const f32x16 (&w)[NTW], int K,
-                                              int wave, int lane) {
-    const int r = lane & 31, half = lane >> 5;
+  __device__ __forceinline__ void store_tiles(float* dst, const f32x16 (&w)[2], int K, int wave,
+                                              int half, int lane) {
+    const int r = lane & 31, q = lane >> 5;
 #pragma unroll
-    for (int n = 0; n < NTW; ++n)
+    for (int n = 0; n < 2; ++n) {
+      if (64 * half + 32 * n >= K) continue;
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        dst[(size_t)(32 * wave + 8 * (i / 4) + 4 * half + i % 4) * K + 32 * n + r] = w[n][i];
+        dst[(size_t)(32 * wave + 8 * (i / 4) + 4 * q + i % 4) * K + 64 * half + 32 * n + r] =
+            w[n][i];
+    }
   }
-  __device__ __forceinline__ void store(float* gd, int wave, int lane) {
-    store_tiles(gd + dense_grad_offset(F, H, 0), w0, K0, wave, lane);
-    store_tiles(gd + dense_grad_offset(F, H, 1), w1, H, wave, lane);
-    store_tiles(gd + dense_grad_offset(F, H, 2), w2, H, wave, lane);
-    store_tiles(gd + dense_grad_offset(F, H, 3), w3, H, wave, lane);
-    const int r = lane & 31, half = lane >> 5;
+  __device__ __forceinline__ void store(float* gd, int wave, int half, int lane) {
+    store_tiles(gd + dense_grad_offset(F, H, 0), w0, K0, wave, half, lane);
+    store_tiles(gd + dense_grad_offset(F, H, 1), w1, H, wave, half, lane);
+    store_tiles(gd + dense_grad_offset(F, H, 2), w2, H, wave, half, lane);
+    store_tiles(gd + dense_grad_offset(F, H, 3), w3, H, wave, half, lane);
     float* gb = gd + dense_grad_offset(F, H, 4);
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
       const float v = b[l] + __shfl_xor(b[l], 32, 64);
-      if (half == 0) gb[l * H + 32 * wave + r] = v;
+      if (half == 0 && lane < 32) gb[l * H + 32 * wave + lane] = v;
     }
   }
 };
-template <int F, int H> struct DenseAcc<F, H, kBF16> : DenseAcc16<F, H, kBF16> {};
-template <int F, int H> struct DenseAcc<F, H, kF16> : DenseAcc16<F, H, kF16> {};
+
+// Maps a volume box to [-1, 1]^3.
+struct BoxMap {
+  const float cx, cy, cz, ihx, ihy, ihz;
+  __device__ __forceinline__ explicit BoxMap(const float* bb)
+      : cx(0.5f * (bb[0] + bb[1])), cy(0.5f * (bb[2] + bb[3])), cz(0.5f * (bb[4] + bb[5])),
+        ihx(2.0f / (bb[1] - bb[0])), ihy(2.0f / (bb[3] - bb[2])), ihz(2.0f / (bb[5] - bb[4])) {}
+};
+
+// Features of all samples and views of a ray into keep, and on the way g_i =
+// dL/dtoken . f(x_i) into s_g: item `it` is (sample it / 16, view it / 4 % 4,
+// channel quarter it % 4), so a sample's 16 items are 16 consecutive lanes;
+// each dots its quarter of the channels with dL/dtoken (dtok), and four
+// shuffles add the quarters and the views.
+template <int F, int PREC, int NTHR>
+__device__ __forceinline__ void ray_features(const RenderArgs& a, int b, const float* dtok,
+                                             const float* s_pos, int S, int tid, float* keep,
+                                             float* s_g) {
+  constexpr int CPL = F / 4, KF = F + 4;
+  for (int it = tid; it < S * kVP * 4; it += NTHR) {
+    const int col = it >> 2, quarter = it & 3;
+    const int sl = col >> 2, v = col & 3;
+    float f[CPL];
+    gather_quarter<F, PREC, false>(a, b, v, s_pos[4 * sl], s_pos[4 * sl + 1],
+                                   s_pos[4 * sl + 2], quarter, f);
+    float* kp = keep + col * KF + quarter * CPL;
+#pragma unroll
+    for (int c = 0; c < CPL; c += 4)
+      *reinterpret_cast<f32x4*>(kp + c) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
+    const float* dtv = dtok + v * F + quarter * CPL;
+    float part = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CPL; c += 4) {
+      const f32x4 d4 = *reinterpret_cast<const f32x4*>(dtv + c);
+      part += d4[0] * f[c] + d4[1] * f[c + 1] + d4[2] * f[c + 2] + d4[3] * f[c + 3];
+    }
+    part += __shfl_xor(part, 1, 64);
+    part += __shfl_xor(part, 2, 64);
+    part += __shfl_xor(part, 4, 64);
+    part += __shfl_xor(part, 8, 64);
+    if ((it & 15) == 0) s_g[sl] = part;
+  }
+}
+
+// Compositing replayed and walked back by one wave, sample i in lane i (S <=
+// 64): the recurrences run in sample order on values broadcast with readlane,
+// the same operations in the same order as the forward's (so the early
+// termination is the forward's), without a branch per sample; what each sample
+// does with its own T and U is done for all of them at once afterwards.  s_dz:
+// dL/d pre-sigmoid; its sum is added to gsb.
+__device__ __forceinline__ void composite_backward(const float* s_alpha, const float* s_g, int S,
+                                                   float t_thres, int lane, float* s_dz,
+                                                   double& gsb) {
+  const float al = lane < S ? s_alpha[lane] : 0.0f;
+  const float gl = lane < S ? s_g[lane] : 0.0f;
+  const float om = 1.0f - al;
+  float T = 1.0f, myT = 0.0f;
+  for (int i0 = 0; i0 < S; i0 += 4)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (lane == i0 + k) myT = T;
+      T *= lane_value(om, i0 + k);
+    }
+  const unsigned long long stop = __ballot(lane < S && myT * om < t_thres);
+  const int last = stop ? __ffsll((long long)stop) - 1 : S - 1;
+  // samples behind the last leave U at 0
+  const float omb = lane <= last ? om : 1.0f, ab = lane <= last ? al : 0.0f;
+  const float gb = lane <= last ? gl : 0.0f;
+  float U = 0.0f, myU = 0.0f;
+  for (int i0 = (S - 1) & ~3; i0 >= 0; i0 -= 4)
+#pragma unroll
+    for (int k = 3; k >= 0; --k) {
+      if (lane == i0 + k) myU = U;
+      U = __builtin_fmaf(lane_value(gb, i0 + k), lane_value(ab, i0 + k),
+                         lane_value(omb, i0 + k) * U);
+    }
+  const float d = myT * (gl - myU) * al * om;
+  const float myd = lane <= last ? d : 0.0f;
+  if (lane < S) s_dz[lane] = myd;
+  double dsum = myd;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) dsum += __shfl_xor(dsum, off, 64);
+  if (lane == 0) gsb += dsum;
+}
+
+// Layer-0 input of the chunk at sample c0: features (from keep) and positional
+// encoding, by threads t0, t0 + tstep, ...
+template <int F, int H, int PREC, int NS>
+__device__ __forceinline__ void build_input(const float* keep, const float* s_pos,
+                                            const BoxMap box, int c0, int t0, int tstep,
+                                            typename Tr<PREC>::E* x0) {
+  typedef typename Tr<PREC>::E E;
+  constexpr int NC = NS * kVP, CE = Tr<PREC>::CE, KF = F + 4;
+  for (int it = t0; it < NC * (F / CE); it += tstep) {
+    const int col = it % NC, ch = it / NC;   // consecutive lanes: consecutive columns
+    const float* kp = keep + ((c0 + (col >> 2)) * kVP + (col & 3)) * KF + ch * CE;
+    E* d = x0 + act_chunk<H, PREC>(col, ch);
+    if constexpr (PREC == kF32) {
+      *reinterpret_cast<f32x4*>(d) = *reinterpret_cast<const f32x4*>(kp);
+    } else {
+      typename Tr<PREC>::V8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = (E)kp[e];
+      *reinterpret_cast<typename Tr<PREC>::V8*>(d) = h;
+    }
+  }
+  // positional encoding: a thread per (sample, frequency, axis) -> its sine
+  // and cosine in the rows of the sample's view slots
+  for (int it = t0; it < NS * 32; it += tstep) {
+    const int sl = it >> 5, q = it & 31;
+    const float* ps = s_pos + 4 * (c0 + sl);
+    const float xn[3] = {(ps[0] - box.cx) * box.ihx, (ps[1] - box.cy) * box.ihy,
+                         (ps[2] - box.cz) * box.ihz};
+    auto put = [&](int k, float val) {
+#pragma unroll
+      for (int v = 0; v < kVP; ++v)
+        x0[act_chunk<H, PREC>(sl * kVP + v, k / CE) + k % CE] = (E)val;
+    };
+    if (q < 30) {
+      const int fr = q / 3, ax = q - 3 * fr;
+      float sn, cs;
+      sincos_pe<PREC>(ldexpf(ax == 0 ? xn[0] : (ax == 1 ? xn[1] : xn[2]), fr), sn, cs);
+      put(F + 3 + 6 * fr + ax, sn);
+      put(F + 6 + 6 * fr + ax, cs);
+    } else if (q == 30) {
+      put(F + 0, xn[0]);
+      put(F + 1, xn[1]);
+      put(F + 2, xn[2]);
+      put(F + 63, 0.0f);
+    }
+  }
+}
 
 // DW: weight gradients accumulated in registers (H = 128 forms) instead of
 // column matrices written for separate GEMMs.
@@ -1842,6 +2004,7 @@ render_backward_kernel(BackArgs ba) {
   constexpr bool F32 = PREC == kF32;
   constexpr int NTL = NC / 16, NT32 = NC / 32;
   static_assert(F32 || NC % 32 == 0, "16-bit forms need chunks of a multiple of 8 samples");
+  static_assert(F32 || !DW, "render_backward16_kernel accumulates weight gradients");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   E* x0 = reinterpret_cast<E*>(smem + L::x0);
   auto hb = [&](int l) { return reinterpret_cast<E*>(smem + L::h0 + l * L::buf); };
@@ -1872,7 +2035,7 @@ render_backward_kernel(BackArgs ba) {
 #pragma unroll
   for (int u = 0; u < NU; ++u) gsw[u] = 0.0f;
   double gsb = 0.0;   // occupancy-bias gradient: a sum of many cancelling terms
-  [[maybe_unused]] DenseAcc<F, H, PREC> dacc;
+  [[maybe_unused]] DenseAcc<F, H> dacc;   // fp32 only (the 16-bit forms: below)
   if constexpr (DW) dacc.zero();
 
   const long long item_end = std::min<long long>(ba.item_end, (long long)*a.n_valid);
@@ -1882,11 +2045,7 @@ render_backward_kernel(BackArgs ba) {
     const int b = (int)(ray / a.rays_per_batch);
     const float* trow = a.t + ray * S;
     const float* rr = a.rays + ray * 6;
-    const float* bb = a.bbox + b * 6;
-    const float cx = 0.5f * (bb[0] + bb[1]), cy = 0.5f * (bb[2] + bb[3]),
-                cz = 0.5f * (bb[4] + bb[5]);
-    const float ihx = 2.0f / (bb[1] - bb[0]), ihy = 2.0f / (bb[3] - bb[2]),
-                ihz = 2.0f / (bb[5] - bb[4]);
+    const BoxMap box(a.bbox + b * 6);
     if (tid < S) {
       const float tv = trow[tid];
       s_pos[4 * tid + 0] = rr[0] + tv * rr[3];
@@ -1895,116 +2054,19 @@ render_backward_kernel(BackArgs ba) {
       s_alpha[tid] = ba.occ[ray * S + tid];
     }
     __syncthreads();
-    // 1. features of all samples and views, and on the way
-    // 2. g_i = dL/dtoken . f(x_i): item `it` is (sample it / 16, view it / 4 %
-    // 4, channel quarter it % 4), so a sample's 16 items are 16 consecutive
-    // lanes; each dots its quarter of the channels with dL/dtoken, and four
-    // shuffles add the quarters and the views
-    for (int it = tid; it < S * kVP * 4; it += kThreads) {
-      const int col = it >> 2, quarter = it & 3;
-      const int sl = col >> 2, v = col & 3;
-      float f[CPL];
-      gather_quarter<F, PREC, false>(a, b, v, s_pos[4 * sl], s_pos[4 * sl + 1],
-                                     s_pos[4 * sl + 2], quarter, f);
-      float* kp = keep + col * KF + quarter * CPL;
-#pragma unroll
-      for (int c = 0; c < CPL; c += 4)
-        *reinterpret_cast<f32x4*>(kp + c) = f32x4{f[c], f[c + 1], f[c + 2], f[c + 3]};
-      const float* dtv = ba.dtok + item * kVP * F + v * F + quarter * CPL;
-      float part = 0.0f;
-#pragma unroll
-      for (int c = 0; c < CPL; c += 4) {
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(dtv + c);
-        part += d4[0] * f[c] + d4[1] * f[c + 1] + d4[2] * f[c + 2] + d4[3] * f[c + 3];
-      }
-      part += __shfl_xor(part, 1, 64);
-      part += __shfl_xor(part, 2, 64);
-      part += __shfl_xor(part, 4, 64);
-      part += __shfl_xor(part, 8, 64);
-      if ((it & 15) == 0) s_g[sl] = part;
-    }
+    ray_features<F, PREC, kThreads>(a, b, ba.dtok + item * kVP * F, s_pos, S, tid, keep, s_g);
     __syncthreads();
-    // layer-0 input of the chunk at sample c0: features (from keep) and
-    // positional encoding, by threads t0, t0 + tstep, ... (building the
-    // first chunk's on waves 1-3 during the replay measured no faster: the
-    // second copy of this code spills registers)
-    auto build_input = [&](int c0, int t0, int tstep) {
-      for (int it = t0; it < NC * (F / CE); it += tstep) {
-        const int col = it % NC, ch = it / NC;   // consecutive lanes: consecutive columns
-        const float* kp = keep + ((c0 + (col >> 2)) * kVP + (col & 3)) * KF + ch * CE;
-        E* d = x0 + act_chunk<H, PREC>(col, ch);
-        if constexpr (F32) {
-          *reinterpret_cast<f32x4*>(d) = *reinterpret_cast<const f32x4*>(kp);
-        } else {
-          typename Tr<PREC>::V8 h;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) h[e] = (E)kp[e];
-          *reinterpret_cast<typename Tr<PREC>::V8*>(d) = h;
-        }
-      }
-      // positional encoding: a thread per (sample, frequency, axis) -> its sine
-      // and cosine in the rows of the sample's view slots
-      for (int it = t0; it < NS * 32; it += tstep) {
-        const int sl = it >> 5, q = it & 31;
-        const float* ps = s_pos + 4 * (c0 + sl);
-        const float xn[3] = {(ps[0] - cx) * ihx, (ps[1] - cy) * ihy, (ps[2] - cz) * ihz};
-        auto put = [&](int k, float val) {
-#pragma unroll
-          for (int v = 0; v < kVP; ++v)
-            x0[act_chunk<H, PREC>(sl * kVP + v, k / CE) + k % CE] = (E)val;
-        };
-        if (q < 30) {
-          const int fr = q / 3, ax = q - 3 * fr;
-          float sn, cs;
-          sincos_pe<PREC>(ldexpf(ax == 0 ? xn[0] : (ax == 1 ? xn[1] : xn[2]), fr), sn, cs);
-          put(F + 3 + 6 * fr + ax, sn);
-          put(F + 6 + 6 * fr + ax, cs);
-        } else if (q == 30) {
-          put(F + 0, xn[0]);
-          put(F + 1, xn[1]);
-          put(F + 2, xn[2]);
-          put(F + 63, 0.0f);
-        }
-      }
+    if (wave == 0) composite_backward(s_alpha, s_g, S, a.t_thres, lane, s_dz, gsb);
+    __syncthreads();
+    // the lambda keeps build_input's inlining late: called directly, the fp32
+    // form spills 50 more registers
+    auto input = [&](int c0) {
+      build_input<F, H, PREC, NS>(keep, s_pos, box, c0, tid, kThreads, x0);
     };
-    // 3. compositing replayed and walked back by wave 0 from registers,
-    // sample i in lane i: the recurrences run in sample order on values
-    // broadcast with readlane, the same operations in the same order as the
-    // forward's (so the early termination is the forward's)
-    if (wave == 0) {
-      const float al = lane < S ? s_alpha[lane] : 0.0f;
-      const float gl = lane < S ? s_g[lane] : 0.0f;
-      float T = 1.0f, myT = 0.0f;
-      int last = S - 1;
-      for (int i = 0; i < S; ++i) {
-        const float ai = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(al), i));
-        if (lane == i) myT = T;
-        T *= 1.0f - ai;
-        if (__builtin_amdgcn_readfirstlane((int)(T < a.t_thres))) {
-          last = i;
-          break;
-        }
-      }
-      float U = 0.0f, myd = 0.0f;
-      for (int i = last; i >= 0; --i) {
-        const float ai = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(al), i));
-        const float gi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gl), i));
-        const float ti = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myT), i));
-        const float d = ti * (gi - U) * ai * (1.0f - ai);
-        if (lane == i) myd = d;
-        U = gi * ai + (1.0f - ai) * U;
-      }
-      if (lane < S) s_dz[lane] = myd;
-      double dsum = myd;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) dsum += __shfl_xor(dsum, off, 64);
-      if (lane == 0) gsb += dsum;
-    }
-    __syncthreads();
     // 4./5. per chunk
     for (int c0 = 0; c0 < S; c0 += NS) {
       const long long col0 = (item - ba.item_begin) * S * kVP + (long long)c0 * kVP;
-      build_input(c0, tid, kThreads);
+      input(c0);
       __syncthreads();
       if constexpr (!DW) store_cols<H, PREC, NC, K0>(x0, ba.A0, col0, tid);
       if constexpr (F32) {
@@ -2096,14 +2158,10 @@ render_backward_kernel(BackArgs ba) {
         }
         write_vals16<H, PREC, NT32>(dl, acc, nullptr, wave, lane);
         __syncthreads();
-        if constexpr (DW) {
-          accum_dw16<H, PREC, NC, H>(dl, hb(2), dacc.w3, dacc.b[3], wave, lane);
-        } else {
-          store_cols<H, PREC, NC, H>(dl, ba.D3, col0, tid);
-          store_cols<H, PREC, NC, H>(hb(0), ba.A1, col0, tid);
-          store_cols<H, PREC, NC, H>(hb(1), ba.A2, col0, tid);
-          store_cols<H, PREC, NC, H>(hb(2), ba.A3, col0, tid);
-        }
+        store_cols<H, PREC, NC, H>(dl, ba.D3, col0, tid);
+        store_cols<H, PREC, NC, H>(hb(0), ba.A1, col0, tid);
+        store_cols<H, PREC, NC, H>(hb(1), ba.A2, col0, tid);
+        store_cols<H, PREC, NC, H>(hb(2), ba.A3, col0, tid);
         void* Ds[3] = {ba.D2, ba.D1, ba.D0};
 #pragma unroll
         for (int l = 0; l < 3; ++l) {
@@ -2111,13 +2169,7 @@ render_backward_kernel(BackArgs ba) {
           __syncthreads();
           write_vals16<H, PREC, NT32>(dl, acc, hb(2 - l), wave, lane);
           __syncthreads();
-          if constexpr (DW) {
-            if (l == 0) accum_dw16<H, PREC, NC, H>(dl, hb(1), dacc.w2, dacc.b[2], wave, lane);
-            else if (l == 1) accum_dw16<H, PREC, NC, H>(dl, hb(0), dacc.w1, dacc.b[1], wave, lane);
-            else accum_dw16<H, PREC, NC, K0>(dl, x0, dacc.w0, dacc.b[0], wave, lane);
-          } else {
-            store_cols<H, PREC, NC, H>(dl, Ds[l], col0, tid);
-          }
+          store_cols<H, PREC, NC, H>(dl, Ds[l], col0, tid);
         }
       }
       __syncthreads();
@@ -2147,6 +2199,206 @@ render_backward_kernel(BackArgs ba) {
   if (tid == 0) gp[so.sigma_b] += (float)gsb;
   if constexpr (DW)
     dacc.store(ba.gdense + (size_t)blockIdx.x * dense_grad_total(F, H), wave, lane);
+}
+
+// The 16-bit forms with weight gradients accumulated in registers (H = 128): 8
+// waves, two per SIMD, where wave w + 4 half owns output units 32 w .. + 31 of
+// the chunk's column half `half` in every layer, and K half `half` of those
+// units' weight gradients (128 of its 256 registers).  A chunk's 13 dependent
+// phases bound it, not its MFMAs (5.4k of about 17k cycles a chunk and SIMD):
+// two waves per SIMD overlap them, each layer's first weights are loaded during
+// the phase before, the deltas alternate between two buffers (9 barriers a
+// chunk), the replay of the compositing runs beside the first chunk's input and
+// the next ray's samples are loaded a ray ahead.  524288 rays, 28 % of them with
+// 48 samples and 4 views each: 18.0 ms; 4 waves that each owned all columns and
+// inputs of their units (one per SIMD, 14 barriers): 25.0 ms.
+constexpr int kBackWaves = 8;
+
+template <int F, int H, int PREC, int NS, int SMAX>
+__global__ void __launch_bounds__(kBackWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+render_backward16_kernel(BackArgs ba) {
+  typedef typename Tr<PREC>::E E;
+  typedef SmemB<F, H, PREC, NS, SMAX> L;
+  typedef Chain16<H, PREC, 1> C;
+  constexpr int NTHR = kBackWaves * 64, NC = L::NC, K0 = F + kPeSlots;
+  constexpr int U0 = K0 / 16, UH = C::UH, NB = C::NB, PD = C::PD;
+  constexpr int O0 = (NB - U0 % NB) % NB;   // layer 0's first buffer: layer 1 starts at 0
+  constexpr SmallOffsets so = small_offsets(F, H);
+  static_assert(H == 128 && NC == 64, "32 units and 32 columns per wave");
+  const RenderArgs& a = ba.r;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  E* x0 = reinterpret_cast<E*>(smem + L::x0);
+  E* h0 = reinterpret_cast<E*>(smem + L::h0);
+  E* h1 = reinterpret_cast<E*>(smem + L::h1);
+  E* h2 = reinterpret_cast<E*>(smem + L::h2);
+  E* da = reinterpret_cast<E*>(smem + L::dl);
+  E* db = reinterpret_cast<E*>(smem + L::total);
+  float* keep = reinterpret_cast<float*>(smem + L::keep);
+  float* s_alpha = reinterpret_cast<float*>(smem + L::alpha);
+  float* s_g = reinterpret_cast<float*>(smem + L::gw);
+  float* s_dz = reinterpret_cast<float*>(smem + L::dz);
+  float* s_pos = reinterpret_cast<float*>(smem + L::pos);
+  float* s_bias = reinterpret_cast<float*>(smem + L::bias);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wid & 3, half = wid >> 2;
+  const int S = a.S, V = a.V;
+  const float* ws = a.wsmall;
+  for (int i = tid; i < 4 * H; i += NTHR) s_bias[i] = a.bdense[i];
+  for (int i = tid; i < H; i += NTHR) s_bias[4 * H + i] = ws[so.sigma_w + i];
+  const float inv_v = 1.0f / (float)V;
+  // this wave's rows of each packed layer
+  const size_t lh_bytes = (size_t)H * H * sizeof(E);
+  const char* wf0 = reinterpret_cast<const char*>(a.wdense) + (size_t)wave * U0 * C::unit_bytes;
+  const char* wfh = reinterpret_cast<const char*>(a.wdense) + (size_t)H * K0 * sizeof(E) +
+                    (size_t)wave * UH * C::unit_bytes;
+  const char* wth = static_cast<const char*>(ba.wdense_t) + (size_t)wave * UH * C::unit_bytes;
+  asm volatile("" : "+s"(wf0), "+s"(wfh), "+s"(wth));  // see dense_chain
+  const int ch = half * 32 * H;   // this wave's columns of an activation buffer
+
+  float gsw[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) gsw[u] = 0.0f;
+  double gsb = 0.0;
+  DenseAcc16<F, H> dacc;
+  dacc.zero();
+  typename C::V abuf[NB][1];
+#pragma unroll
+  for (int j = 0; j < PD; ++j) load_a16<H, PREC, 1>(wf0, j, 16 * lane, abuf[(O0 + j) % NB]);
+
+  // lane, as a value the compiler cannot follow: the LDS addresses of a phase
+  // would else be kept in registers over the whole loop (200 spilled)
+  auto fresh_lane = [&] {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+
+  const long long item_end = std::min<long long>(ba.item_end, (long long)*a.n_valid);
+  long long item = ba.item_begin + blockIdx.x;
+  long long ray = item < item_end ? a.list[item] : 0;
+  float tv = 0.0f, oc = 0.0f;
+  if (item < item_end && tid < S) {
+    tv = a.t[ray * S + tid];
+    oc = ba.occ[ray * S + tid];
+  }
+  for (; item < item_end; item += gridDim.x) {
+    __syncthreads();
+    const int b = (int)(ray / a.rays_per_batch);
+    const float* rr = a.rays + ray * 6;
+    const BoxMap box(a.bbox + b * 6);
+    if (tid < S) {
+      s_pos[4 * tid + 0] = rr[0] + tv * rr[3];
+      s_pos[4 * tid + 1] = rr[1] + tv * rr[4];
+      s_pos[4 * tid + 2] = rr[2] + tv * rr[5];
+      s_alpha[tid] = oc;
+    }
+    __syncthreads();
+    // the next ray's samples, on the way while this one is worked on
+    if (item + gridDim.x < item_end) {
+      ray = a.list[item + gridDim.x];
+      if (tid < S) {
+        tv = a.t[ray * S + tid];
+        oc = ba.occ[ray * S + tid];
+      }
+    }
+    ray_features<F, PREC, NTHR>(a, b, ba.dtok + item * kVP * F, s_pos, S, tid, keep, s_g);
+    __syncthreads();
+    for (int c0 = 0; c0 < S; c0 += NS) {
+      // the replay of the compositing (wave 0) beside the first chunk's input
+      const int first = c0 == 0 ? 64 : 0;
+      if (wid == 0 && c0 == 0)
+        composite_backward(s_alpha, s_g, S, a.t_thres, lane, s_dz, gsb);
+      else
+        build_input<F, H, PREC, NS>(keep, s_pos, box, c0, tid - first, NTHR - first, x0);
+      __syncthreads();
+      f32x16 acc[1][1];
+      int ln = fresh_lane();
+      // forward, keeping every layer's output
+      chain_layer16<H, PREC, K0, O0>(wf0, wfh, 16 * ln, x0 + ch, s_bias, wave, ln, abuf, acc);
+      write_act16<H, PREC, 1>(h0 + ch, wave, ln, acc);
+      __syncthreads();
+      ln = fresh_lane();
+      chain_layer16<H, PREC, H, 0>(wfh, wfh + lh_bytes, 16 * ln, h0 + ch, s_bias + H, wave,
+                                   ln, abuf, acc);
+      write_act16<H, PREC, 1>(h1 + ch, wave, ln, acc);
+      __syncthreads();
+      ln = fresh_lane();
+      chain_layer16<H, PREC, H, 0>(wfh + lh_bytes, wfh + 2 * lh_bytes, 16 * ln, h1 + ch,
+                                   s_bias + 2 * H, wave, ln, abuf, acc);
+      write_act16<H, PREC, 1>(h2 + ch, wave, ln, acc);
+      __syncthreads();
+      ln = fresh_lane();
+      chain_layer16<H, PREC, H, 0>(wfh + 2 * lh_bytes, wth, 16 * ln, h2 + ch, s_bias + 3 * H,
+                                   wave, ln, abuf, acc);
+      // delta_3 = dz / V sigma_w [pre_3 > 0] (real views); sigma_w gradient
+      {
+        const int col = 32 * half + (ln & 31);
+        const float dzc = (col & 3) < V ? s_dz[c0 + (col >> 2)] * inv_v : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          const f32x4 sw = *reinterpret_cast<const f32x4*>(
+              s_bias + 4 * H + unit_of32<H>(wave, 0, ln >> 5, r));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float pre = acc[0][0][r + i];
+            gsw[r + i] += dzc * fmaxf(pre, 0.0f);
+            acc[0][0][r + i] = pre > 0.0f ? dzc * sw[i] : 0.0f;
+          }
+        }
+      }
+      write_vals16<H, PREC, 1>(da + ch, acc, nullptr, wave, ln);
+      __syncthreads();
+      ln = fresh_lane();
+      // delta_{2-l} = W_{3-l}^T delta [h_{2-l} > 0], and the weight gradients
+      accum_dw16<H, PREC, NC, H>(da, h2, dacc.w3, dacc.b[3], wave, half, ln);
+      chain_layer16<H, PREC, H, 0>(wth, wth + lh_bytes, 16 * ln, da + ch, nullptr, wave, ln,
+                                   abuf, acc);
+      write_vals16<H, PREC, 1>(db + ch, acc, h2 + ch, wave, ln);
+      __syncthreads();
+      ln = fresh_lane();
+      accum_dw16<H, PREC, NC, H>(db, h1, dacc.w2, dacc.b[2], wave, half, ln);
+      chain_layer16<H, PREC, H, 0>(wth + lh_bytes, wth + 2 * lh_bytes, 16 * ln, db + ch,
+                                   nullptr, wave, ln, abuf, acc);
+      write_vals16<H, PREC, 1>(da + ch, acc, h1 + ch, wave, ln);
+      __syncthreads();
+      ln = fresh_lane();
+      accum_dw16<H, PREC, NC, H>(da, h0, dacc.w1, dacc.b[1], wave, half, ln);
+      chain_layer16<H, PREC, H, 0>(wth + 2 * lh_bytes, wf0, 16 * ln, da + ch, nullptr, wave,
+                                   ln, abuf, acc);
+      write_vals16<H, PREC, 1>(db + ch, acc, h0 + ch, wave, ln);
+      {   // the next chunk's first weights, into layer 0's buffers
+        typename C::V head[PD];
+#pragma unroll
+        for (int j = 0; j < PD; ++j) head[j] = abuf[j][0];
+#pragma unroll
+        for (int j = 0; j < PD; ++j) abuf[(O0 + j) % NB][0] = head[j];
+      }
+      __syncthreads();
+      ln = fresh_lane();
+      accum_dw16<H, PREC, NC, K0>(db, x0, dacc.w0, dacc.b[0], wave, half, ln);
+      __syncthreads();
+    }
+  }
+  // occupancy-head gradient partials of this workgroup: the two column halves
+  float* gp = ba.gpart + (size_t)blockIdx.x * so.total;
+  float* s_sum = reinterpret_cast<float*>(smem);
+  __syncthreads();
+  const int u0 = unit_of32<H>(wave, 0, lane >> 5, 0);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) gsw[k] += __shfl_xor(gsw[k], off, 64);
+    if (half == 1 && (lane & 31) == 0) s_sum[u0 + k] = gsw[k];
+  }
+  __syncthreads();
+  if (half == 0 && (lane & 31) == 0) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) gp[so.sigma_w + u0 + k] += gsw[k] + s_sum[u0 + k];
+  }
+  if (tid == 0) gp[so.sigma_b] += (float)gsb;
+  dacc.store(ba.gdense + (size_t)blockIdx.x * dense_grad_total(F, H), wave, half, lane);
 }
 
 // ---- Backward of the Hydra encoder + RGB head ------------------------------
@@ -3584,25 +3836,30 @@ int sample_backward_launch_ns(BackArgs& ba, int parts, float* grad_small, float*
                               hipStream_t st) {
   constexpr SmallOffsets so = small_offsets(F, H);
   typedef SmemB<F, H, PREC, NS, SMAX> L;
-  static_assert(L::total <= kLdsBytes, "backward LDS");
+  constexpr bool W8 = DW && PREC != kF32;   // the 8-wave form, with a second delta buffer
+  constexpr size_t lds = L::total + (W8 ? L::buf : 0);
+  constexpr int threads = W8 ? kBackWaves * 64 : kThreads;
+  static_assert(lds <= kLdsBytes, "backward LDS");
   SAILOR_REQUIRE(ba.r.S % NS == 0 && ba.r.S <= SMAX,
                  "render_sample_backward: S=%d must be a multiple of %d and at most %d",
                  ba.r.S, NS, SMAX);
-  auto kern = render_backward_kernel<F, H, PREC, NS, DW, SMAX>;
+  void (*kern)(BackArgs);
+  if constexpr (W8) kern = render_backward16_kernel<F, H, PREC, NS, SMAX>;
+  else kern = render_backward_kernel<F, H, PREC, NS, DW, SMAX>;
   static std::atomic<bool> init[sailor::kMaxDevices];   // LDS limit set, per device
   int dev = 0;
   if (int e = sailor::device_slot(&dev)) return e;
   if (!init[dev].load(std::memory_order_acquire)) {
     SAILOR_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)L::total));
+                                       (int)lds));
     init[dev].store(true, std::memory_order_release);
   }
   const long long nz = (long long)parts * so.total;
   hipLaunchKernelGGL(fill_zero, dim3((unsigned)std::min<long long>((nz + 255) / 256, 4096)),
                      dim3(256), 0, st, ba.gpart, nz);
   if (int err = sailor::check_launch("render_sample_backward (zero)")) return err;
-  hipLaunchKernelGGL(kern, dim3(parts), dim3(kThreads), L::total, st, ba);
+  hipLaunchKernelGGL(kern, dim3(parts), dim3(threads), lds, st, ba);
   if (int err = sailor::check_launch("render_sample_backward")) return err;
   launch_sum_partials(ba.gpart, parts, so.total, grad_small, 1, st);
   if (int err = sailor::check_launch("render_sample_backward (sum)")) return err;
@@ -3616,9 +3873,8 @@ int sample_backward_launch_ns(BackArgs& ba, int parts, float* grad_small, float*
 
 // Samples per chunk: fp32 with in-kernel weight gradients 8 (measured 9 %
 // faster per C4 step than 4 despite ~50 spilled registers), fp32 column
-// form 4; 16-bit with in-kernel weight gradients 16 (24 would cut the chunk
-// phases by a third but spills ~120 registers per lane beside the
-// weight-gradient accumulators and runs slower); 16-bit column form 8.
+// form 4; 16-bit with in-kernel weight gradients 16 (64 columns: 32 for each of
+// the two waves of a unit range); 16-bit column form 8.
 template <int F, int H, int PREC, bool DW>
 int sample_backward_launch(BackArgs& ba, int parts, float* grad_small, float* grad_dense,
                            hipStream_t st) {

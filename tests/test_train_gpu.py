@@ -264,6 +264,48 @@ def test_fused_weight_gradients_match_column_form(prec):
     assert not bad, bad
 
 
+@pytest.mark.parametrize("prec", ["bf16", "fp16"])
+@pytest.mark.parametrize("S,V,n", [(16, 4, 1), (32, 1, 37), (48, 3, 300), (64, 2, 515)])
+def test_fused_16bit_gradients_over_samples_views_and_rays(prec, S, V, n):
+    """The fused form's weight gradients vs float64 products D^T A of the
+    column form's matrices at the ends of the 16-bit range: one to four
+    16-sample chunks, masked view slots, fewer and more rays than workgroups.
+    bf16: both hold the same 16-bit values, so only the float32 summation
+    differs (the bound of the comparison above).  fp16: one of the two rounds
+    dL/dz w straight to 16 bits (a mixed-precision product), the other by way of
+    float32, which differs by an ulp (2^-10) in one element of 2^13: 1e-5 of a
+    delta's norm.  That turns the rounding (2^-11) of 1e-5 / 2^-11 = 2 % of the
+    next deltas, 7e-5 of their norm at most: bound 1e-4."""
+    from sailor_amd.model import NerfWeights
+    from sailor_amd.train import RenderTrainer
+    p = pipe()
+    w = NerfWeights.init(p.mc.F, p.mc.H, perturb_std=0.01)
+    w.dense_b = [np.random.default_rng(40 + l).normal(0, 0.01, p.mc.H).astype(np.float32)
+                 for l in range(4)]
+    tr = RenderTrainer(w, prec, "cuda", batch_items=4096)
+    sel = torch.nonzero(p.sorted[0, :, 0] >= 0).flatten()[:n]
+    near = p.sorted[:, sel, :1]
+    far = p.sorted[:, sel].max(dim=2, keepdim=True).values
+    t = (near + (far - near) * torch.linspace(0, 1, S, device="cuda")).contiguous()
+    t[:, 1::5] = -1.0   # rays without samples between the others
+    tr.forward(t, p.rays[:, sel].contiguous(), p.K[:, :V].contiguous(),
+               p.RT[:, :V].contiguous(), (p.cfg.img, p.cfg.img), p.fmap[:, :V].contiguous(),
+               p.bbox, p.zdir)
+    g = torch.from_numpy(np.random.default_rng(3).normal(size=(1, sel.numel(), 3))
+                         .astype(np.float32)).cuda()
+    gr = tr.backward(g)
+    fused = [x.double().cpu().numpy() for k in ("dense_w", "dense_b") for x in gr[k]]
+    tr.backward(g, keep_columns=True)
+    A, D = ([m.double().cpu().numpy() for m in ms] for ms in tr.columns)
+    from sailor_amd.train import natural_first_layer_grad
+    want = [d.T @ x for d, x in zip(D, A)]
+    want[0] = natural_first_layer_grad(torch.from_numpy(want[0]), p.mc.F).numpy()
+    want += [d.sum(0) for d in D]
+    for i, (a, b) in enumerate(zip(fused, want)):
+        assert np.isfinite(a).all() and np.abs(b).max() > 0
+        assert np.linalg.norm(a - b) <= (1e-5 if prec == "bf16" else 1e-4) * np.linalg.norm(b), i
+
+
 def test_fused_gradients_match_central_differences():
     """Fused fp32 gradients of L = sum(g . rgb) vs central finite differences
     of the float64 restatement on 12 random parameters: dense weights and
