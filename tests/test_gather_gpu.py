@@ -67,6 +67,26 @@ def test_sample_features_match_float64(B):
     assert (geo > 0).float().mean() > 0.2 and (geo == 0).any()
 
 
+@pytest.mark.parametrize("V,R,S", [(1, 1, 1), (3, 13, 5), (8, 64, 1), (2, 127, 33)])
+def test_sample_features_at_wave_remainders(V, R, S):
+    """Fewer pairs than a wave's 64, one more than a wave, exactly one, and
+    odd sample counts.  Bound: the float32 projection places a tap within 8
+    roundings of a coordinate up to 128 pixels, 6e-5 pixels, times a slope of
+    at most 8 per pixel of an N(0, 1) map: 5e-4 (tpsdf: divided by 0.01 m)."""
+    from sailor_amd.fastnerf import sample_features
+    rays, dists, K, RT, maps, mid, dist = _case(V=V, R=R, S=S, seed=V)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    got = sample_features(cu(rays), cu(dists), cu(K), cu(RT), _cl(maps["geo"]),
+                          cu(maps["dep"][:, :, 0]), _cl(maps["rgbf"]), _cl(maps["rgb"]), cu(mid),
+                          cu(dist), res=512)
+    torch.cuda.synchronize()
+    ref = gr.sample_features(rays, dists, K, RT, maps["geo"], maps["dep"], maps["rgbf"],
+                             maps["rgb"], mid, dist, res=512)
+    for name, g in zip(("z", "tpsdf", "geo", "rgbf", "rgb", "dir"), got):
+        np.testing.assert_allclose(g.double().cpu().numpy(), ref[name].numpy(),
+                                   atol=5e-3 if name == "tpsdf" else 5e-4, err_msg=name)
+
+
 def test_forward_nerf_chain_matches_float64():
     from sailor_amd.fastnerf import forward_nerf
     rays, dists, K, RT, maps, mid, dist = _case(B=1, R=40, S=8, seed=4)
