@@ -81,7 +81,7 @@ def forward_nerf(ray_ori, ray_dir, sorted_dists, ks, rts, geo_cl, depths, rgbf_c
     o_c = torch.zeros((1, R, 3), dtype=_f32, device=dev)
     o_d = torch.zeros((1, R, 1), dtype=_f32, device=dev)
     o_f = torch.zeros((1, R, 30), dtype=_f32, device=dev)
-    valid = torch.where(torch.prod(sorted_dists != -1, dim=-1)[0])[0]
+    valid = torch.where((sorted_dists != -1).all(dim=-1)[0])[0]
     if valid.numel() == 0:
         return o_c, o_d, o_f
     rays = torch.cat([ray_ori[:, valid], ray_dir[:, valid]], -1)
