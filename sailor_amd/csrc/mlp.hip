@@ -2205,7 +2205,7 @@ render_backward_kernel(BackArgs ba) {
 // waves, two per SIMD, where wave w + 4 half owns output units 32 w .. + 31 of
 // the chunk's column half `half` in every layer, and K half `half` of those
 // units' weight gradients (128 of its 256 registers).  A chunk's 13 dependent
-// phases bound it, not its MFMAs (5.4k of about 17k cycles a chunk and SIMD):
+// phases bound it, not its MFMAs (5.4k of about 20k cycles a chunk and SIMD):
 // two waves per SIMD overlap them, each layer's first weights are loaded during
 // the phase before, the deltas alternate between two buffers (9 barriers a
 // chunk), the replay of the compositing runs beside the first chunk's input and
