@@ -369,3 +369,41 @@ def test_get_nodes_records():
             assert nodes[k].father_gindex == nd.gindex and nodes[k].size == 1
         if nd.father_gindex < 0:
             assert nd.size == rate and nd.depth == 3
+
+
+@pytest.mark.parametrize("n,S,n_max", [(1, 1, 128), (7, 5, 129), (77, 33, 131), (1001, 48, 1024)])
+def test_walks_at_group_remainders(n, S, n_max):
+    """Traversal and sampling where rays do not fill a wave's 8 groups of 8
+    lanes, rows are not aligned to them and samples end within one: bit for bit
+    the oracle's."""
+    from sailor_amd import VoxelEncoding as VE
+    HW, fx, dim, rate, tHW, tfx, _ = CASES["small_r4"]
+    inp = scene_inputs(0, 4, HW, HW, fx)
+    o = orc.integrate(inp["K"], inp["RT"], inp["R"], inp["T"], inp["colors"], inp["depths"],
+                      (dim, dim, dim), fixed_bbox=None)
+    oc, ocnt = orc.merge(o["occ"], rate)
+    n0, n1 = int(o["num_occ"].sum()), int(ocnt.sum())
+    tr = orc.tree_build(o["occ"], oc, o["voxel_size"], o["vol_bbox"], n0, n0 + n1)
+    tree = VE.MultiLayerOctree(2, 1, rate, 0)
+    tree.init_octree([_t(o["occ"]), _t(oc)], [n0, n1],
+                     [_t(o["num_occ"].astype(np.int32).reshape(1, 1)),
+                      _t(ocnt.astype(np.int32).reshape(1, 1))], [0, n0],
+                     _t(o["voxel_size"].reshape(1, 1)), _t(o["vol_bbox"]))
+    tree.build_octree()
+    r6 = orc.rays(*target_rays_np(tHW, tHW, tfx), tHW, tHW)[0, 0].reshape(1, -1, 6)
+    pick = np.linspace(0.2 * r6.shape[1], 0.8 * r6.shape[1], n).astype(int)   # the middle rows
+    ori, dirs = (np.ascontiguousarray(r6[:, pick, k:k + 3]) for k in (0, 3))
+    want = orc.traverse(tr["vol_coarse"], tr["node_pos"], tr["node_info"], o["vol_bbox"],
+                        o["voxel_size"], dim, rate, ori, dirs, n_max)
+    idx, tmin, tmax, vl = tree.voxel_traversal(_t(ori), _t(dirs), n_max, 0, -1, False, -1)
+    for name, got in (("idx", idx), ("tmin", tmin), ("tmax", tmax)):
+        np.testing.assert_array_equal(got.cpu().numpy(), want[name], err_msg=name)
+    np.testing.assert_array_equal(vl.cpu().numpy().reshape(1, -1), want["valid_len"])
+    if n > 7:
+        assert (want["idx"] >= 0).any()
+    noise = np.random.default_rng(n).random((1, n, S)).astype(np.float32)
+    sidx, st = tree.ray_voxels_points_sampling_coarse(idx, tmin, tmax, _t(noise), vl, 0, S)
+    ws = orc.sampling(want["idx"], want["tmin"], want["tmax"], noise, want["valid_len"],
+                      tr["node_pos"], o["voxel_size"], S, rate, want["gmax"])
+    np.testing.assert_array_equal(sidx.cpu().numpy(), ws[0])
+    np.testing.assert_array_equal(st.cpu().numpy(), ws[1])
