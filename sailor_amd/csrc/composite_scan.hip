@@ -19,23 +19,24 @@
 //   density:   dL/dsigma_k = delta_k [ exp(-e_k) (G_k T_k + g_a w_k) - S_k ]
 //   occupancy: dL/dalpha_k = G_k T_k + g_a w_k - S_k / (1 - alpha_k + 1e-6)
 //   dL/df_k = w_k g_f.
-// The backward's first walk parks T_k in the gradient row it later
-// overwrites, so the reverse walk needs no division by transmittances.
 //
-// Work split: a segment of 8, 16, 32 or 64 lanes (the power of two that holds
-// the row, rows over 64 in pieces) owns a ray, a lane a sample, so rows are
-// read and written whole lines at a time; transmittances are a product (sum)
-// scan over the segment and the suffix sums a scan from its end.  Feature rows
+// Work split: a segment of 16, 32 or 64 lanes (backward: 8 too; the power of two
+// that holds the row, rows over 64 in pieces) owns a ray, a lane a sample, so
+// rows are read and written whole lines at a time; transmittances are a product
+// (sum) scan over the segment and the suffix sums a scan from its end (of a row
+// in pieces the backward keeps the state before each piece in the gradient row
+// that it overwrites later).  Feature rows
 // are walked flat, 16 bytes a lane where F % 4 == 0.  What bounds it is HBM:
 // 65,536 rays x 48 x 16 channels move 0.23 GB forward and 0.43 GB backward.
 // One lane per ray, each load of a wave in 64 different lines, took 127.5 and
-// 462.6 us there; this form takes 52.0 and 87.3 us (4.3 and 4.9 TB/s).
+// 462.6 us there; this form takes 52.0 and 87.3 us (4.3 and 4.9 TB/s).  Short
+// rows take a lane per ray (lane_forward_pays).
 //
 // With `compensated` the forward keeps Kahan-compensated running sums (the
 // density form's exponent prefix sum and the four output sums), one lane per
-// ray in sample order; channels are processed in groups of up to FG per lane
-// (grid.y = channel groups), each lane re-running the cheap scalar recurrence
-// of its ray.
+// ray in sample order.  The lane forms' channels are processed in groups of up
+// to FG per lane (grid.y = channel groups), each lane re-running the cheap
+// scalar recurrence of its ray.
 #include "common.h"
 
 namespace {
@@ -43,26 +44,30 @@ namespace {
 constexpr int kThreads = 128;
 constexpr float kOccEps = 1e-6f;
 
-struct Kahan {
+template <bool COMP>
+struct Sum {
   float s = 0.0f, c = 0.0f;
   __device__ __forceinline__ void add(float x) {
+    if constexpr (!COMP) {
+      s += x;
+      return;
+    }
     const float y = x - c;
     const float t = s + y;
     c = (t - s) - y;
     s = t;
   }
-  // the compensated value of the sum (c holds the negated lost low bits)
+  // the value of the sum (c holds the negated lost low bits)
   __device__ __forceinline__ float value() const { return s - c; }
 };
 
-template <int FG>
+template <int FG, bool COMP>
 __global__ void __launch_bounds__(kThreads)
-scan_forward_compensated(const float* __restrict__ t, const float* __restrict__ sigma,
-                         const float* __restrict__ feats,
-                         const unsigned char* __restrict__ valid, long long n_rays, int S,
-                         int F, int occ_mode, float* __restrict__ out_feats,
-                         float* __restrict__ out_depth, float* __restrict__ out_ws,
-                         float* __restrict__ out_alpha) {
+lane_forward(const float* __restrict__ t, const float* __restrict__ sigma,
+             const float* __restrict__ feats, const unsigned char* __restrict__ valid,
+             long long n_rays, int S, int F, int occ_mode, float* __restrict__ out_feats,
+             float* __restrict__ out_depth, float* __restrict__ out_ws,
+             float* __restrict__ out_alpha) {
   const long long ray = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (ray >= n_rays) return;
   const int f0 = blockIdx.y * FG;
@@ -70,10 +75,9 @@ scan_forward_compensated(const float* __restrict__ t, const float* __restrict__ 
   const float* tr = t + ray * S;
   const float* sr = sigma + ray * S;
   const float* fr = feats + ray * (long long)S * F + f0;
-  Kahan acc[FG], dep, ws, al, pre;
-  float Tprod = 1.0f;
-  const bool live = valid == nullptr || valid[ray] != 0;
-  if (live) {
+  Sum<COMP> acc[FG], dep, ws, al, pre;
+  if (valid == nullptr || valid[ray] != 0) {
+    float Tprod = 1.0f;
     for (int i = 0; i < S; ++i) {
       const float z = tr[i];
       float alpha, T;
@@ -99,14 +103,88 @@ scan_forward_compensated(const float* __restrict__ t, const float* __restrict__ 
       }
     }
   }
-  float* of = out_feats + ray * F + f0;
 #pragma unroll
   for (int j = 0; j < FG; ++j)
-    if (j < nf) of[j] = acc[j].value();
+    if (j < nf) out_feats[ray * F + f0 + j] = acc[j].value();
   if (f0 == 0) {
     out_depth[ray] = dep.value();
     out_ws[ray] = ws.value();
     out_alpha[ray] = al.value();
+  }
+}
+
+// All channels in one lane: G_i needs the full dot product g_f . f_i.  The
+// first walk parks T_k in the gradient row that the second overwrites.
+template <int FMAX>
+__global__ void __launch_bounds__(kThreads)
+lane_backward(const float* __restrict__ g_feats, const float* __restrict__ g_depth,
+              const float* __restrict__ g_ws, const float* __restrict__ g_alpha,
+              const float* __restrict__ t, const float* __restrict__ sigma,
+              const float* __restrict__ feats, const unsigned char* __restrict__ valid,
+              long long n_rays, int S, int F, int occ_mode, float* __restrict__ grad_sigma,
+              float* __restrict__ grad_feats) {
+  const long long ray = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (ray >= n_rays) return;
+  const float* tr = t + ray * S;
+  const float* sr = sigma + ray * S;
+  const float* fr = feats + ray * (long long)S * F;
+  float* gs = grad_sigma + ray * S;
+  float* gf = grad_feats + ray * (long long)S * F;
+  if (valid != nullptr && valid[ray] == 0) {
+    for (int i = 0; i < S; ++i) gs[i] = 0.0f;
+    for (int i = 0; i < S * F; ++i) gf[i] = 0.0f;
+    return;
+  }
+  float gF[FMAX];
+#pragma unroll
+  for (int j = 0; j < FMAX; ++j) gF[j] = j < F ? g_feats[ray * F + j] : 0.0f;
+  const float gD = g_depth[ray], gW = g_ws[ray], gA = g_alpha[ray];
+  float pre = 0.0f, Tprod = 1.0f;
+  for (int i = 0; i < S; ++i) {
+    float alpha, T;
+    if (occ_mode) {
+      alpha = sr[i];
+      T = Tprod;
+      Tprod *= 1.0f - alpha + kOccEps;
+    } else {
+      const float delta = i + 1 < S ? tr[i + 1] - tr[i] : 0.0f;
+      const float e = delta * sr[i];
+      T = expf(-pre);
+      alpha = 1.0f - expf(-e);
+      pre += e;
+    }
+    const float w = alpha * T;
+    gs[i] = T;
+#pragma unroll
+    for (int j = 0; j < FMAX; ++j)
+      if (j < F) gf[(size_t)i * F + j] = w * gF[j];
+  }
+  float suffix = 0.0f;   // last sample first
+  for (int i = S - 1; i >= 0; --i) {
+    const float T = gs[i];
+    const float z = tr[i];
+    float G = gD * z + gW;
+#pragma unroll
+    for (int j = 0; j < FMAX; ++j)
+      if (j < F) G += gF[j] * fr[(size_t)i * F + j];
+    float grad;
+    float w;
+    if (occ_mode) {
+      const float alpha = sr[i];
+      w = alpha * T;
+      G += gA * alpha;
+      grad = G * T + gA * w - suffix / (1.0f - alpha + kOccEps);
+    } else {
+      const float delta = i + 1 < S ? tr[i + 1] - z : 0.0f;
+      const float e = delta * sr[i];
+      const float keep = expf(-e);
+      const float alpha = 1.0f - keep;
+      w = alpha * T;
+      G += gA * alpha;
+      grad = delta * (keep * (G * T + gA * w) - suffix);
+    }
+    gs[i] = grad;
+    suffix += G * w;
   }
 }
 
@@ -380,6 +458,24 @@ scan_backward(const float* __restrict__ g_feats, const float* __restrict__ g_dep
 // lanes of a ray's segment
 int seg_of(int S) { return S <= 8 ? 8 : S <= 16 ? 16 : S <= 32 ? 32 : 64; }
 
+// Calls a lane per ray is faster for: a segment spends most of a short row on
+// its reduction and leaves lanes idle, while a lane per ray waits for its
+// samples one after another (so rays have to be many for it) and loses its rows
+// from the caches once they are much larger than those.  Forward, lane and
+// segment, occupancies, us: 1,048,576 rays of 4 x 4 (samples x channels) 63 and
+// 453, 65,536 of 8 x 8 14 and 33, of 16 x 8 27 and 35, of 16 x 16 41 and 31;
+// 262,144 of 8 x 8 81 and 115, of 16 x 4 138 and 122; 4,096 of 16 x 4 12 and
+// 8.5.  Backward: 524,288 of 1 x 4 6 and 47, of 4 x 4 53 and 70, of 6 x 4 124
+// and 88.
+bool lane_forward_pays(long long n_rays, int S, int F) {
+  const bool four = F % 4 == 0;   // 16 bytes a lane in the segments
+  const long long row = (long long)S * F;
+  if (S <= 8 && row <= (four ? 32 : 24)) return true;
+  return S <= std::min<long long>(20, 4 + n_rays / 3072) && row <= (four ? 128 : 80) &&
+         n_rays * row <= (four ? 1 << 24 : 1 << 23) && n_rays * S <= 3 << 20;
+}
+bool lane_backward_pays(int S, int F) { return S <= 4 && F <= 16 && S * F <= 20; }
+
 int check_args(long long n_rays, int S, int F) {
   SAILOR_REQUIRE(n_rays >= 0 && S >= 1 && F >= 1,
                  "volume_render_torch: need n_rays >= 0, S >= 1, F >= 1 (got %lld, %d, %d)",
@@ -402,9 +498,10 @@ extern "C" int sailor_volume_render_torch_forward(const float* t, const float* s
   hipStream_t st = sailor::as_stream(stream);
   constexpr int FG = 8;
   SAILOR_REQUIRE((F + FG - 1) / FG <= 65535, "volume_render_torch: F = %d too large", F);
-  if (compensated) {
-    hipLaunchKernelGGL(scan_forward_compensated<FG>,
-                       dim3(sailor::ceil_div(n_rays, kThreads), (F + FG - 1) / FG),
+  if (compensated || lane_forward_pays(n_rays, S, F)) {
+    auto kern = lane_forward<FG, false>;
+    if (compensated) kern = lane_forward<FG, true>;
+    hipLaunchKernelGGL(kern, dim3(sailor::ceil_div(n_rays, kThreads), (F + FG - 1) / FG),
                        dim3(kThreads), 0, st, t, sigma, feats, valid, n_rays, S, F, occ_mode,
                        out_feats, out_depth, out_ws, out_alpha);
     return sailor::check_launch("volume_render_torch_forward");
@@ -418,7 +515,7 @@ extern "C" int sailor_volume_render_torch_forward(const float* t, const float* s
                      dim3(kThreads), 0, st, t, sigma, feats, valid, n_rays, S, F, occ_mode,   \
                      out_feats, out_depth, out_ws, out_alpha)
   switch (seg_of(S)) {
-    case 8: if (vec) SAILOR_SCAN_FWD(8, 4); else SAILOR_SCAN_FWD(8, 1); break;
+    case 8:    // 8 rays' accumulators in a lane leave one wave per SIMD
     case 16: if (vec) SAILOR_SCAN_FWD(16, 4); else SAILOR_SCAN_FWD(16, 1); break;
     case 32: if (vec) SAILOR_SCAN_FWD(32, 4); else SAILOR_SCAN_FWD(32, 1); break;
     default: if (vec) SAILOR_SCAN_FWD(64, 4); else SAILOR_SCAN_FWD(64, 1);
@@ -437,6 +534,14 @@ extern "C" int sailor_volume_render_torch_backward(
   SAILOR_REQUIRE(F <= 64, "volume_render_torch_backward: at most 64 channels (got %d)", F);
   if (n_rays == 0) return SAILOR_OK;
   hipStream_t st = sailor::as_stream(stream);
+  if (lane_backward_pays(S, F)) {
+    auto kern = lane_backward<16>;
+    if (F <= 4) kern = lane_backward<4>;
+    hipLaunchKernelGGL(kern, dim3(sailor::ceil_div(n_rays, kThreads)), dim3(kThreads), 0, st,
+                       g_feats, g_depth, g_ws, g_alpha, t, sigma, feats, valid, n_rays, S, F,
+                       occ_mode, grad_sigma, grad_feats);
+    return sailor::check_launch("volume_render_torch_backward");
+  }
   const bool vec = F % 4 == 0 &&
                    (((uintptr_t)feats | (uintptr_t)g_feats | (uintptr_t)grad_feats) & 15) == 0;
 #define SAILOR_SCAN_BWD(SEG, VEC, FM)                                                         \

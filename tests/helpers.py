@@ -33,3 +33,25 @@ def max_abs(a, b):
     a = np.asarray(a, np.float64)
     b = np.asarray(b, np.float64)
     return float(np.max(np.abs(a - b))) if a.size else 0.0
+
+
+def graph_us(fn, inner=5):
+    """GPU time of one call of fn in microseconds: the best of five replays of
+    a graph of `inner` calls."""
+    import torch
+    fn()
+    torch.cuda.synchronize()
+    s, best = torch.cuda.Stream(), float("inf")
+    with torch.cuda.stream(s):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            for _ in range(inner):
+                fn()
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record(s)
+            g.replay()
+            b.record(s)
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / inner)
+    return best

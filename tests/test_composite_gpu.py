@@ -14,6 +14,7 @@ import pytest
 import torch
 
 from oracle import composite_ref as cr
+from tests.helpers import graph_us
 
 pytestmark = pytest.mark.gpu
 
@@ -170,3 +171,51 @@ def test_every_segment_shape_matches_float64(S, F, occ_mode):
         for o, r in ((gs, rs.numpy()[..., 0]), (gf, rf.numpy())):
             assert np.abs(o.cpu().numpy() - r).max() <= (S + F + 16) * 2.0 ** -24 * max(
                 1.0, np.abs(r).max()) * 4
+
+
+@pytest.mark.parametrize("S,F", [(1, 4), (4, 4), (8, 4)])
+def test_short_rows_keep_up_with_a_copy(S, F):
+    """Many short rows are composited in at most 14 times the time that a copy of
+    their inputs takes, both ways (measured: 1 to 8 times; a segment of 8 lanes per
+    ray took 25 to 100 times forward)."""
+    import sailor_amd.VoxelEncoding as VE
+    R = 1 << 20
+    g = torch.Generator(device="cuda").manual_seed(S)
+    t = torch.rand((1, R, S), generator=g, device="cuda").sort(-1)[0]
+    s = torch.rand((1, R, S), generator=g, device="cuda") * 0.3
+    f = torch.randn((1, R, S, F), generator=g, device="cuda")
+    grads = [torch.randn((1, R, n), generator=g, device="cuda") for n in (F, 1, 1, 1)]
+    copy = graph_us(lambda: f.clone()) * (1 + 2 / F) + 5.0
+    fwd = graph_us(lambda: VE.volume_render_torch_forward(t, s, f, None, True))
+    bwd = graph_us(lambda: VE.volume_render_torch_backward(*grads, t, s, f, None, True))
+    print(f"{S} x {F}: copy {copy:.1f}, forward {fwd:.1f}, backward {bwd:.1f} us")
+    assert fwd <= 14 * copy and bwd <= 14 * copy
+
+
+@pytest.mark.parametrize("R", [64, 5000, 70000])
+@pytest.mark.parametrize("S,F", [(1, 1), (2, 16), (3, 5), (4, 4), (4, 5), (5, 4), (8, 4), (8, 5),
+                                 (9, 3), (16, 8), (20, 4), (21, 4), (12, 7), (10, 13), (1, 20)])
+@pytest.mark.parametrize("occ_mode", [False, True])
+def test_both_sides_of_the_short_row_rule_match_float64(R, S, F, occ_mode):
+    """Rows and ray counts at the edges of the rule that gives a ray a lane or
+    a segment of lanes; bounds as in test_every_segment_shape_matches_float64."""
+    import sailor_amd.VoxelEncoding as VE
+    t, s, f, valid = _case(occ_mode, B=1, R=R, S=S, F=F, seed=R + 7 * S)
+    rng = np.random.default_rng(S * 100 + F)
+    grads = [rng.normal(0, 1, (1, R, n)).astype(np.float32) for n in (F, 1, 1, 1)]
+    s64 = torch.from_numpy(s).double().requires_grad_()
+    f64 = torch.from_numpy(f).double().requires_grad_()
+    ref = cr.render(torch.from_numpy(t).double(), s64, f64, occ_mode, torch.from_numpy(valid))
+    rs, rf = torch.autograd.grad(ref, [s64, f64], [torch.from_numpy(g).double() for g in grads])
+    cu = lambda a: torch.from_numpy(a).cuda()
+    vr = cu(valid).to(torch.uint8)
+    out = VE.volume_render_torch_forward(cu(t), cu(s[..., 0]), cu(f), vr, occ_mode)
+    for o, r in zip(out, ref):
+        r = r.detach().numpy()
+        assert np.abs(o.cpu().numpy() - r).max() <= (S + 8) * 2.0 ** -24 * max(
+            1.0, np.abs(r).max()) * 2
+    gs, gf = VE.volume_render_torch_backward(*[cu(g) for g in grads], cu(t), cu(s[..., 0]),
+                                             cu(f), vr, occ_mode)
+    for o, r in ((gs, rs.numpy()[..., 0]), (gf, rf.numpy())):
+        assert np.abs(o.cpu().numpy() - r).max() <= (S + F + 16) * 2.0 ** -24 * max(
+            1.0, np.abs(r).max()) * 4
