@@ -292,21 +292,22 @@ __device__ __forceinline__ void mfma_layer_r(const f16x8 (&w)[2][STEPS], const f
       acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[mt][s], bin[s], acc[mt], 0, 0, 0);
 }
 
-// Per wave and step 32 consecutive points as VS tiles of P = 32 / VS points:
-// each tile's columns are its (point, view) pairs through the feature layers;
-// after the view mean the VS lanes of a point hold the same values, so lane v
-// of each point keeps them for tile v, and the occupancy layers run once for
-// all 32 points.  The feature layers' fragments (112 registers) stay in
+// Per wave and step kt <= VS tiles of P = 32 / VS consecutive points, which may
+// belong to several batches: each tile's columns are its (point, view) pairs
+// through the feature layers; after the view mean the VS lanes of a point hold
+// the same values, so lane v of each point keeps them for tile v, and the
+// occupancy layers run once for all of the step's points.  The feature layers' fragments (112 registers) stay in
 // registers at two waves per SIMD, the others in LDS.
 // Bound by vector issue: per tile 28 + 3 + 16 / VS MFMAs and about as many
 // vector instruction cycles for bias, ReLU and rounding (65,536 rays x 48
 // samples x 4 views: 1264 us with the occupancy layers run per tile, view sums
 // through LDS shuffles and two v_max per ReLU; 722 us now).
-template <int VS>
+// FULL: one batch and kt == VS, known to the compiler.
+template <int VS, bool FULL>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
 density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__ z,
                     const float* __restrict__ tpsdf, const float* __restrict__ geo, int B,
-                    long long n_pts, int V, float* __restrict__ occ,
+                    long long n_pts, int V, int kt_arg, float* __restrict__ occ,
                     float* __restrict__ geo_out, int n_geo_out) {
   __shared__ DensityMfmaLds L;
   // ---- stage the permuted A fragments, biases and the small weights
@@ -333,7 +334,9 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
   constexpr int P = 32 / VS;
   const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
   const int v = n % VS, lp = n / VS;
-  const long long steps = (n_pts + 31) / 32;
+  const int kt = FULL ? VS : kt_arg;
+  const long long total = FULL ? n_pts : (long long)B * n_pts;
+  const long long steps = (total + kt * P - 1) / (kt * P);
   const long long wave0 = (long long)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   const long long n_waves = (long long)gridDim.x * (kBlock / 64);
   const float inv = 1.0f / (float)V;
@@ -350,114 +353,119 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
   }
   float inf = __builtin_inff();
   asm("" : "+s"(inf));   // kept from the compiler, which would make the median a maximum again
-  for (int b = blockIdx.y; b < B; b += gridDim.y) {
-    // this lane's share of a column's inputs x = [z, tpsdf, geo 0..15]: half 0
-    // holds x 0..7 and x 16..17, half 1 holds x 8..15 (its layer-0 B
-    // operand); the next tile's share is loaded before the current tile's
-    // MFMA chain runs
-    const long long col0 = ((long long)b * V + (v < V ? v : 0)) * n_pts;
-    auto load_share = [&](long long tile, float (&x)[10]) {
+  // points are numbered over all batches: point p of batch b is
+  // p + b (V - 1) n_pts of view 0's inputs and p of the outputs
+  const bool narrow = total <= 0xffffffffll;
+  auto batch_of = [&](long long p) -> long long {
+    if (FULL) return 0;
+    return narrow ? (long long)((unsigned)p / (unsigned)n_pts) : p / n_pts;
+  };
+  // this lane's share of a column's inputs x = [z, tpsdf, geo 0..15]: half 0
+  // holds x 0..7 and x 16..17, half 1 holds x 8..15 (its layer-0 B
+  // operand); the next tile's share is loaded before the current tile's
+  // MFMA chain runs
+  auto load_share = [&](long long tile, float (&x)[10]) {
 #pragma unroll
-      for (int i = 0; i < 10; ++i) x[i] = 0.0f;
-      const long long p = tile * P + lp;
-      if (p < n_pts && v < V) {
-        const float* g = geo + (col0 + p) * 16;
-        const float4 a = *reinterpret_cast<const float4*>(g + (h ? 8 : 0));
-        const float2 c = *reinterpret_cast<const float2*>(g + (h ? 6 : 4));
-        const float2 d = *reinterpret_cast<const float2*>(g + (h ? 12 : 14));
-        float2 f = c;
-        if (h == 0) f = make_float2(z[col0 + p], tpsdf[col0 + p]);
-        x[0] = f.x; x[1] = f.y;
-        x[2] = a.x; x[3] = a.y; x[4] = a.z; x[5] = a.w;
-        x[6] = h ? d.x : c.x;
-        x[7] = h ? d.y : c.y;
-        x[8] = h ? 0.0f : d.x;
-        x[9] = h ? 0.0f : d.y;
-      }
-    };
-    float xc[10];
-    load_share(wave0 * VS, xc);
-    for (long long it = wave0; it < steps; it += n_waves) {
-      f16x8 comb[4] = {};
-      int zo;
-#pragma unroll 1
-      for (int k = 0; k < VS; ++k) {
-        const long long tile = it * VS + k;
-        float xn[10];
-        load_share(k + 1 < VS ? tile + 1 : (it + n_waves) * VS, xn);
-        const long long p = tile * P + lp;
-        const bool col_ok = p < n_pts && v < V;
-        f16x8 bin[4];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          bin[0][j] = (half_t)xc[j];
-          bin[1][j] = (half_t)(j < 2 ? xc[8 + j] : 0.0f);
-        }
-        // an opaque zero redefined every tile keeps the bias reads in the
-        // loop, so the registers go to the weight fragments
-        asm volatile("v_mov_b32 %0, 0" : "=v"(zo));
-        f32x16 acc[2];
-        // geometry features of the texture views: 18 -> 16 -> 8 on MFMA from
-        // the layer-0 operand; hidden unit 8 h + r sits in accumulator r < 8
-        // of half h, which is the next layer's B operand, and output r < 8
-        // lands in accumulator r of half 0.  The whole wave runs the MFMAs (an
-        // MFMA reads the A and B registers of every lane, so a lane-dependent
-        // branch around it would feed it stale rows); only the store is per
-        // lane.
-        if (geo_out) {
-          f32x16 g;
-          f16x8 gb[4];
-          mfma_layer1<2>(L, 6, bin, g, lane, 4 * zo);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) gb[0][j] = (half_t)g[j];
-          gb[0] = relu8(gb[0]);
-          mfma_layer1<1>(L, 7, gb, g, lane, 4 * zo);
-          if (h == 0 && col_ok && v < n_geo_out) {
-            float4* o4 = reinterpret_cast<float4*>(
-                geo_out + (((long long)b * n_geo_out + v) * n_pts + p) * 8);
-            o4[0] = make_float4(fmaxf(g[0], 0.f), fmaxf(g[1], 0.f), fmaxf(g[2], 0.f),
-                                fmaxf(g[3], 0.f));
-            o4[1] = make_float4(fmaxf(g[4], 0.f), fmaxf(g[5], 0.f), fmaxf(g[6], 0.f),
-                                fmaxf(g[7], 0.f));
-          }
-        }
-        mfma_layer_r<2>(w0, L.bias[0], bin, acc, lane, zo);
-#pragma unroll
-        for (int l = 0; l < 3; ++l) {
-          relu_to_b(acc, bin);
-          mfma_layer_r<4>(wf[l], L.bias[l + 1], bin, acc, lane, zo);
-        }
-        // mean of the ReLU outputs over the point's views (fp32): the median
-        // of x, 0 and the bound is the ReLU, and 0 in a column without a view
-        const float bound = col_ok ? inf : 0.0f;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          f16x8 m;
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            m[j] = (half_t)(view_sum<VS>(__builtin_amdgcn_fmed3f(acc[s / 2][8 * (s % 2) + j],
-                                                                 0.0f, bound)) * inv);
-          comb[s] = VS == 1 || v == k ? m : comb[s];
-        }
-#pragma unroll
-        for (int i = 0; i < 10; ++i) xc[i] = xn[i];
-      }
-      // occupancy layers: column n is point lp of tile v
-      f32x16 acc[2];
-      mfma_layer<4>(L, 4, comb, acc, lane, 4 * zo);
-      relu_to_b(acc, comb);
-      mfma_layer<4>(L, 5, comb, acc, lane, 4 * zo);
-      float part = 0.0f;
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          part += L.w_out[acc_unit(mt, r, h)] * __builtin_amdgcn_fmed3f(acc[mt][r], 0.0f, inf);
-      part += __shfl_xor(part, 32, 64);
-      const long long p = (it * VS + v) * P + lp;
-      if (h == 0 && p < n_pts)
-        occ[(long long)b * n_pts + p] = 1.0f / (1.0f + expf(-(part + L.b_out)));
+    for (int i = 0; i < 10; ++i) x[i] = 0.0f;
+    const long long p = tile * P + lp;
+    if (p < total && v < V) {
+      const long long e = p + (batch_of(p) * (V - 1) + v) * n_pts;
+      const float* g = geo + e * 16;
+      const float4 a = *reinterpret_cast<const float4*>(g + (h ? 8 : 0));
+      const float2 c = *reinterpret_cast<const float2*>(g + (h ? 6 : 4));
+      const float2 d = *reinterpret_cast<const float2*>(g + (h ? 12 : 14));
+      float2 f = c;
+      if (h == 0) f = make_float2(z[e], tpsdf[e]);
+      x[0] = f.x; x[1] = f.y;
+      x[2] = a.x; x[3] = a.y; x[4] = a.z; x[5] = a.w;
+      x[6] = h ? d.x : c.x;
+      x[7] = h ? d.y : c.y;
+      x[8] = h ? 0.0f : d.x;
+      x[9] = h ? 0.0f : d.y;
     }
+  };
+  float xc[10];
+  load_share(wave0 * kt, xc);
+  for (long long it = wave0; it < steps; it += n_waves) {
+    f16x8 comb[4] = {};
+    int zo;
+#pragma unroll 1
+    for (int k = 0; k < kt; ++k) {
+      const long long tile = it * kt + k;
+      float xn[10];
+      load_share(k + 1 < kt ? tile + 1 : (it + n_waves) * kt, xn);
+      const long long p = tile * P + lp;
+      const bool col_ok = p < total && v < V;
+      f16x8 bin[4];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        bin[0][j] = (half_t)xc[j];
+        bin[1][j] = (half_t)(j < 2 ? xc[8 + j] : 0.0f);
+      }
+      // an opaque zero redefined every tile keeps the bias reads in the
+      // loop, so the registers go to the weight fragments
+      asm volatile("v_mov_b32 %0, 0" : "=v"(zo));
+      f32x16 acc[2];
+      // geometry features of the texture views: 18 -> 16 -> 8 on MFMA from
+      // the layer-0 operand; hidden unit 8 h + r sits in accumulator r < 8
+      // of half h, which is the next layer's B operand, and output r < 8
+      // lands in accumulator r of half 0.  The whole wave runs the MFMAs (an
+      // MFMA reads the A and B registers of every lane, so a lane-dependent
+      // branch around it would feed it stale rows); only the store is per
+      // lane.
+      if (geo_out) {
+        f32x16 g;
+        f16x8 gb[4];
+        mfma_layer1<2>(L, 6, bin, g, lane, 4 * zo);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) gb[0][j] = (half_t)g[j];
+        gb[0] = relu8(gb[0]);
+        mfma_layer1<1>(L, 7, gb, g, lane, 4 * zo);
+        if (h == 0 && col_ok && v < n_geo_out) {
+          float4* o4 = reinterpret_cast<float4*>(
+              geo_out + (p + (batch_of(p) * (n_geo_out - 1) + v) * n_pts) * 8);
+          o4[0] = make_float4(fmaxf(g[0], 0.f), fmaxf(g[1], 0.f), fmaxf(g[2], 0.f),
+                              fmaxf(g[3], 0.f));
+          o4[1] = make_float4(fmaxf(g[4], 0.f), fmaxf(g[5], 0.f), fmaxf(g[6], 0.f),
+                              fmaxf(g[7], 0.f));
+        }
+      }
+      mfma_layer_r<2>(w0, L.bias[0], bin, acc, lane, zo);
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+        relu_to_b(acc, bin);
+        mfma_layer_r<4>(wf[l], L.bias[l + 1], bin, acc, lane, zo);
+      }
+      // mean of the ReLU outputs over the point's views (fp32): the median
+      // of x, 0 and the bound is the ReLU, and 0 in a column without a view
+      const float bound = col_ok ? inf : 0.0f;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        f16x8 m;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          m[j] = (half_t)(view_sum<VS>(__builtin_amdgcn_fmed3f(acc[s / 2][8 * (s % 2) + j],
+                                                               0.0f, bound)) * inv);
+        comb[s] = VS == 1 || v == k ? m : comb[s];
+      }
+#pragma unroll
+      for (int i = 0; i < 10; ++i) xc[i] = xn[i];
+    }
+    // occupancy layers: column n is point lp of tile v
+    f32x16 acc[2];
+    mfma_layer<4>(L, 4, comb, acc, lane, 4 * zo);
+    relu_to_b(acc, comb);
+    mfma_layer<4>(L, 5, comb, acc, lane, 4 * zo);
+    float part = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        part += L.w_out[acc_unit(mt, r, h)] * __builtin_amdgcn_fmed3f(acc[mt][r], 0.0f, inf);
+    part += __shfl_xor(part, 32, 64);
+    const long long p = (it * kt + v) * P + lp;
+    if (h == 0 && v < kt && p < total)
+      occ[p] = 1.0f / (1.0f + expf(-(part + L.b_out)));
   }
 }
 
@@ -1374,20 +1382,30 @@ int launch_density(bool mfma, const half_t* pd, const float* z, const float* tps
                    int n_geo_out, hipStream_t st) {
   if (mfma && V <= 8) {
     const int VS = V <= 1 ? 1 : V <= 2 ? 2 : V <= 4 ? 4 : 8;
-    const long long steps = (n_pts + 31) / 32;
+    const long long tiles = ((long long)B * n_pts + 32 / VS - 1) / (32 / VS);
     // persistent workgroups, 2 per CU (256 registers per lane, 50 KB of LDS):
     // the weights are staged once per workgroup
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    const long long slots = std::max<long long>(1, 2LL * cus / std::min(B, 2 * cus));
+    // tiles of a step: with 8 view slots fewer where they leave compute units
+    // without a workgroup (8 views of 1,000 points 64.5 us, 70 with 8 tiles; a
+    // step of 4 or fewer costs nothing to speak of beside the staging)
+    const long long waves = (long long)cus * (kBlock / 64);
+    const int kt = VS < 8 ? VS
+                          : (int)std::min<long long>(
+                                VS, std::max<long long>(1, (tiles + waves - 1) / waves));
+    const long long steps = (tiles + kt - 1) / kt;
     const dim3 grid((unsigned)std::max<long long>(
-                        1, std::min<long long>((steps + kBlock / 64 - 1) / (kBlock / 64), slots)),
-                    (unsigned)std::min(B, 65535));
-#define SAILOR_DENSITY_MFMA(N)                                                            \
-  hipLaunchKernelGGL(density_mfma_kernel<N>, grid, dim3(kBlock), 0, st, pd, z, tpsdf, \
-                     geo, B, n_pts, V, occ, geo_out, n_geo_out)
+        1, std::min<long long>((steps + kBlock / 64 - 1) / (kBlock / 64), 2LL * cus)));
+#define SAILOR_DENSITY_MFMA(N)                                                             \
+  do {                                                                                     \
+    auto kern = density_mfma_kernel<N, false>;                                             \
+    if (B == 1 && kt == N) kern = density_mfma_kernel<N, true>;                            \
+    hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, st, pd, z, tpsdf, geo, B, n_pts, V,     \
+                       kt, occ, geo_out, n_geo_out);                                       \
+  } while (0)
     if (VS == 1) SAILOR_DENSITY_MFMA(1);
     else if (VS == 2) SAILOR_DENSITY_MFMA(2);
     else if (VS == 4) SAILOR_DENSITY_MFMA(4);
