@@ -212,6 +212,7 @@ depth_tiles_kernel(const float* __restrict__ depths, int H, int W, int tiles_x, 
 // per pass.
 constexpr int kBx = 4, kBy = 4, kBz = 16;
 constexpr int kPassY = 64 / kBz;
+constexpr int kPasses = kBx * kBy / kPassY;
 static_assert(64 % kBz == 0 && kBy % kPassY == 0, "whole passes over the brick");
 
 struct Bricks {
@@ -318,19 +319,20 @@ observing_views_kernel(const float* __restrict__ vol_bbox, const float* __restri
   }
 }
 
-// One lane per voxel, a brick per wave; grid = (ceil(bricks / 4), B).  masks:
-// the views to evaluate for each brick (null: all of them).  Bound by vector
-// issue where views remain (the reference's IEEE divisions, 7 per view and
-// voxel) and by the 16 B written per voxel elsewhere: 256^3 voxels, 4 views of
-// 1024^2 around one performer 290 us without the masks, 93 us with them and
-// about 20 us to make them (0.27 GB written; bricks of 4 x 4 x 32 and 8^3
-// voxels -8 and +27 us, but at 128^3 the former costs 15 us more); masks made
-// by one wave of each 512-voxel workgroup before its voxels: 156 us.  COMP (precision form): the TSDF is
+// One lane per voxel; a brick per wave, or SPLIT = 4 waves per brick with a
+// pass each; grid = (ceil(bricks * SPLIT / 4), B).  masks: the views to evaluate
+// for each brick (null: all of them).  Bound by vector issue where views remain
+// (the reference's IEEE divisions, 7 per view and voxel) and by the 16 B written
+// per voxel elsewhere: 256^3 voxels, 4 views of 1024^2 around one performer
+// 290 us without the masks, 93 us with them and about 20 us to make them
+// (0.27 GB written; bricks of 4 x 4 x 32 and 8^3 voxels -8 and +27 us, but at
+// 128^3 the former costs 15 us more); masks made by one wave of each 512-voxel
+// workgroup before its voxels: 156 us.  COMP (precision form): the TSDF is
 // formed as the Kahan-compensated sum of obs_weight * dist over the observing
 // views divided once by the weight sum, instead of the reference's running
 // average (tsdf * w_old + obs_weight * dist) / w_new -- the same value in exact
 // arithmetic, with one rounding of the sum instead of one per view.
-template <bool COMP>
+template <bool COMP, int SPLIT>
 __global__ void __launch_bounds__(kThreads)
 integrate_kernel(float* __restrict__ tsdf_vol, float* __restrict__ weight_vol,
                  float* __restrict__ color_vol, int* __restrict__ occ_vol,
@@ -342,6 +344,8 @@ integrate_kernel(float* __restrict__ tsdf_vol, float* __restrict__ weight_vol,
                  const unsigned long long* __restrict__ masks, float obs_weight, int H,
                  int W, int V, int X, int Y, int Z, float trunc_weight,
                  float th_low, float th_high) {
+  static_assert(kPasses % SPLIT == 0, "whole passes per wave");
+  constexpr int passes = kPasses / SPLIT;
   __shared__ int s_cnt[kThreads / 64];
   const Bricks br(X, Y, Z);
   const int b = blockIdx.y;
@@ -351,15 +355,17 @@ integrate_kernel(float* __restrict__ tsdf_vol, float* __restrict__ weight_vol,
   const float trunc = vs * trunc_weight;
   const float* bb = vol_bbox + b * 6;
   int count = 0;
-  for (unsigned brick = blockIdx.x * (kThreads / 64) + wid; brick < br.n;
-       brick += gridDim.x * (kThreads / 64)) {
+  for (unsigned item = blockIdx.x * (kThreads / 64) + wid; item < br.n * SPLIT;
+       item += gridDim.x * (kThreads / 64)) {
+    const unsigned brick = item / SPLIT;
+    const int pass0 = (int)(item % SPLIT) * passes;
     int x0, y0, z0;
     br.corner(brick, x0, y0, z0);
     unsigned long long views = V < 64 ? (1ull << V) - 1 : ~0ull;
     if (masks) views = masks[(size_t)b * br.n + brick];
     const int vz = z0 + lane % kBz;
 #pragma unroll 1
-    for (int pass = 0; pass < kBx * kBy / kPassY; ++pass) {
+    for (int pass = pass0; pass < pass0 + passes; ++pass) {
       const int vx = x0 + pass / (kBy / kPassY);
       const int vy = y0 + pass % (kBy / kPassY) * kPassY + lane / kBz;
       bool occupied = false;
@@ -529,6 +535,25 @@ int launch_bbox(const float* depths, const float* K, const float* R,
   return sailor::check_launch("bbox_reduce");
 }
 
+// Masks pay for their two kernels and a pass over the depth maps (about 10 us
+// and the maps' bytes) where voxels x views are many: 4 views of 1024^2, with
+// and without masks 74 and 69 us at 128^3, 79 and 90 us at 160^3, 143 and
+// 229 us at 256^3; 8 of 512^2 82 and 80 us at 96^3, 87 and 91 us at 112^3; 1 of
+// 512^2 59 and 61 us at 192^3; 4 of 1024^2 at 32^3 99 and 42 us (whole call).
+bool use_masks(int V, int H, int W, int X, int Y, int Z) {
+  return (double)X * Y * Z * V > (double)(1 << 23) + (double)V * H * W;
+}
+// Waves per brick: a wave's 4 passes one after another take V projections each,
+// which a chip that is not full waits for; a full one gains from fewer, longer
+// waves.  1 and 4 waves: 4 views of 1024^2 55 and 42 us at 32^3, 83 and 69 us at
+// 128^3, 142 and 176 us at 256^3 (masks); 1 view of 64^2 14.7 and 12.9 us at
+// 32^3, 14.8 and 16.1 us at 48^3, 30 and 36 us at 160^3; 20 of 256^2 122 and
+// 81 us at 64^3, 425 and 481 us at 256^3.
+unsigned brick_split(long long bricks, int V) {
+  const long long few = V < 4 ? 256LL * V * V : std::min(4096LL * V, 32768LL);
+  return bricks < few ? 4 : 1;
+}
+
 }  // namespace
 
 // Workspace: a mask of views per brick, then the depth of each pixel tile.
@@ -572,7 +597,7 @@ int integrate_impl(bool comp, int32_t* occ_vol, int32_t* num_occ, const float* K
     SAILOR_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 7) == 0,
                    "integrate: workspace must be 8-byte aligned");
     // the tiles' launch takes a grid plane per view and a row per tile row
-    if ((long long)B * V <= 65535 && tiles_y <= 65535) {
+    if (use_masks(V, H, W, X, Y, Z) && (long long)B * V <= 65535 && tiles_y <= 65535) {
       masks = static_cast<unsigned long long*>(workspace);
       float* tiles = reinterpret_cast<float*>(masks + (size_t)B * n);
       hipLaunchKernelGGL(depth_tiles_kernel, dim3(sailor::ceil_div(tiles_x, 4), tiles_y, B * V),
@@ -586,12 +611,16 @@ int integrate_impl(bool comp, int32_t* occ_vol, int32_t* num_occ, const float* K
                          trunc_weight, masks);
     }
   }
-  dim3 grid = blocks(((long long)n + kThreads / 64 - 1) / (kThreads / 64));
+  const unsigned split = brick_split((long long)n * B, V);
+  dim3 grid = blocks(((long long)n * split + kThreads / 64 - 1) / (kThreads / 64));
   grid.y = B;
-  hipLaunchKernelGGL(comp ? integrate_kernel<true> : integrate_kernel<false>, grid,
-                     dim3(kThreads), 0, st, tsdf, weight, color, occ_vol, num_occ, vol_bbox, K,
-                     RT, colors, depths, voxel_size, masks, obs_weight, H, W, V, X, Y, Z,
-                     trunc_weight, tsdf_th_low, tsdf_th_high);
+  auto kern = integrate_kernel<false, 1>;
+  if (split == 1 && comp) kern = integrate_kernel<true, 1>;
+  if (split == 4) kern = integrate_kernel<false, 4>;
+  if (split == 4 && comp) kern = integrate_kernel<true, 4>;
+  hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, st, tsdf, weight, color, occ_vol, num_occ,
+                     vol_bbox, K, RT, colors, depths, voxel_size, masks, obs_weight, H, W, V, X,
+                     Y, Z, trunc_weight, tsdf_th_low, tsdf_th_high);
   return sailor::check_launch("integrate");
 }
 
