@@ -35,6 +35,16 @@ int device_slot(int* slot);
 
 inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
+// A launch holds fewer than 2^32 lanes: calls with up to 64 lanes per ray go in
+// parts of this many rays, run(first, rays) for each.
+constexpr long long kRaysPerLaunch = 1LL << 25;
+template <class Run>
+inline int in_parts(long long n_rays, Run run) {
+  for (long long first = 0; first < n_rays; first += kRaysPerLaunch)
+    if (int e = run(first, std::min(kRaysPerLaunch, n_rays - first))) return e;
+  return SAILOR_OK;
+}
+
 // Float -> int conversion with fully defined results for every input:
 // NaN -> 0, values at or beyond the int32 range saturate.  In-range values
 // truncate toward zero exactly like a C cast.  The CPU oracle uses the same

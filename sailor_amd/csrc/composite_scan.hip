@@ -483,22 +483,12 @@ int check_args(long long n_rays, int S, int F) {
   return SAILOR_OK;
 }
 
-}  // namespace
-
-extern "C" int sailor_volume_render_torch_forward(const float* t, const float* sigma,
-                                                  const float* feats,
-                                                  const unsigned char* valid, long long n_rays,
-                                                  int S, int F, int occ_mode, int compensated,
-                                                  float* out_feats, float* out_depth,
-                                                  float* out_ws, float* out_alpha,
-                                                  void* stream) {
-  int rc = check_args(n_rays, S, F);
-  if (rc) return rc;
-  if (n_rays == 0) return SAILOR_OK;
-  hipStream_t st = sailor::as_stream(stream);
-  constexpr int FG = 8;
-  SAILOR_REQUIRE((F + FG - 1) / FG <= 65535, "volume_render_torch: F = %d too large", F);
-  if (compensated || lane_forward_pays(n_rays, S, F)) {
+int launch_forward(bool lane, const float* t, const float* sigma, const float* feats,
+                   const unsigned char* valid, long long n_rays, int S, int F, int occ_mode,
+                   int compensated, float* out_feats, float* out_depth, float* out_ws,
+                   float* out_alpha, hipStream_t st) {
+  if (lane) {
+    constexpr int FG = 8;
     auto kern = lane_forward<FG, false>;
     if (compensated) kern = lane_forward<FG, true>;
     hipLaunchKernelGGL(kern, dim3(sailor::ceil_div(n_rays, kThreads), (F + FG - 1) / FG),
@@ -524,16 +514,10 @@ extern "C" int sailor_volume_render_torch_forward(const float* t, const float* s
   return sailor::check_launch("volume_render_torch_forward");
 }
 
-extern "C" int sailor_volume_render_torch_backward(
-    const float* g_feats, const float* g_depth, const float* g_ws, const float* g_alpha,
-    const float* t, const float* sigma, const float* feats, const unsigned char* valid,
-    long long n_rays, int S, int F, int occ_mode, float* grad_sigma, float* grad_feats,
-    void* stream) {
-  int rc = check_args(n_rays, S, F);
-  if (rc) return rc;
-  SAILOR_REQUIRE(F <= 64, "volume_render_torch_backward: at most 64 channels (got %d)", F);
-  if (n_rays == 0) return SAILOR_OK;
-  hipStream_t st = sailor::as_stream(stream);
+int launch_backward(const float* g_feats, const float* g_depth, const float* g_ws,
+                    const float* g_alpha, const float* t, const float* sigma, const float* feats,
+                    const unsigned char* valid, long long n_rays, int S, int F, int occ_mode,
+                    float* grad_sigma, float* grad_feats, hipStream_t st) {
   if (lane_backward_pays(S, F)) {
     auto kern = lane_backward<16>;
     if (F <= 4) kern = lane_backward<4>;
@@ -564,4 +548,41 @@ extern "C" int sailor_volume_render_torch_backward(
 #undef SAILOR_SCAN_BWD_F
 #undef SAILOR_SCAN_BWD
   return sailor::check_launch("volume_render_torch_backward");
+}
+
+}  // namespace
+
+extern "C" int sailor_volume_render_torch_forward(const float* t, const float* sigma,
+                                                  const float* feats,
+                                                  const unsigned char* valid, long long n_rays,
+                                                  int S, int F, int occ_mode, int compensated,
+                                                  float* out_feats, float* out_depth,
+                                                  float* out_ws, float* out_alpha,
+                                                  void* stream) {
+  int rc = check_args(n_rays, S, F);
+  if (rc) return rc;
+  SAILOR_REQUIRE((F + 7) / 8 <= 65535, "volume_render_torch: F = %d too large", F);
+  const bool lane = compensated || lane_forward_pays(n_rays, S, F);
+  return sailor::in_parts(n_rays, [&](long long r, long long n) {
+    return launch_forward(lane, t + r * S, sigma + r * S, feats + r * S * F,
+                          valid ? valid + r : nullptr, n, S, F, occ_mode, compensated,
+                          out_feats + r * F, out_depth + r, out_ws + r, out_alpha + r,
+                          sailor::as_stream(stream));
+  });
+}
+
+extern "C" int sailor_volume_render_torch_backward(
+    const float* g_feats, const float* g_depth, const float* g_ws, const float* g_alpha,
+    const float* t, const float* sigma, const float* feats, const unsigned char* valid,
+    long long n_rays, int S, int F, int occ_mode, float* grad_sigma, float* grad_feats,
+    void* stream) {
+  int rc = check_args(n_rays, S, F);
+  if (rc) return rc;
+  SAILOR_REQUIRE(F <= 64, "volume_render_torch_backward: at most 64 channels (got %d)", F);
+  return sailor::in_parts(n_rays, [&](long long r, long long n) {
+    return launch_backward(g_feats + r * F, g_depth + r, g_ws + r, g_alpha + r, t + r * S,
+                           sigma + r * S, feats + r * S * F, valid ? valid + r : nullptr, n, S,
+                           F, occ_mode, grad_sigma + r * S, grad_feats + r * S * F,
+                           sailor::as_stream(stream));
+  });
 }

@@ -109,10 +109,11 @@ __device__ __forceinline__ void inv3(const float* M, float* out) {
   out[8] = (b2 * a1 - a2 * b1) / det;
 }
 
-// grid = (ceil(H*W / kRays), B); 8 lanes per target pixel.
+// grid = (ceil(pixels / kRays), B), pixels from `first` on; 8 lanes per target
+// pixel.
 __global__ void __launch_bounds__(kThreads, 6)
 trace_kernel(const float* __restrict__ K, const float* __restrict__ Rm,
-             const float* __restrict__ Tv, int H, int W,
+             const float* __restrict__ Tv, int H, int W, int first,
              const int* __restrict__ vc, const float4* __restrict__ node_pos,
              const int4* __restrict__ node_info, int n_nodes,
              const float* __restrict__ vol_bbox, const float* __restrict__ voxel_size,
@@ -128,7 +129,7 @@ trace_kernel(const float* __restrict__ K, const float* __restrict__ Rm,
   const LaneGroup grp;
   const int slot = threadIdx.x / kGroup;
   const int HW = H * W;
-  const long long p64 = (long long)blockIdx.x * kRays + slot;
+  const long long p64 = first + (long long)blockIdx.x * kRays + slot;
   // groups past the image carry no ray but stay for the wave's tail fill
   const bool live = p64 < HW;
   const int p = (int)p64;
@@ -228,11 +229,13 @@ extern "C" int sailor_trace_sample(const float* K, const float* R, const float* 
   SAILOR_REQUIRE(B > 0 && H > 0 && W > 0 && S > 0, "trace_sample: bad sizes");
   SAILOR_REQUIRE(dim_coarse > 0 && dim_fine % dim_coarse == 0, "trace_sample: bad dims");
   const int rate = dim_fine / dim_coarse;
-  hipLaunchKernelGGL(trace_kernel, dim3(sailor::ceil_div((long long)H * W, kRays), B),
-                     dim3(kThreads), 0, sailor::as_stream(stream), K, R, T, H, W, vol_coarse,
-                     reinterpret_cast<const float4*>(node_pos),
-                     reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,
-                     dim_fine, dim_coarse, rate, start_scale, S, noise, rays_out, sampled_idx,
-                     sampled_t, valid_len);
-  return sailor::check_launch("trace_sample");
+  return sailor::in_parts((long long)H * W, [&](long long first, long long n) {
+    hipLaunchKernelGGL(trace_kernel, dim3(sailor::ceil_div(n, kRays), B), dim3(kThreads), 0,
+                       sailor::as_stream(stream), K, R, T, H, W, (int)first, vol_coarse,
+                       reinterpret_cast<const float4*>(node_pos),
+                       reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,
+                       dim_fine, dim_coarse, rate, start_scale, S, noise, rays_out, sampled_idx,
+                       sampled_t, valid_len);
+    return sailor::check_launch("trace_sample");
+  });
 }

@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(kWalkThreads)
 octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos,
                         const int4* __restrict__ node_info, int n_nodes,
                         const float* __restrict__ vol_bbox, const float* __restrict__ voxel_size,
-                        int B, int dim_fine, int dim_coarse, int rate,
+                        long long first, long long ray_end, int dim_fine, int dim_coarse, int rate,
                         const float* __restrict__ ray_ori, const float* __restrict__ ray_dir,
                         int R, int n_max_c, int n_max, int th_early_stop, int opt_num,
                         int* __restrict__ idx_c, float* __restrict__ t0_c,
@@ -183,10 +183,10 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
   __shared__ float s_t0[kEntries * kRays], s_t1[kEntries * kRays];
   const LaneGroup grp;
   const int slot = threadIdx.x / kGroup;
-  const long long ray = (long long)blockIdx.x * kRays + slot;
+  const long long ray = first + (long long)blockIdx.x * kRays + slot;
   int n_coarse = 0, n_fine = 0, filled_c = n_max_c, filled = n_max;
   bool overflow = false;
-  if (ray < (long long)B * R) {
+  if (ray < ray_end) {
     const int b = (int)(ray / R);
     sailor::RayCtx ctx;
     ctx.init(vc, node_pos, node_info, n_nodes, vol_bbox, voxel_size, b, dim_fine, dim_coarse,
@@ -241,12 +241,12 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
                          const float* __restrict__ tmax, const float* __restrict__ noise,
                          const float* __restrict__ valid_len,
                          const float4* __restrict__ node_pos, int n_nodes,
-                         const float* __restrict__ voxel_size, int B, int R, int n_max,
-                         int max_hits, int S, int start_scale, int* __restrict__ sidx,
+                         const float* __restrict__ voxel_size, long long first, long long ray_end,
+                         int R, int n_max, int max_hits, int S, int start_scale, int* __restrict__ sidx,
                          float* __restrict__ st) {
   const LaneGroup grp;
-  const long long ray = (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
-  if (ray >= (long long)B * R) return;   // whole groups
+  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
+  if (ray >= ray_end) return;   // whole groups
   const int b = (int)(ray / R);
   const int* hi = hit_idx + ray * n_max;
   const float* mn_ = tmin + ray * n_max;
@@ -525,14 +525,17 @@ extern "C" int sailor_octree_traversal(
   SAILOR_REQUIRE(dim_coarse > 0 && rate >= 1 && n_nodes >= 0, "octree_traversal: bad tree dims");
   if (R == 0) return SAILOR_OK;
   hipStream_t st = sailor::as_stream(stream);
-  hipLaunchKernelGGL(octree_traversal_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kWalkThreads), 0, st, vol_coarse,
-                     reinterpret_cast<const float4*>(node_pos),
-                     reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size, B,
-                     dim_fine, dim_coarse, rate, ray_ori, ray_dir, R, n_max_hits_coarse,
-                     n_max_hits, th_early_stop, opt_num_intersected, hit_idx_coarse,
-                     tmin_coarse, tmax_coarse, hit_idx, tmin, tmax, valid_len, status);
-  return sailor::check_launch("octree_traversal");
+  return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
+    hipLaunchKernelGGL(octree_traversal_kernel, dim3(sailor::ceil_div(n, kRays)),
+                       dim3(kWalkThreads), 0, st, vol_coarse,
+                       reinterpret_cast<const float4*>(node_pos),
+                       reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,
+                       first, first + n, dim_fine, dim_coarse, rate, ray_ori, ray_dir, R,
+                       n_max_hits_coarse, n_max_hits, th_early_stop, opt_num_intersected,
+                       hit_idx_coarse, tmin_coarse, tmax_coarse, hit_idx, tmin, tmax, valid_len,
+                       status);
+    return sailor::check_launch("octree_traversal");
+  });
 }
 
 extern "C" int sailor_octree_sampling(const int32_t* hit_idx, const float* tmin,
@@ -546,11 +549,14 @@ extern "C" int sailor_octree_sampling(const int32_t* hit_idx, const float* tmin,
   SAILOR_REQUIRE(max_hits >= 0 && max_hits <= n_max_hits,
                  "ray_voxels_points_sampling: max_hits %d outside [0, %d]", max_hits, n_max_hits);
   if (R == 0) return SAILOR_OK;
-  hipLaunchKernelGGL(adaptive_sampling_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kWalkThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax, noise,
-                     valid_len, reinterpret_cast<const float4*>(node_pos), n_nodes, voxel_size,
-                     B, R, n_max_hits, max_hits, S, start_scale, sampled_idx, sampled_t);
-  return sailor::check_launch("ray_voxels_points_sampling");
+  return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
+    hipLaunchKernelGGL(adaptive_sampling_kernel, dim3(sailor::ceil_div(n, kRays)),
+                       dim3(kWalkThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax,
+                       noise, valid_len, reinterpret_cast<const float4*>(node_pos), n_nodes,
+                       voxel_size, first, first + n, R, n_max_hits, max_hits, S, start_scale,
+                       sampled_idx, sampled_t);
+    return sailor::check_launch("ray_voxels_points_sampling");
+  });
 }
 
 extern "C" int sailor_trilinear_aggregate(const float* node_pos, int n_nodes,

@@ -63,18 +63,18 @@ __global__ void __launch_bounds__(kWalkThreads)
 traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos,
                  const int4* __restrict__ node_info, int n_nodes,
                  const float* __restrict__ vol_bbox,
-                 const float* __restrict__ voxel_size, int B, int dim_fine,
-                 int dim_coarse, int rate, const float* __restrict__ ray_ori,
+                 const float* __restrict__ voxel_size, long long first, long long ray_end,
+                 int dim_fine, int dim_coarse, int rate, const float* __restrict__ ray_ori,
                  const float* __restrict__ ray_dir, int R, int n_max,
                  int th_early_stop, int is_training, int opt_num,
                  int* __restrict__ hit_idx, float* __restrict__ tmin,
                  float* __restrict__ tmax, float* __restrict__ valid_len,
                  int* __restrict__ status) {
   const LaneGroup grp;
-  const long long ray = (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
+  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
   int count = 0, filled = n_max;
   bool overflow = false;
-  if (ray < (long long)B * R) {
+  if (ray < ray_end) {
     const int b = (int)(ray / R);
     sailor::RayCtx ctx;
     ctx.init(vc, node_pos, node_info, n_nodes, vol_bbox, voxel_size, b, dim_fine,
@@ -114,13 +114,13 @@ sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
                 const float* __restrict__ tmax, const float* __restrict__ noise,
                 const float* __restrict__ valid_len,
                 const float4* __restrict__ node_pos,
-                const float* __restrict__ voxel_size, int B, int R, int n_max,
-                int S, int start_scale, int* __restrict__ sidx,
+                const float* __restrict__ voxel_size, long long first, long long ray_end, int R,
+                int n_max, int S, int start_scale, int* __restrict__ sidx,
                 float* __restrict__ st) {
   const LaneGroup grp;
-  const long long ray = (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
+  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
   int has = S;   // rows past the batch have no tail
-  if (ray < (long long)B * R) {
+  if (ray < ray_end) {
     const int b = (int)(ray / R);
     const int* hi = hit_idx + ray * n_max;
     const float* h0 = tmin + ray * n_max;
@@ -232,15 +232,15 @@ extern "C" int sailor_octree_voxel_traversal(
   SAILOR_REQUIRE(dim_coarse > 0 && rate >= 1, "voxel_traversal: bad tree dims");
   hipStream_t st = sailor::as_stream(stream);
   if (R == 0) return SAILOR_OK;
-  hipLaunchKernelGGL(traversal_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kWalkThreads), 0, st, vol_coarse,
-                     reinterpret_cast<const float4*>(node_pos),
-                     reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox,
-                     voxel_size, B,
-                     dim_fine, dim_coarse, rate, ray_ori, ray_dir, R, n_max_hits,
-                     th_early_stop, is_training, opt_num_intersected, hit_idx, tmin,
-                     tmax, valid_len, status);
-  return sailor::check_launch("voxel_traversal");
+  return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
+    hipLaunchKernelGGL(traversal_kernel, dim3(sailor::ceil_div(n, kRays)), dim3(kWalkThreads), 0,
+                       st, vol_coarse, reinterpret_cast<const float4*>(node_pos),
+                       reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,
+                       first, first + n, dim_fine, dim_coarse, rate, ray_ori, ray_dir, R,
+                       n_max_hits, th_early_stop, is_training, opt_num_intersected, hit_idx,
+                       tmin, tmax, valid_len, status);
+    return sailor::check_launch("voxel_traversal");
+  });
 }
 
 extern "C" int sailor_octree_sampling_coarse(
@@ -250,12 +250,13 @@ extern "C" int sailor_octree_sampling_coarse(
     int32_t* sampled_idx, float* sampled_t, void* stream) {
   SAILOR_REQUIRE(B > 0 && R >= 0 && S > 0 && n_max_hits > 0, "sampling: bad sizes");
   if (R == 0) return SAILOR_OK;
-  hipLaunchKernelGGL(sampling_kernel, dim3(sailor::ceil_div((long long)B * R, kRays)),
-                     dim3(kWalkThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax,
-                     noise, valid_len, reinterpret_cast<const float4*>(node_pos),
-                     voxel_size, B, R, n_max_hits, S, start_scale, sampled_idx,
-                     sampled_t);
-  return sailor::check_launch("sampling_coarse");
+  return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
+    hipLaunchKernelGGL(sampling_kernel, dim3(sailor::ceil_div(n, kRays)), dim3(kWalkThreads), 0,
+                       sailor::as_stream(stream), hit_idx, tmin, tmax, noise, valid_len,
+                       reinterpret_cast<const float4*>(node_pos), voxel_size, first, first + n,
+                       R, n_max_hits, S, start_scale, sampled_idx, sampled_t);
+    return sailor::check_launch("sampling_coarse");
+  });
 }
 
 extern "C" int sailor_sort_samplings(const float* t, int n_rows, int S, float* sorted,
