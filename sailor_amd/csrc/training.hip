@@ -288,6 +288,7 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
   // lane's own hits in order, then the lanes'
   float min_mid = 99999.0f, min_vs = 99999.0f, z0 = -1.0f, z1 = -1.0f;
   int min_idx = -1, min_at = n_max;
+  bool nan_mid = false;
   bool end = cnt >= S;   // no slot left to fill
   for (int i0 = 0; i0 < n_max && !end; i0 += kGroup) {
     const int i = i0 + grp.sub;
@@ -299,6 +300,7 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
     if (!(vs <= min_vs)) continue;
     const float a = mn_[i], c = mx_[i];
     const float mid = (float)((double)(a + c) / 2.0);
+    nan_mid |= mid != mid;
     if (vs < min_vs || mid < min_mid) {
       min_mid = mid;
       z0 = a;
@@ -307,6 +309,28 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
       min_at = i;
     }
     min_vs = vs;
+  }
+  // a NaN midpoint (lists of another origin) stays if it comes first and never
+  // replaces another: the hits of all lanes in order, by every lane
+  if (grp.vote(nan_mid)) {
+    min_mid = min_vs = 99999.0f;
+    min_idx = -1;
+    for (int i = 0; i < n_max && hi[i] != -1; ++i) {
+      const int vi = hi[i];
+      if (vi < 0 || vi >= n_nodes) continue;
+      const float vs = node_pos[vi].w;
+      if (!(vs <= min_vs)) continue;
+      const float a = mn_[i], c = mx_[i];
+      const float mid = (float)((double)(a + c) / 2.0);
+      if (vs < min_vs || mid < min_mid) {
+        min_mid = mid;
+        z0 = a;
+        z1 = c;
+        min_idx = vi;
+      }
+      min_vs = vs;
+    }
+    min_at = 0;   // all lanes agree
   }
 #pragma unroll
   for (int o = 1; o < kGroup; o <<= 1) {

@@ -153,3 +153,34 @@ def test_project_sampled_xyz_bitexact(case, corners):
                           K, RT, 128, 128, corners)
     np.testing.assert_array_equal(xy.cpu().numpy(), rxy)
     np.testing.assert_array_equal(z.cpu().numpy(), rz)
+
+
+@pytest.mark.parametrize("n_max,S", [(1, 5), (7, 8), (40, 33)])
+def test_adaptive_sampling_of_lists_with_nan_and_infinite_intervals(case, n_max, S):
+    """Lists that did not come from a traversal: nodes of both sizes in any order,
+    intervals with NaN and infinite ends, lists of every length.  The fill-up
+    interval is the one a walk in list order picks (a NaN midpoint stays if it
+    comes first and never replaces another)."""
+    dim, rate, tree, _, _, h = case
+    rng = np.random.default_rng(n_max)
+    R = 301
+    n = int((h["info"][:, 0] >= 0).sum())
+    idx = rng.integers(0, n, (1, R, n_max)).astype(np.int32)
+    idx[0, np.arange(R), :] = np.where(np.arange(n_max)[None] < rng.integers(0, n_max + 1, (R, 1)),
+                                       idx[0], -1)
+    t0 = rng.uniform(0.5, 3.0, idx.shape).astype(np.float32)
+    t1 = (t0 + rng.uniform(0, 0.2, idx.shape)).astype(np.float32)
+    t0[rng.random(idx.shape) < 0.3] = np.nan
+    t1[rng.random(idx.shape) < 0.1] = np.inf
+    t0[rng.random(idx.shape) < 0.05] = -np.inf
+    vl = rng.uniform(0.5, 40.0, (1, R)).astype(np.float32)
+    nz = rng.random((1, R, S)).astype(np.float32)
+    held = getattr(tree, "num_max_intersected_voxels_fine", None)
+    tree.num_max_intersected_voxels_fine = n_max
+    sidx, st = tree.ray_voxels_points_sampling(_t(idx), _t(t0), _t(t1), _t(vl[..., None]), _t(nz),
+                                               0, S)
+    tree.num_max_intersected_voxels_fine = held
+    ri, rt = orc.sampling_adaptive(idx, t0, t1, nz, vl, h["pos"], h["vs"], S, 2, n_max)
+    np.testing.assert_array_equal(sidx.cpu().numpy(), ri)
+    np.testing.assert_array_equal(st.cpu().numpy(), rt)
+    assert (ri >= 0).any() and np.isnan(rt).any()
