@@ -27,19 +27,20 @@ constexpr int kThreads = 256;
 using sailor::kGroup;
 using sailor::LaneGroup;
 
-constexpr int kWalkThreads = 64;               // one wave: rays differ widely in length
-constexpr int kRays = kWalkThreads / kGroup;   // rays of a workgroup, 8 lanes each
-constexpr int kEntries = 32;               // entries of a coarse hit kept in LDS per ray
+constexpr int kWalkThreads = 64;   // one wave: rays differ widely in length
+constexpr int kEntries = 32;       // entries of a coarse hit kept in LDS per ray
 
 // Receives the coarse hits of the DDA (RayVoxelIntersectionNodeList) and
 // expands each into its fine entries right away: the coarse entry, then the
 // children in stack order (last child first) that the slab test hits; an
 // interval equal to one already listed for this coarse hit keeps the
-// smaller node (ray_octree_traversal :518-567).  The ray's 8 lanes test 8
-// children at a time and compare a hit with 8 listed entries at a time; a
+// smaller node (ray_octree_traversal :518-567).  The ray's G lanes test G
+// children at a time and compare a hit with G listed entries at a time; a
 // coarse hit's entries are kept in LDS (a ray meets at most 22 of 8^3
 // children), those past kEntries are read back from their row.
+template <int G>
 struct TreeSink {
+  static constexpr int kRays = kWalkThreads / G;
   const float4* np;
   const int4* ni;
   int n_nodes;
@@ -52,7 +53,7 @@ struct TreeSink {
   float* t0;
   float* t1;
   int cap;
-  const LaneGroup& grp;
+  const LaneGroup<G>& grp;
   int* e_node;     // [kEntries] of this ray, one slot every kRays words
   float *e_t0, *e_t1;
   int cnt;
@@ -93,9 +94,9 @@ struct TreeSink {
       const int last = min(info.z + info.w, n_nodes) - 1;
       int ch = last - grp.sub;
       float4 qn = ch >= info.z ? np[ch] : make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int ch0 = last; ch0 >= info.z; ch0 -= kGroup, ch -= kGroup) {
+      for (int ch0 = last; ch0 >= info.z; ch0 -= G, ch -= G) {
         const float4 q = qn;
-        if (ch - kGroup >= info.z) qn = np[ch - kGroup];
+        if (ch - G >= info.z) qn = np[ch - G];
         const float2 cd = sailor::slab_test(o, inv, make_float3(q.x, q.y, q.z), q.w);
         unsigned votes = grp.vote(ch >= info.z && !(cd.x == -1.0f || cd.y == -1.0f));
         while (votes) {
@@ -106,7 +107,7 @@ struct TreeSink {
           // the first listed entry of this coarse hit with the same interval
           const int lim = cnt < cap ? cnt : cap;
           int same = -1;
-          for (int j0 = g0; j0 < lim && same < 0; j0 += kGroup) {
+          for (int j0 = g0; j0 < lim && same < 0; j0 += G) {
             const int j = j0 + grp.sub, k = j - g0;
             bool eq = false;
             if (j < lim) {
@@ -138,7 +139,7 @@ struct TreeSink {
     // valid length of the listed entries, in order
     const int lim = cnt < cap ? cnt : cap;
     sailor::wave_fence();
-    for (int j0 = g0; j0 < lim; j0 += kGroup) {
+    for (int j0 = g0; j0 < lim; j0 += G) {
       const int j = j0 + grp.sub, k = j - g0;
       float part = 0.0f;
       if (j < lim) {
@@ -157,7 +158,7 @@ struct TreeSink {
         const float scale = start_vs / np[nd].w;
         part = (a1 - a0) * scale;
       }
-      const int n = min(kGroup, lim - j0);
+      const int n = min(G, lim - j0);
       for (int i = 0; i < n; ++i) vl += grp.from(part, i);
     }
   }
@@ -165,9 +166,10 @@ struct TreeSink {
   __device__ __forceinline__ bool stop() const { return false; }
 };
 
-// 8 lanes per ray (traversal_common.h); each wave then fills what its 8 rows
-// have left with -1.  20,000 random rays through a 128^3 tree filled 79 of 256
+// G lanes per ray (traversal_common.h); each wave then fills what its rows have
+// left with -1.  20,000 random rays through a 128^3 tree filled 79 of 256
 // CUs with a lane per ray and took 1221 us after two fills, now 171 us in all.
+template <int G>
 __global__ void __launch_bounds__(kWalkThreads)
 octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos,
                         const int4* __restrict__ node_info, int n_nodes,
@@ -179,10 +181,11 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
                         float* __restrict__ t1_c, int* __restrict__ idx,
                         float* __restrict__ t0, float* __restrict__ t1,
                         float* __restrict__ valid_len, int* __restrict__ status) {
+  constexpr int kRays = kWalkThreads / G;
   __shared__ int s_node[kEntries * kRays];
   __shared__ float s_t0[kEntries * kRays], s_t1[kEntries * kRays];
-  const LaneGroup grp;
-  const int slot = threadIdx.x / kGroup;
+  const LaneGroup<G> grp;
+  const int slot = threadIdx.x / G;
   const long long ray = first + (long long)blockIdx.x * kRays + slot;
   int n_coarse = 0, n_fine = 0, filled_c = n_max_c, filled = n_max;
   bool overflow = false;
@@ -191,7 +194,7 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
     sailor::RayCtx ctx;
     ctx.init(vc, node_pos, node_info, n_nodes, vol_bbox, voxel_size, b, dim_fine, dim_coarse,
              rate, ray_ori + ray * 3, ray_dir + ray * 3);
-    TreeSink sink{node_pos, node_info, n_nodes, ctx.o, ctx.inv,
+    TreeSink<G> sink{node_pos, node_info, n_nodes, ctx.o, ctx.inv,
                   idx_c + ray * n_max_c, t0_c + ray * n_max_c, t1_c + ray * n_max_c, n_max_c,
                   idx + ray * n_max, t0 + ray * n_max, t1 + ray * n_max, n_max,
                   grp, s_node + slot, s_t0 + slot, s_t1 + slot,
@@ -204,11 +207,11 @@ octree_traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ n
     filled_c = min(n_coarse, n_max_c);
     filled = min(n_fine, n_max);
   }
-  const long long ray0 = ray - grp.base / kGroup;
+  const long long ray0 = ray - grp.base / G;
   auto fill = [&](int used, int cap, int* ids, float* a, float* c) {
 #pragma unroll 1
-    for (int k = 0; k < 64 / kGroup; ++k) {
-      const int from = __builtin_amdgcn_readlane(used, k * kGroup);
+    for (int k = 0; k < 64 / G; ++k) {
+      const int from = __builtin_amdgcn_readlane(used, k * G);
       if (from >= cap) continue;
       const long long row = (ray0 + k) * cap;
       const int lane = threadIdx.x & 63;
@@ -244,7 +247,8 @@ adaptive_sampling_kernel(const int* __restrict__ hit_idx, const float* __restric
                          const float* __restrict__ voxel_size, long long first, long long ray_end,
                          int R, int n_max, int max_hits, int S, int start_scale, int* __restrict__ sidx,
                          float* __restrict__ st) {
-  const LaneGroup grp;
+  constexpr int kRays = kWalkThreads / kGroup;
+  const LaneGroup<kGroup> grp;
   const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
   if (ray >= ray_end) return;   // whole groups
   const int b = (int)(ray / R);
@@ -549,8 +553,16 @@ extern "C" int sailor_octree_traversal(
   SAILOR_REQUIRE(dim_coarse > 0 && rate >= 1 && n_nodes >= 0, "octree_traversal: bad tree dims");
   if (R == 0) return SAILOR_OK;
   hipStream_t st = sailor::as_stream(stream);
-  return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
-    hipLaunchKernelGGL(octree_traversal_kernel, dim3(sailor::ceil_div(n, kRays)),
+  // 8 and 4 lanes, us, rows of 128 + 128: rate 2 32,768 random rays 175 and 169,
+  // 65,536 263 and 221, 1,048,576 2789 and 1858 (2 lanes 2140); rate 4 131,072
+  // in raster order 321 and 360, random 437 and 318, 1,048,576 3244 and 1766;
+  // rate 8 1,048,576 in raster order 1274 and 1310, random 3309 and 2447
+  const long long rays = (long long)B * R;
+  const int lanes = rate < 8 && rays >= (rate < 4 ? 1 << 16 : 1 << 18) ? 4 : kGroup;
+  auto kern = octree_traversal_kernel<8>;
+  if (lanes == 4) kern = octree_traversal_kernel<4>;
+  return sailor::in_parts(rays, [&](long long first, long long n) {
+    hipLaunchKernelGGL(kern, dim3(sailor::ceil_div(n, kWalkThreads / lanes)),
                        dim3(kWalkThreads), 0, st, vol_coarse,
                        reinterpret_cast<const float4*>(node_pos),
                        reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,
@@ -574,7 +586,8 @@ extern "C" int sailor_octree_sampling(const int32_t* hit_idx, const float* tmin,
                  "ray_voxels_points_sampling: max_hits %d outside [0, %d]", max_hits, n_max_hits);
   if (R == 0) return SAILOR_OK;
   return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
-    hipLaunchKernelGGL(adaptive_sampling_kernel, dim3(sailor::ceil_div(n, kRays)),
+    hipLaunchKernelGGL(adaptive_sampling_kernel,
+                       dim3(sailor::ceil_div(n, kWalkThreads / kGroup)),
                        dim3(kWalkThreads), 0, sailor::as_stream(stream), hit_idx, tmin, tmax,
                        noise, valid_len, reinterpret_cast<const float4*>(node_pos), n_nodes,
                        voxel_size, first, first + n, R, n_max_hits, max_hits, S, start_scale,

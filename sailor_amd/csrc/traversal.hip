@@ -22,20 +22,29 @@ namespace {
 
 constexpr int kThreads = 256;
 
-using sailor::kGroup;
 using sailor::LaneGroup;
 using sailor::SampleRow;
 
-constexpr int kWalkThreads = 64;               // one wave: rays differ widely in length
-constexpr int kRays = kWalkThreads / kGroup;   // rays of a workgroup, 8 lanes each
+constexpr int kWalkThreads = 64;   // one wave: rays differ widely in length
 
+__global__ void fill_lists(int* __restrict__ idx, float* __restrict__ a, float* __restrict__ b,
+                           long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    idx[i] = -1;
+    a[i] = -1.0f;
+    b[i] = -1.0f;
+  }
+}
+
+template <int G>
 struct ListSink {
   int* idx;
   float* tmin;
   float* tmax;
   int cap;
   bool overflow;
-  const LaneGroup& grp;
+  const LaneGroup<G>& grp;
   __device__ __forceinline__ void store(int pos, int node, float t0, float t1) {
     if (pos < cap) {
       idx[pos] = node;
@@ -55,10 +64,12 @@ struct ListSink {
   __device__ __forceinline__ bool stop() const { return false; }
 };
 
-// 8 lanes per ray (traversal_common.h); each wave then fills what its 8 rows
-// have left with -1.  The rows are what bounds the call (n_max 1024: 12 KB a
-// ray), so they are written once: a fill of all rows before a lane-per-ray
-// walk took 225 + 256 us for 102,400 rays, this kernel 239 us (5.3 TB/s).
+// G lanes per ray (traversal_common.h); each wave then fills what its rows have
+// left with -1.  The rows are what bounds the call (n_max 1024: 12 KB a ray), so
+// they are written once: a fill of all rows before a lane-per-ray walk took
+// 225 + 256 us for 102,400 rays, this kernel 239 us (5.3 TB/s).  A lane per ray
+// (G = 1) finds its rows filled.
+template <int G>
 __global__ void __launch_bounds__(kWalkThreads)
 traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos,
                  const int4* __restrict__ node_info, int n_nodes,
@@ -70,8 +81,9 @@ traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos
                  int* __restrict__ hit_idx, float* __restrict__ tmin,
                  float* __restrict__ tmax, float* __restrict__ valid_len,
                  int* __restrict__ status) {
-  const LaneGroup grp;
-  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
+  constexpr int kRays = kWalkThreads / G;
+  const LaneGroup<G> grp;
+  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / G;
   int count = 0, filled = n_max;
   bool overflow = false;
   if (ray < ray_end) {
@@ -79,19 +91,19 @@ traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos
     sailor::RayCtx ctx;
     ctx.init(vc, node_pos, node_info, n_nodes, vol_bbox, voxel_size, b, dim_fine,
              dim_coarse, rate, ray_ori + ray * 3, ray_dir + ray * 3);
-    ListSink sink{hit_idx + ray * n_max, tmin + ray * n_max, tmax + ray * n_max,
-                  n_max, false, grp};
+    ListSink<G> sink{hit_idx + ray * n_max, tmin + ray * n_max, tmax + ray * n_max,
+                     n_max, false, grp};
     float vl = 0.0f;
     count = sailor::traverse(ctx, grp, th_early_stop, is_training != 0, opt_num, sink, &vl);
     if (grp.sub == 0) valid_len[ray] = vl;
     overflow = sink.overflow;
-    filled = min(count, n_max);
+    if (G > 1) filled = min(count, n_max);
   }
   const int lane = threadIdx.x & 63;
-  const long long ray0 = ray - grp.base / kGroup;
+  const long long ray0 = ray - grp.base / G;
 #pragma unroll 1
-  for (int k = 0; k < 64 / kGroup; ++k) {
-    const int from = __builtin_amdgcn_readlane(filled, k * kGroup);
+  for (int k = 0; k < (G > 1 ? 64 / G : 0); ++k) {
+    const int from = __builtin_amdgcn_readlane(filled, k * G);
     if (from >= n_max) continue;
     const long long row = (ray0 + k) * n_max;
     sailor::fill_row(reinterpret_cast<unsigned*>(hit_idx + row), from, n_max, 0xffffffffu, lane);
@@ -108,7 +120,8 @@ traversal_kernel(const int* __restrict__ vc, const float4* __restrict__ node_pos
   }
 }
 
-// 8 lanes per ray, 8 hits at a time; the row's unused slots are -1.
+// G lanes per ray, G hits at a time; the row's unused slots are -1.
+template <int G>
 __global__ void __launch_bounds__(kWalkThreads)
 sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
                 const float* __restrict__ tmax, const float* __restrict__ noise,
@@ -117,8 +130,9 @@ sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
                 const float* __restrict__ voxel_size, long long first, long long ray_end, int R,
                 int n_max, int S, int start_scale, int* __restrict__ sidx,
                 float* __restrict__ st) {
-  const LaneGroup grp;
-  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / kGroup;
+  constexpr int kRays = kWalkThreads / G;
+  const LaneGroup<G> grp;
+  const long long ray = first + (long long)blockIdx.x * kRays + threadIdx.x / G;
   int has = S;   // rows past the batch have no tail
   if (ray < ray_end) {
     const int b = (int)(ray / R);
@@ -130,7 +144,7 @@ sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
              sidx + ray * S, st + ray * S);
     if (hi[0] >= 0) {
       bool end = false;   // a slot without a hit ends the list
-      for (int i0 = 0; i0 < n_max && !end && row.has < S; i0 += kGroup) {
+      for (int i0 = 0; i0 < n_max && !end && row.has < S; i0 += G) {
         const int i = i0 + grp.sub;
         int v = -1;
         float mn = -1.0f, mx = -1.0f;
@@ -148,7 +162,7 @@ sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
       const int left = min(S - row.has, n_max);
       int placed = 0;
       end = false;
-      for (int i0 = 0; i0 < left && !end; i0 += kGroup) {
+      for (int i0 = 0; i0 < left && !end; i0 += G) {
         const int i = i0 + grp.sub;
         int v = -1;
         float mn = -1.0f, mx = -1.0f;
@@ -158,7 +172,7 @@ sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
           mx = h1[i];
         }
         const unsigned gone = grp.vote(v < 0 || mn < 0 || mx < 0);
-        const int n = gone ? __ffs(gone) - 1 : kGroup;
+        const int n = gone ? __ffs(gone) - 1 : G;
         end = gone != 0;
         if (grp.sub < n) row.leftover(row.has + i, v, mn, mx);
         placed += n;
@@ -167,11 +181,18 @@ sampling_kernel(const int* __restrict__ hit_idx, const float* __restrict__ tmin,
     }
     has = row.has;
   }
+  if constexpr (G == 1) {
+    for (int j = has; j < S; ++j) {
+      sidx[ray * S + j] = -1;
+      st[ray * S + j] = -1.0f;
+    }
+    return;
+  }
   const int lane = threadIdx.x & 63;
-  const long long ray0 = ray - grp.base / kGroup;
+  const long long ray0 = ray - grp.base / G;
 #pragma unroll
-  for (int k = 0; k < 64 / kGroup; ++k) {
-    const int hk = __builtin_amdgcn_readlane(has, k * kGroup);
+  for (int k = 0; k < 64 / G; ++k) {
+    const int hk = __builtin_amdgcn_readlane(has, k * G);
     for (int j = hk + lane; j < S; j += 64) {
       sidx[(ray0 + k) * S + j] = -1;
       st[(ray0 + k) * S + j] = -1.0f;
@@ -219,6 +240,22 @@ sort_rows(const float* __restrict__ t, int n_rows, int S, float* __restrict__ ou
   }
 }
 
+// Lanes per ray.  With is_training a node's children are not tested, so there is
+// nothing to share; wide rows are bound by their writes.  8 lanes and (lanes
+// taken), us: is_training, rate 4, n_max 128, random rays 4,096 33 and (1) 34,
+// 16,384 50 and 36, 1,048,576 1514 and 526; n_max 1024 16,384 58 and 64, 65,536
+// 193 and 178.  Otherwise, n_max 128, rate 2 65,536 167 and (2) 151, 131,072 259
+// and 181, 1,048,576 1585 and 947; rate 4 262,144 in raster order 279 and (4)
+// 286, 524,288 random 742 and 571; rate 8 1,048,576 1521 and (4) 1723; n_max 1024
+// rate 2 262,144 734 and (2) 802.
+int traversal_lanes(long long rays, int rate, int n_max, bool training) {
+  const bool narrow = n_max < 512;
+  if (training) return rays >= (narrow ? 8192 : 65536) ? 1 : 8;
+  if (narrow && rate < 4 && rays >= 1 << 17) return 2;
+  if (narrow && rate < 8 && rays >= 1 << 19) return 4;
+  return 8;
+}
+
 }  // namespace
 
 extern "C" int sailor_octree_voxel_traversal(
@@ -232,8 +269,21 @@ extern "C" int sailor_octree_voxel_traversal(
   SAILOR_REQUIRE(dim_coarse > 0 && rate >= 1, "voxel_traversal: bad tree dims");
   hipStream_t st = sailor::as_stream(stream);
   if (R == 0) return SAILOR_OK;
-  return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
-    hipLaunchKernelGGL(traversal_kernel, dim3(sailor::ceil_div(n, kRays)), dim3(kWalkThreads), 0,
+  const long long rays = (long long)B * R;
+  const int lanes = traversal_lanes(rays, rate, n_max_hits, is_training != 0);
+  auto kern = traversal_kernel<8>;
+  if (lanes == 4) kern = traversal_kernel<4>;
+  if (lanes == 2) kern = traversal_kernel<2>;
+  if (lanes == 1) {
+    kern = traversal_kernel<1>;
+    const long long n = rays * n_max_hits;
+    hipLaunchKernelGGL(fill_lists,
+                       dim3((unsigned)std::min<long long>((n + kThreads - 1) / kThreads, 65535)),
+                       dim3(kThreads), 0, st, hit_idx, tmin, tmax, n);
+    if (int e = sailor::check_launch("voxel_traversal (fill)")) return e;
+  }
+  return sailor::in_parts(rays, [&](long long first, long long n) {
+    hipLaunchKernelGGL(kern, dim3(sailor::ceil_div(n, kWalkThreads / lanes)), dim3(kWalkThreads), 0,
                        st, vol_coarse, reinterpret_cast<const float4*>(node_pos),
                        reinterpret_cast<const int4*>(node_info), n_nodes, vol_bbox, voxel_size,
                        first, first + n, dim_fine, dim_coarse, rate, ray_ori, ray_dir, R,
@@ -250,8 +300,13 @@ extern "C" int sailor_octree_sampling_coarse(
     int32_t* sampled_idx, float* sampled_t, void* stream) {
   SAILOR_REQUIRE(B > 0 && R >= 0 && S > 0 && n_max_hits > 0, "sampling: bad sizes");
   if (R == 0) return SAILOR_OK;
+  // 8 lanes and a lane per ray, us: 131,072 rays of 1 sample 13 and 7.5, of 4
+  // 14 and 11; 524,288 of 1 sample 36 and 22, of 2 26 and 42
+  const int lanes = S == 1 || (S <= 4 && (long long)B * R < 1 << 18) ? 1 : sailor::kGroup;
+  auto kern = sampling_kernel<8>;
+  if (lanes == 1) kern = sampling_kernel<1>;
   return sailor::in_parts((long long)B * R, [&](long long first, long long n) {
-    hipLaunchKernelGGL(sampling_kernel, dim3(sailor::ceil_div(n, kRays)), dim3(kWalkThreads), 0,
+    hipLaunchKernelGGL(kern, dim3(sailor::ceil_div(n, kWalkThreads / lanes)), dim3(kWalkThreads), 0,
                        sailor::as_stream(stream), hit_idx, tmin, tmax, noise, valid_len,
                        reinterpret_cast<const float4*>(node_pos), voxel_size, first, first + n,
                        R, n_max_hits, S, start_scale, sampled_idx, sampled_t);

@@ -122,36 +122,39 @@ struct Dda {
 };
 
 // ---- Lane groups -----------------------------------------------------------
-// kGroup lanes walk a ray together: all of them run the same DDA, and a
-// coarse node's children (up to rate^3 records, contiguous in the node array)
-// are tested kGroup at a time, so a test is one coalesced load and one slab
-// test instead of a serial chain of them.  8 lanes: a wave is as long as the
-// longest of 8 rays instead of 64, a launch has 8 times the waves to hide the
-// chain's loads behind, and the DDA that all lanes repeat is still cheap
-// (a wave per ray spends its time there).
+// G lanes walk a ray together: all of them run the same DDA, and a coarse
+// node's children (up to rate^3 records, contiguous in the node array) are
+// tested G at a time, so a test is one coalesced load and one slab test instead
+// of a serial chain of them.  8 lanes: a wave is as long as the longest of 8
+// rays instead of 64, a launch has 8 times the waves to hide the chain's loads
+// behind, and the DDA that all lanes repeat is still cheap (a wave per ray
+// spends its time there).  Calls with more rays than the chip holds waves for,
+// and few children per node to share, take fewer (rules at the entry points).
 constexpr int kGroup = 8;
 constexpr int kChildBatch = 2;   // children per lane loaded together (4: the same)
 
+template <int G>
 struct LaneGroup {
+  static constexpr int size = G;
   int sub, base;   // lane within the group, first lane of the group in its wave
   __device__ __forceinline__ LaneGroup() {
     const int lane = threadIdx.x & 63;
-    sub = lane % kGroup;
+    sub = lane % G;
     base = lane - sub;
   }
   // the group's lanes for which p holds, bit i = lane i
   __device__ __forceinline__ unsigned vote(bool p) const {
-    return (unsigned)(__ballot(p) >> base) & ((1u << kGroup) - 1);
+    return (unsigned)(__ballot(p) >> base) & ((1u << G) - 1);
   }
-  __device__ __forceinline__ float from(float x, int i) const { return __shfl(x, i, kGroup); }
-  __device__ __forceinline__ int from(int x, int i) const { return __shfl(x, i, kGroup); }
+  __device__ __forceinline__ float from(float x, int i) const { return __shfl(x, i, G); }
+  __device__ __forceinline__ int from(int x, int i) const { return __shfl(x, i, G); }
   __device__ __forceinline__ int before(unsigned votes) const {
     return __popc(votes & ((1u << sub) - 1));
   }
   __device__ __forceinline__ int inclusive_sum(int x) const {
 #pragma unroll
-    for (int o = 1; o < kGroup; o <<= 1) {
-      const int y = __shfl_up(x, o, kGroup);
+    for (int o = 1; o < G; o <<= 1) {
+      const int y = __shfl_up(x, o, G);
       if (sub >= o) x += y;
     }
     return x;
@@ -179,17 +182,17 @@ __device__ __forceinline__ void fill_row(unsigned* row, int from, int n, unsigne
 
 // Sink interface (every lane of the group makes the same calls):
 // put(pos, node, t0, t1) receives hit number `pos`; put_lanes(pos, node, t0,
-// t1, hit, votes) the hits of up to kGroup children, one per lane in order,
+// t1, hit, votes) the hits of up to G children, one per lane in order,
 // the first of them number `pos`; stop() is polled after every coarse cell
 // and may end the walk early (used once all samples are placed; never changes
 // hits that were already emitted).
 //
 // Returns the number of hits; *vl_out receives the weighted valid length
 // (children weighted by `rate`, the coarse interval by 1).
-template <class Sink>
-__device__ __forceinline__ int traverse(const RayCtx& c, const LaneGroup& grp, int th_early_stop,
-                                        bool training, int opt_num, Sink& sink,
-                                        float* vl_out) {
+template <int G, class Sink>
+__device__ __forceinline__ int traverse(const RayCtx& c, const LaneGroup<G>& grp,
+                                        int th_early_stop, bool training, int opt_num,
+                                        Sink& sink, float* vl_out) {
   float vl = 0.0f;
   int count = 0;
   float2 dep = slab_test(c.o, c.inv, c.center, c.vs_top * (float)c.dc);
@@ -225,17 +228,17 @@ __device__ __forceinline__ int traverse(const RayCtx& c, const LaneGroup& grp, i
           if (!training && info.z >= 0) {
             const int ch_end = min(info.z + info.w, c.n_nodes);
             // the records of up to kChildBatch children per lane are loaded
-            // together: a round of loads tests 16 children
-            for (int ch0 = info.z; ch0 < ch_end; ch0 += kGroup * kChildBatch) {
+            // together: a round of loads tests 2 G children
+            for (int ch0 = info.z; ch0 < ch_end; ch0 += G * kChildBatch) {
               float4 q[kChildBatch];
 #pragma unroll
               for (int u = 0; u < kChildBatch; ++u) {
-                const int ch = ch0 + u * kGroup + grp.sub;
+                const int ch = ch0 + u * G + grp.sub;
                 q[u] = c.np[ch < ch_end ? ch : ch_end - 1];
               }
 #pragma unroll
               for (int u = 0; u < kChildBatch; ++u) {
-                const int ch = ch0 + u * kGroup + grp.sub;
+                const int ch = ch0 + u * G + grp.sub;
                 const float2 cd =
                     slab_test(c.o, c.inv, make_float3(q[u].x, q[u].y, q[u].z), q[u].w);
                 const bool hit = ch < ch_end && !(cd.x < 0 || cd.y < 0);
@@ -288,7 +291,7 @@ __device__ __forceinline__ int traverse(const RayCtx& c, const LaneGroup& grp, i
 }
 
 // Length-weighted per-interval sampling (sampling_kernel.cu:1125-1174) of one
-// row by a lane group: kGroup hits at a time, one per lane in hit order.
+// row by a lane group: G hits at a time, one per lane in hit order.
 struct SampleRow {
   float valid_len, start_vs;
   int S;
@@ -321,7 +324,8 @@ struct SampleRow {
   // Places the samples of this lane's interval (mn, mx) of node v, size cvs:
   // as many as its share of the valid length, at least one, at most what the
   // intervals before it left.
-  __device__ __forceinline__ void intervals(const LaneGroup& grp, bool on, int v, float mn,
+  template <int G>
+  __device__ __forceinline__ void intervals(const LaneGroup<G>& grp, bool on, int v, float mn,
                                             float mx, float cvs) {
     int want = 0;
     if (on) {
@@ -348,7 +352,7 @@ struct SampleRow {
           oi[slot + j0 + j] = v;
         }
     }
-    has = min(S, has + grp.from(end, kGroup - 1));
+    has = min(S, has + grp.from(end, G - 1));
   }
   // One midpoint sample of a hit into `slot`.
   __device__ __forceinline__ void leftover(int slot, int v, float mn, float mx) {
