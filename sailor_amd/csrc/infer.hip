@@ -271,6 +271,11 @@ __device__ __forceinline__ float view_sum(float x) {
   return x;
 }
 
+// Several floats of an input that starts on any float: wide loads need 4-byte
+// alignment only, the type has to say so.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+
 // acc = bias + W x with the layer's A fragments in registers
 template <int STEPS>
 __device__ __forceinline__ void mfma_layer_r(const f16x8 (&w)[2][STEPS], const float* bias,
@@ -371,11 +376,11 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
     if (p < total && v < V) {
       const long long e = p + (batch_of(p) * (V - 1) + v) * n_pts;
       const float* g = geo + e * 16;
-      const float4 a = *reinterpret_cast<const float4*>(g + (h ? 8 : 0));
-      const float2 c = *reinterpret_cast<const float2*>(g + (h ? 6 : 4));
-      const float2 d = *reinterpret_cast<const float2*>(g + (h ? 12 : 14));
-      float2 f = c;
-      if (h == 0) f = make_float2(z[e], tpsdf[e]);
+      const f32x4u a = *reinterpret_cast<const f32x4u*>(g + (h ? 8 : 0));
+      const f32x2u c = *reinterpret_cast<const f32x2u*>(g + (h ? 6 : 4));
+      const f32x2u d = *reinterpret_cast<const f32x2u*>(g + (h ? 12 : 14));
+      f32x2u f = c;
+      if (h == 0) f = f32x2u{z[e], tpsdf[e]};
       x[0] = f.x; x[1] = f.y;
       x[2] = a.x; x[3] = a.y; x[4] = a.z; x[5] = a.w;
       x[6] = h ? d.x : c.x;

@@ -171,3 +171,20 @@ def test_many_short_batches_take_the_time_of_their_points():
     one = graph_us(lambda: InferNerf.infer_density(z, z, geo, pd, 1, B * N, V, 0))
     print(f"{B} batches {many:.1f} us, one {one:.1f} us")
     assert many <= 1.6 * one
+
+
+@pytest.mark.parametrize("V", [1, 3, 8])
+def test_density_features_may_start_on_any_float(V):
+    """Geometry features that are a view at an odd float of a larger tensor."""
+    from sailor_amd import InferNerf
+    pd = _cu(fc.params()[0], torch.float16)
+    N = 77
+    _, z, ps, geo, _, _, _ = fc.nerf_inputs(1, N, 1, V, 1, seed=V)
+    z, ps, geo = _cu(z), _cu(ps), _cu(geo)
+    want = InferNerf.infer_density(z, ps, geo, pd, 1, N, V, 0)
+    for shift in (1, 2, 3):
+        held = torch.empty(geo.numel() + shift, device="cuda")
+        odd = held[shift:].view(geo.shape)
+        odd.copy_(geo)
+        assert odd.data_ptr() % 16 == 4 * shift and odd.is_contiguous()
+        assert torch.equal(InferNerf.infer_density(z, ps, odd, pd, 1, N, V, 0), want)
