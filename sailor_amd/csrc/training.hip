@@ -36,8 +36,9 @@ constexpr int kEntries = 32;       // entries of a coarse hit kept in LDS per ra
 // interval equal to one already listed for this coarse hit keeps the
 // smaller node (ray_octree_traversal :518-567).  The ray's G lanes test G
 // children at a time and compare a hit with G listed entries at a time; a
-// coarse hit's entries are kept in LDS (a ray meets at most 22 of 8^3
-// children), those past kEntries are read back from their row.
+// coarse hit's entries are kept in LDS, those past kEntries are read back from
+// their row: a ray in general position meets at most 3 n - 2 of n^3 children (22
+// at rate 8, 46 at rate 16), one along shared faces or edges more.
 template <int G>
 struct TreeSink {
   static constexpr int kRays = kWalkThreads / G;

@@ -150,3 +150,115 @@ def test_large_target_of_a_rate_2_tree():
             tree.voxel_size, 128, rate, noise)))
     print("rate 2 %.0f us, rate 4 %.0f us" % tuple(us))
     assert us[0] <= 1.3 * us[1]
+
+
+def _two_scenes(rate=4, dim=32):
+    """A tree over two batches and what the oracle needs of it."""
+    from sailor_amd import VoxelEncoding as VE
+    ins = [scene_inputs(k, 4, 128, 128, 150.0) for k in (0, 3)]
+    o = orc.integrate(*[np.concatenate([i[k] for i in ins]) for k in
+                        ("K", "RT", "R", "T", "colors", "depths")], (dim, dim, dim),
+                      fixed_bbox=None)
+    oc, ocnt = orc.merge(o["occ"], rate)
+    n0, n1 = int(o["num_occ"].sum()), int(ocnt.sum())
+    tree = VE.MultiLayerOctree(2, 2, rate, 0)
+    tree.init_octree([_t(o["occ"]), _t(oc)], [n0, n1],
+                     [_t(o["num_occ"].astype(np.int32).reshape(2, 1)),
+                      _t(ocnt.astype(np.int32).reshape(2, 1))], [0, n0],
+                     _t(o["voxel_size"].reshape(2, 1)), _t(o["vol_bbox"]))
+    tree.build_octree()
+    return tree, dict(vc=tree._vols[1].cpu().numpy(), pos=tree.node_pos.cpu().numpy(),
+                      info=tree.node_info.cpu().numpy(), bbox=o["vol_bbox"], vs=o["voxel_size"])
+
+
+def _cameras(H, W, fx):
+    return [np.concatenate(x) for x in zip(*[[y[0] for y in target_rays_np(H, W, fx, phase)]
+                                             for phase in (0.7, 2.1)])]
+
+
+@pytest.mark.parametrize("H,W,S", [(13, 7, 5), (13, 7, 33), (1, 1, 48), (9, 31, 7)])
+def test_trace_on_partial_waves_matches_the_oracle(H, W, S):
+    """Pixels that do not fill a wave's 8 groups, samples that end within a
+    group, two batches."""
+    from sailor_amd.render import trace_sample
+    tree, h = _two_scenes()
+    K, R, T = _cameras(H, W, 1.1 * max(H, W))
+    noise = np.random.default_rng(S).random((2, H * W, S)).astype(np.float32)
+    rays, sidx, st, vl = trace_sample(_t(K), _t(R), _t(T), (H, W), tree._vols[1], tree.node_pos,
+                                      tree.node_info, tree.volume_bbox, tree.voxel_size, 32, 4,
+                                      _t(noise))
+    r6 = orc.rays(K[:, None], R[:, None], T[:, None], H, W).reshape(2, -1, 6)
+    np.testing.assert_array_equal(rays.cpu().numpy(), r6)
+    w = orc.traverse(h["vc"], h["pos"], h["info"], h["bbox"], h["vs"], 32, 4, r6[..., :3],
+                     r6[..., 3:], 512)
+    ri, rt = orc.sampling(w["idx"], w["tmin"], w["tmax"], noise, w["valid_len"], h["pos"], h["vs"],
+                          S, 4, w["gmax"])
+    np.testing.assert_array_equal(vl.cpu().numpy(), w["valid_len"])
+    np.testing.assert_array_equal(sidx.cpu().numpy(), ri)
+    np.testing.assert_array_equal(st.cpu().numpy(), rt)
+    assert (ri >= 0).any()
+
+
+@pytest.mark.parametrize("n,S", [(1, 5), (7, 33), (77, 5), (77, 33)])
+def test_recursive_walks_on_partial_waves_match_the_oracle(n, S):
+    """Rays that do not fill a wave's 8 groups, list rows that start on any
+    float, two batches; the coarse traversal with is_training as well."""
+    tree, h = _two_scenes()
+    K, R, T = _cameras(24, 24, 26.0)
+    r6 = orc.rays(K[:, None], R[:, None], T[:, None], 24, 24).reshape(2, -1, 6)
+    pick = np.linspace(0.3 * 576, 0.7 * 576, n).astype(int)
+    ori, dirs = (np.ascontiguousarray(r6[:, pick, k:k + 3]) for k in (0, 3))
+    args = (h["vc"], h["pos"], h["info"], h["bbox"], h["vs"], 32, 4, ori, dirs)
+    got = tree.octree_traversal(_t(ori), _t(dirs), 97, 257, 0, -1, -1)
+    ref = orc.octree_traversal(*args, 97, 257)
+    for name, g in zip(("idx", "tmin", "tmax", "valid_len", "idx_c", "tmin_c", "tmax_c"), got):
+        np.testing.assert_array_equal(g.cpu().numpy().reshape(ref[name].shape), ref[name],
+                                      err_msg=name)
+    assert (ref["idx"] >= 0).any()
+    noise = np.random.default_rng(n + S).random((2, n, S)).astype(np.float32)
+    sidx, st = tree.ray_voxels_points_sampling(*got[:4], _t(noise), 0, S)
+    ri, rt = orc.sampling_adaptive(ref["idx"], ref["tmin"], ref["tmax"], noise, ref["valid_len"],
+                                   h["pos"], h["vs"], S, 2, tree.num_max_intersected_voxels_fine)
+    np.testing.assert_array_equal(sidx.cpu().numpy(), ri)
+    np.testing.assert_array_equal(st.cpu().numpy(), rt)
+    got = tree.voxel_traversal(_t(ori), _t(dirs), 129, 0, -1, True, -1)
+    ref = orc.traverse(*args, 129, is_training=True)
+    for name, g in zip(("idx", "tmin", "tmax", "valid_len"), got):
+        np.testing.assert_array_equal(g.cpu().numpy().reshape(ref[name].shape), ref[name],
+                                      err_msg=name)
+
+
+def test_recursive_walk_of_nodes_with_many_children_matches_the_oracle():
+    """A fully occupied tree of rate 16: a coarse hit lists more entries than
+    are kept on the chip (32).  Rays through faces, edges and corners of the
+    cells, whose children share intervals, among them."""
+    from sailor_amd import VoxelEncoding as VE
+    dim, rate = 64, 16
+    occ = np.arange(dim ** 3, dtype=np.int32).reshape(1, dim, dim, dim)
+    oc, ocnt = orc.merge(occ, rate)
+    vs = np.float32([2.0 / (dim - 1)])
+    box = np.float32([[[-1.0, 1.0]] * 3])
+    n0, n1 = dim ** 3, int(ocnt.sum())
+    tree = VE.MultiLayerOctree(2, 1, rate, 0)
+    tree.init_octree([_t(occ), _t(oc)], [n0, n1], [_t(np.int32([[n0]])), _t(np.int32([[n1]]))],
+                     [0, n0], _t(vs.reshape(1, 1)), _t(box))
+    tree.build_octree()
+    rng = np.random.default_rng(0)
+    dirs = np.concatenate([rng.normal(0, 1, (60, 3)), [[1, 1, 1], [1, -1, 1], [1, 1, 0],
+                                                       [0, 1, 0], [1, 1, 1e-3]]])
+    dirs = (dirs / np.linalg.norm(dirs, axis=1, keepdims=True)).astype(np.float32)
+    through = rng.uniform(-0.5, 0.5, dirs.shape)
+    through[-5:] = float(vs[0]) / 2      # between two cells of every axis
+    ori = (through - 3.0 * dirs).astype(np.float32)[None]
+    dirs = dirs[None]
+    got = tree.octree_traversal(_t(ori), _t(dirs), 64, 900, 0, -1, -1)
+    info, pos = tree.node_info.cpu().numpy(), tree.node_pos.cpu().numpy()
+    vc = tree._vols[1].cpu().numpy()
+    ref = orc.octree_traversal(vc, pos, info, box, vs, dim, rate, ori, dirs, 64, 900)
+    for name, g in zip(("idx", "tmin", "tmax", "valid_len", "idx_c", "tmin_c", "tmax_c"), got):
+        np.testing.assert_array_equal(g.cpu().numpy().reshape(ref[name].shape), ref[name],
+                                      err_msg=name)
+    parents = np.where(ref["idx"] >= 0, info[ref["idx"], 1], -1)
+    most = max(np.unique(row[row >= 0], return_counts=True)[1].max() for row in parents[0])
+    print("most children listed for a coarse hit:", most)
+    assert most > 32
