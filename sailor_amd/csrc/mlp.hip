@@ -55,6 +55,7 @@
 
 #include "common.h"
 #include "mlp_layout.h"
+#include "pe_sincos.h"
 
 namespace {
 
@@ -156,14 +157,10 @@ __device__ __forceinline__ float opaque_inf() {
 __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // sin(x) and cos(x) of a positional-encoding argument.  fp32 form: two sinf,
-// the cosine as sinf(x + pi/2) as freq_encoding.cu:37-45 writes it.  16-bit
-// forms: x minus the nearest multiple n of pi/2 (three fma with pi/2 split
-// into 24-bit parts, Cody-Waite), then odd / even polynomials on
-// [-pi/4, pi/4] (weighted least-squares minimax fits, 2e-9 and 1e-10 off), one
-// reduction for both values.  Against 64-bit values over |x| <= 1e6: rms
-// 2.1e-8, max 1e-7 (correctly rounded: 1.5e-8, 3e-8; x + pi/2 rounded to 32
-// bits makes the cosine of the other form up to 2.6e-5 off at |x| = 512).
-// Larger, infinite and NaN arguments take the library's.
+// the cosine as sinf(x + pi/2) as freq_encoding.cu:37-45 writes it (x + pi/2
+// rounded to 32 bits is up to 2.6e-5 off at |x| = 512).  16-bit forms: one
+// reduction and two polynomials (pe_sincos.h), no less exact than sinf; larger,
+// infinite and NaN arguments take the library's.
 template <int PREC>
 __device__ __forceinline__ void sincos_pe(float x, float& s, float& c) {
   if constexpr (PREC == kF32) {
@@ -171,26 +168,12 @@ __device__ __forceinline__ void sincos_pe(float x, float& s, float& c) {
     c = sinf(x + kHalfPi);
     return;
   }
-  if (!(fabsf(x) <= 1.0e6f)) {
+  if (!(fabsf(x) <= sailor::kPeSincosMax)) {
     s = sinf(x);
     c = cosf(x);
     return;
   }
-  const float n = rintf(x * 0.63661977236758134f);
-  float r = fmaf(-n, 1.5707963705062866f, x);
-  r = fmaf(-n, -4.3711388286737929e-8f, r);
-  r = fmaf(-n, -1.7151245100059e-15f, r);
-  const float z = r * r;
-  float p = fmaf(-1.9494950539e-4f, z, 8.3319731057e-3f);
-  p = fmaf(p, z, -1.6666650772e-1f);
-  const float sr = fmaf(p, z * r, r);
-  float q = fmaf(2.4437731554e-5f, z, -1.3887361856e-3f);
-  q = fmaf(q, z, 4.1666645557e-2f);
-  const float cr = fmaf(q, z * z, fmaf(z, -0.5f, 1.0f));
-  const int m = (int)n;
-  const float ss = (m & 1) ? cr : sr, cc = (m & 1) ? sr : cr;
-  s = __int_as_float(__float_as_int(ss) ^ ((m << 30) & 0x80000000));
-  c = __int_as_float(__float_as_int(cc) ^ (((m + 1) << 30) & 0x80000000));
+  sailor::pe_sincos(x, s, c);
 }
 
 // LDS written by some lanes of a wave and read by others of the same wave:
