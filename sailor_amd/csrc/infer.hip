@@ -271,10 +271,13 @@ __device__ __forceinline__ float view_sum(float x) {
   return x;
 }
 
-// Several floats of an input that starts on any float: wide loads need 4-byte
-// alignment only, the type has to say so.
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+// Several floats of an input that starts on any float (one wide load each, which
+// needs 4-byte alignment; through a vector type that says so the density kernel
+// moved 20 more registers per tile, 6 % of its time).
+__device__ __forceinline__ float4 read4(const float* p) {
+  return make_float4(p[0], p[1], p[2], p[3]);
+}
+__device__ __forceinline__ float2 read2(const float* p) { return make_float2(p[0], p[1]); }
 
 // acc = bias + W x with the layer's A fragments in registers
 template <int STEPS>
@@ -358,12 +361,14 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
   }
   float inf = __builtin_inff();
   asm("" : "+s"(inf));   // kept from the compiler, which would make the median a maximum again
-  // points are numbered over all batches: point p of batch b is
-  // p + b (V - 1) n_pts of view 0's inputs and p of the outputs
+  // points are numbered over all batches: of n views' values point p of batch b
+  // has p + (b (n - 1) + v) n_pts in view v
   const bool narrow = total <= 0xffffffffll;
-  auto batch_of = [&](long long p) -> long long {
-    if (FULL) return 0;
-    return narrow ? (long long)((unsigned)p / (unsigned)n_pts) : p / n_pts;
+  const long long col0 = (long long)(v < V ? v : 0) * n_pts;
+  auto element = [&](long long p, int n) -> long long {
+    if constexpr (FULL) return col0 + p;
+    const long long b = narrow ? (long long)((unsigned)p / (unsigned)n_pts) : p / n_pts;
+    return col0 + p + b * (n - 1) * n_pts;
   };
   // this lane's share of a column's inputs x = [z, tpsdf, geo 0..15]: half 0
   // holds x 0..7 and x 16..17, half 1 holds x 8..15 (its layer-0 B
@@ -374,13 +379,13 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
     for (int i = 0; i < 10; ++i) x[i] = 0.0f;
     const long long p = tile * P + lp;
     if (p < total && v < V) {
-      const long long e = p + (batch_of(p) * (V - 1) + v) * n_pts;
+      const long long e = element(p, V);
       const float* g = geo + e * 16;
-      const f32x4u a = *reinterpret_cast<const f32x4u*>(g + (h ? 8 : 0));
-      const f32x2u c = *reinterpret_cast<const f32x2u*>(g + (h ? 6 : 4));
-      const f32x2u d = *reinterpret_cast<const f32x2u*>(g + (h ? 12 : 14));
-      f32x2u f = c;
-      if (h == 0) f = f32x2u{z[e], tpsdf[e]};
+      const float4 a = read4(g + (h ? 8 : 0));
+      const float2 c = read2(g + (h ? 6 : 4));
+      const float2 d = read2(g + (h ? 12 : 14));
+      float2 f = c;
+      if (h == 0) f = make_float2(z[e], tpsdf[e]);
       x[0] = f.x; x[1] = f.y;
       x[2] = a.x; x[3] = a.y; x[4] = a.z; x[5] = a.w;
       x[6] = h ? d.x : c.x;
@@ -428,7 +433,7 @@ density_mfma_kernel(const half_t* __restrict__ params, const float* __restrict__
         mfma_layer1<1>(L, 7, gb, g, lane, 4 * zo);
         if (h == 0 && col_ok && v < n_geo_out) {
           float4* o4 = reinterpret_cast<float4*>(
-              geo_out + (p + (batch_of(p) * (n_geo_out - 1) + v) * n_pts) * 8);
+              geo_out + element(p, n_geo_out) * 8);
           o4[0] = make_float4(fmaxf(g[0], 0.f), fmaxf(g[1], 0.f), fmaxf(g[2], 0.f),
                               fmaxf(g[3], 0.f));
           o4[1] = make_float4(fmaxf(g[4], 0.f), fmaxf(g[5], 0.f), fmaxf(g[6], 0.f),
@@ -1394,13 +1399,10 @@ int launch_density(bool mfma, const half_t* pd, const float* z, const float* tps
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       cus = 256;
-    // tiles of a step: with 8 view slots fewer where they leave compute units
-    // without a workgroup (8 views of 1,000 points 64.5 us, 70 with 8 tiles; a
-    // step of 4 or fewer costs nothing to speak of beside the staging)
+    // tiles of a step: all VS, fewer where that leaves compute units without a
+    // workgroup (8 views of 1,000 points 70 us with 8 tiles a step, 62 now)
     const long long waves = (long long)cus * (kBlock / 64);
-    const int kt = VS < 8 ? VS
-                          : (int)std::min<long long>(
-                                VS, std::max<long long>(1, (tiles + waves - 1) / waves));
+    const int kt = (int)std::min<long long>(VS, std::max<long long>(1, (tiles + waves - 1) / waves));
     const long long steps = (tiles + kt - 1) / kt;
     const dim3 grid((unsigned)std::max<long long>(
         1, std::min<long long>((steps + kBlock / 64 - 1) / (kBlock / 64), 2LL * cus)));
