@@ -25,7 +25,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import as_input, call, check_input, ptr, stream_of
+from ._lib import as_input, call, check_input, on_device, ptr, stream_of
 
 _f32, _i32 = torch.float32, torch.int32
 
@@ -54,7 +54,7 @@ def integrate(occupied_vol, num_occ_voxel, cam_intr, cam_pose, cam_R, cam_T, col
     B, X, Y, Z = occupied_vol.shape
     colors = as_input(color_ims, "color_ims", _f32, dev)
     depths = as_input(depth_ims, "depth_ims", _f32, dev)
-    masks = as_input(mask_ims, "mask_ims", _i32, dev)
+    on_device(mask_ims, "mask_ims", dev)   # no kernel reads the masks
     if depths.dim() != 4 or depths.shape[0] != B:
         raise RuntimeError(f"depth_ims must be [B,V,H,W] with B={B}, got {tuple(depths.shape)}")
     _, V, H, W = depths.shape

@@ -156,13 +156,18 @@ def check_input(t, name, dtype=None, device=None):
     return t
 
 
-def as_input(t, name, dtype, device=None):
-    """Read-only input: cast/contiguous copies are allowed (the reference calls
-    .contiguous().data_ptr() on its inputs)."""
+def on_device(t, name, device=None):
+    """Validation of an input of any dtype and layout."""
     if not isinstance(t, torch.Tensor):
         raise RuntimeError(f"{name} input must be a tensor")
     if not t.is_cuda:
         raise RuntimeError(f"{name} input must be a cuda tensor")
     if device is not None and t.device != device:
         raise RuntimeError(f"{name} is on {t.device}, expected {device}")
-    return t.to(dtype).contiguous()
+    return t
+
+
+def as_input(t, name, dtype, device=None):
+    """Read-only input: cast/contiguous copies are allowed (the reference calls
+    .contiguous().data_ptr() on its inputs)."""
+    return on_device(t, name, device).to(dtype).contiguous()

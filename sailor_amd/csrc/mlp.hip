@@ -126,19 +126,19 @@ struct RenderArgs {
 template <int PREC> struct Tr;
 template <> struct Tr<kF32> {
   typedef float E;
-  static constexpr int EPL = 1, CE = 4;  // CE: elements per 16-byte chunk
+  static constexpr int CE = 4;  // elements per 16-byte chunk
 };
 template <> struct Tr<kBF16> {
   typedef __bf16 E;
   typedef bf16x8 V8;
   typedef bf16x4 V4;
-  static constexpr int EPL = 8, CE = 8;
+  static constexpr int CE = 8;
 };
 template <> struct Tr<kF16> {
   typedef _Float16 E;
   typedef f16x8 V8;
   typedef f16x4 V4;
-  static constexpr int EPL = 8, CE = 8;
+  static constexpr int CE = 8;
 };
 
 // max(x, 0), 0 for a NaN: what fmaxf gives, in one instruction (the median
@@ -618,13 +618,12 @@ constexpr size_t kLdsBytes = 160 * 1024;  // LDS per workgroup on gfx950
 // Bilinear feature gather of one quarter of the F channels (CPL = F/4) of
 // view v at world point (x, y, z): proj_persp (utils_render.py:380-410; depth
 // < 0.01 reads nothing) + grid_sample(align_corners=True, zero padding)
-// (SRONet/BasicRenNet.py:245-259) on channels-last maps, one 16-byte load
-// per 4 fp32 or 8 16-bit channels of a tap.
-template <int F, int PREC, bool HALF_MAP>
+// (SRONet/BasicRenNet.py:245-259) on channels-last fp32 maps, one 16-byte load
+// per 4 channels of a tap.
+template <int F>
 __device__ __forceinline__ void gather_quarter(const RenderArgs& a, int b, int v, float x,
                                                float y, float z, int quarter,
                                                float (&f)[F / 4]) {
-  typedef typename Tr<PREC>::E E;
   constexpr int CPL = F / 4;
   const int V = a.V;
 #pragma unroll
@@ -655,25 +654,14 @@ __device__ __forceinline__ void gather_quarter(const RenderArgs& a, int b, int v
     if (xx < 0 || xx >= a.Wf || yy < 0 || yy >= a.Hf) continue;
     const float wt = ((tap & 1) ? ax : 1.0f - ax) * ((tap >> 1) ? ay : 1.0f - ay);
     const size_t off = base + ((size_t)yy * a.Wf + xx) * F;
-    if constexpr (HALF_MAP) {
-      typedef typename Tr<PREC>::V8 V8;
-      const V8* src = reinterpret_cast<const V8*>(static_cast<const E*>(a.fmap) + off);
+    const f32x4* src = reinterpret_cast<const f32x4*>(static_cast<const float*>(a.fmap) + off);
 #pragma unroll
-      for (int qq = 0; qq < CPL / 8; ++qq) {
-        const V8 v8 = src[qq];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[8 * qq + e] += wt * (float)v8[e];
-      }
-    } else {
-      const f32x4* src = reinterpret_cast<const f32x4*>(static_cast<const float*>(a.fmap) + off);
-#pragma unroll
-      for (int qq = 0; qq < CPL / 4; ++qq) {
-        const f32x4 v4 = src[qq];
-        f[4 * qq + 0] += wt * v4[0];
-        f[4 * qq + 1] += wt * v4[1];
-        f[4 * qq + 2] += wt * v4[2];
-        f[4 * qq + 3] += wt * v4[3];
-      }
+    for (int qq = 0; qq < CPL / 4; ++qq) {
+      const f32x4 v4 = src[qq];
+      f[4 * qq + 0] += wt * v4[0];
+      f[4 * qq + 1] += wt * v4[1];
+      f[4 * qq + 2] += wt * v4[2];
+      f[4 * qq + 3] += wt * v4[3];
     }
   }
 }
@@ -846,7 +834,7 @@ render_kernel(RenderArgs a) {
       for (int j = 0; j < VPW; ++j) {
         const int v = wave + kWaves * j;
         const size_t vbase = ((size_t)b * V + (v < V ? v : 0)) * a.Hf * a.Wf * F;
-        auto finish = [&](int it, const f32x4& w4, const float (&f)[8]) {
+        auto finish = [&](int it, const float (&f)[8]) {
           const int sl = it / NP, part = it % NP, col = sl * VP + v;
           float* kp = keep + col * KF + part * 8;
           *reinterpret_cast<f32x4*>(kp) = f32x4{f[0], f[1], f[2], f[3]};
@@ -896,7 +884,7 @@ render_kernel(RenderArgs a) {
                 for (int tap = 0; tap < 4; ++tap)
 #pragma unroll
                   for (int i = 0; i < 8; ++i) f[i] += w4[r][tap] * (float)raw[r][tap][i];
-                finish(it, w4[r], f);
+                finish(it, f);
               }
             }
           }
@@ -921,7 +909,7 @@ render_kernel(RenderArgs a) {
             for (int tap = 0; tap < 4; ++tap)
 #pragma unroll
               for (int i = 0; i < 8; ++i) f[i] += w4[tap] * raw[tap][i / 4][i % 4];
-            finish(it, w4, f);
+            finish(it, f);
           }
         }
       }
@@ -1854,7 +1842,7 @@ struct BoxMap {
 // channel quarter it % 4), so a sample's 16 items are 16 consecutive lanes;
 // each dots its quarter of the channels with dL/dtoken (dtok), and four
 // shuffles add the quarters and the views.
-template <int F, int PREC, int NTHR>
+template <int F, int NTHR>
 __device__ __forceinline__ void ray_features(const RenderArgs& a, int b, const float* dtok,
                                              const float* s_pos, int S, int tid, float* keep,
                                              float* s_g) {
@@ -1863,7 +1851,7 @@ __device__ __forceinline__ void ray_features(const RenderArgs& a, int b, const f
     const int col = it >> 2, quarter = it & 3;
     const int sl = col >> 2, v = col & 3;
     float f[CPL];
-    gather_quarter<F, PREC, false>(a, b, v, s_pos[4 * sl], s_pos[4 * sl + 1],
+    gather_quarter<F>(a, b, v, s_pos[4 * sl], s_pos[4 * sl + 1],
                                    s_pos[4 * sl + 2], quarter, f);
     float* kp = keep + col * KF + quarter * CPL;
 #pragma unroll
@@ -1981,8 +1969,7 @@ render_backward_kernel(BackArgs ba) {
   typedef typename Tr<PREC>::E E;
   typedef SmemB<F, H, PREC, NS, SMAX> L;
   const RenderArgs& a = ba.r;
-  constexpr int NC = L::NC, KF = L::KF, MTW = H / 64, CE = Tr<PREC>::CE;
-  constexpr int CPL = F / 4, K0 = F + kPeSlots;
+  constexpr int NC = L::NC, MTW = H / 64, K0 = F + kPeSlots;
   constexpr SmallOffsets so = small_offsets(F, H);
   constexpr bool F32 = PREC == kF32;
   constexpr int NTL = NC / 16, NT32 = NC / 32;
@@ -2037,7 +2024,7 @@ render_backward_kernel(BackArgs ba) {
       s_alpha[tid] = ba.occ[ray * S + tid];
     }
     __syncthreads();
-    ray_features<F, PREC, kThreads>(a, b, ba.dtok + item * kVP * F, s_pos, S, tid, keep, s_g);
+    ray_features<F, kThreads>(a, b, ba.dtok + item * kVP * F, s_pos, S, tid, keep, s_g);
     __syncthreads();
     if (wave == 0) composite_backward(s_alpha, s_g, S, a.t_thres, lane, s_dz, gsb);
     __syncthreads();
@@ -2286,7 +2273,7 @@ render_backward16_kernel(BackArgs ba) {
         oc = ba.occ[ray * S + tid];
       }
     }
-    ray_features<F, PREC, NTHR>(a, b, ba.dtok + item * kVP * F, s_pos, S, tid, keep, s_g);
+    ray_features<F, NTHR>(a, b, ba.dtok + item * kVP * F, s_pos, S, tid, keep, s_g);
     __syncthreads();
     for (int c0 = 0; c0 < S; c0 += NS) {
       // the replay of the compositing (wave 0) beside the first chunk's input
